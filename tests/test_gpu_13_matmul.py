@@ -119,3 +119,28 @@ def test_tensor_matmul_plain_with_its_chain(rt):
   assert z.dtype == "fp32" and z.shape == (2, 9, 20)
   want = a.astype(np.float64) @ w[:30, :20]
   assert np.abs(np.array(z.tolist()) - want).max() <= 2 ** -14 * (np.abs(a) @ np.abs(w[:30, :20])).max()
+
+
+@pytest.mark.parametrize("M,K,N", [
+  (1, 64, 8), (129, 64, 136), (255, 128, 264),      # a tile and a row or a piece more or less; one K step, two
+  (2047, 192, 2048), (2049, 256, 2056),             # 128 x 128 tiles from LDS loads: 3 and 4 steps of a 4-stage ring
+  (4095, 320, 4104),                                # 128 x 256 tiles, 5 steps of a 3-stage ring
+  (2048, 66, 2050), (4097, 130, 4099),              # K past whole steps, odd rows: 128 and 256 wide tiles by registers
+  (300, 60, 1001),
+])
+def test_tiles_and_strides_give_the_same_bits(cuda, M, K, N):
+  """Each kernel and tile against the sums in float64 (exact products, fp32 sums over at most K / 16 chained MFMAs:
+  2^-21 of sum |a b|), and operands at odd and at even strides against the contiguous ones, bit for bit (the products
+  come in one order in every kernel). Rows and columns past M and N hold NaN: none of them may reach a sum."""
+  g = torch.Generator(device="cuda").manual_seed(M * 7 + K * 3 + N)
+  a, b = (torch.randn(1, *s, generator=g, device="cuda").to(torch.bfloat16) for s in ((M, K), (K, N)))
+  got = ops().matmul(a, b)
+  want, mag = a.double()[0] @ b.double()[0], a.double()[0].abs() @ b.double()[0].abs()
+  assert ((got[0].double() - want).abs() <= 2 ** -21 * mag).all()
+  for pad in (1, 2, 8):
+    wide = [torch.full((1, t.shape[1], t.shape[2] + pad), float("nan"), dtype=t.dtype, device="cuda") for t in (a, b)]
+    for w, t in zip(wide, (a, b)): w[:, :, :t.shape[2]] = t
+    again = ops().matmul(wide[0][:, :, :K], wide[1][:, :, :N])
+    assert torch.equal(again, got), pad
+  half = ops().matmul(a, b, out_dtype=torch.bfloat16)
+  assert torch.equal(half, got.to(torch.bfloat16))  # rounded once, to nearest even, in vector and in single stores
