@@ -20,7 +20,7 @@
 // weight lies expert_mant / expert_exps bytes on; its rows are the first counts[e] (at most M) of its list, x row
 // x_rows[e M + r] (row e M + r where x_rows is null), output row e M + r, scaled by row_w[e M + r] (scale_rows); a
 // row tile past the expert's count returns at once, so the grid is sized for the most rows an expert can have.
-#include "fh_epilogue.h"
+#include "fh_gemm.h"
 
 namespace fh {
 
@@ -29,29 +29,6 @@ constexpr int GM_LD = GM_BK + 8;     // LDS row of a tile operand, bf16: 144 byt
 constexpr int GM_LDC = GM_BN + 4;    // LDS row of the fp32 output tile
 constexpr int GM_THREADS = 256;
 constexpr int GM_GROUP = 8;          // row tiles a group (tile order)
-
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
-
-__device__ inline uint32_t pack_bf16_exact(float lo, float hi) {  // both exact in bf16: the high halves
-  // (the high halves of two floats whose low halves are 0: one byte permute, v_perm_b32)
-  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-__device__ inline uint32_t pack_bf16_rne(float lo, float hi) { return bf16_rne_f(lo) | (bf16_rne_f(hi) << 16); }
-
-// the run a tile's local run lr (0 .. RUNS - 1) stands for, or -1 past the weight: RUNS runs of 16 columns a tile, or
-// RUNS / 2 pairs (the first runs, then their partners)
-template <int RUNS = 8>
-__device__ inline int64_t tile_run(const MatArgs& a, int tn, int lr) {
-  if (a.P == 1) {
-    const int64_t nb = (int64_t)tn * RUNS + lr;
-    return nb < a.N / 16 ? nb : -1;
-  }
-  const int64_t it = (int64_t)tn * (RUNS / 2) + lr % (RUNS / 2);
-  if (it >= a.items) return -1;
-  const int64_t nb0 = pair_first(it, a.pair_half);
-  return lr < RUNS / 2 ? nb0 : nb0 + a.pair_half;
-}
 
 // RoPE's per-row values for the epilogue, staged in LDS while the tile's first loads are in flight: row ar's place and
 // cache row (m: the row, clamped into the matrix)
@@ -607,7 +584,7 @@ __global__ __launch_bounds__(2 * GM_THREADS, 1) void gemm_pp_kernel(MatArgs a, i
 }
 
 // The tiled kernel over a's M rows (per expert, gathered, when g.counts is set: grid.y = experts)
-int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, hipStream_t s) {
+int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void* workspace, size_t ws_bytes, hipStream_t s) {
   // 256-row tiles (8 waves, the weight's conversion shared by twice the rows) where they still give every CU a
   // workgroup or fewer (measured at 2048 rows of the 8B shapes: o 720 -> 765 TFLOP/s, down 780 -> 895; qkv and gate_up,
   // with more tiles than CUs, slower), 128-row tiles (4 waves, two workgroups a CU) otherwise
@@ -631,6 +608,20 @@ int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, hipSt
       const int64_t rounds = (tiles + cus - 1) / cus;
       const bool fills = tiles <= cus || tiles * 8 >= rounds * cus * 7;
       if (fills && (best == 0 || rounds * wn <= best)) { WNv = wn; best = rounds * wn; }
+    }
+  }
+  // gemm_lds (fh_gemm_lds.hip) for whatever it takes, but where one round of 192-column tiles of gemm_pp_kernel beats it
+  // (1.9 us a step: qkv at 2048 rows 130 us in its 256 tiles against 136 in 384 of 128 columns, at 1500 rows 113 against
+  // 134), and a mixture's experts past 512 rows a pass, several 128-row tiles an expert, where gemm_kernel's are
+  // faster (the Mixtral layer at 1000 tokens: 1168 us against 1279; at 300 even, at 100 616 against 485)
+  if (gemm_lds_takes(a)) {
+    if (g.counts) {
+      if (a.M <= 512) return gemm_lds(a, g, fmt, experts, gemm_lds_plan(a.M, a.K, a.N, experts, false), nullptr, s);
+    } else {
+      GemmPlan p = gemm_lds_plan(a.M, a.K, a.N, 0, workspace != nullptr);
+      if (gemm_lds_bytes(p, a.M, a.N) > ws_bytes) p = gemm_lds_plan(a.M, a.K, a.N, 0, false);
+      const int64_t tiles3 = (a.M + 2 * GM_BM - 1) / (2 * GM_BM) * (a.P == 1 ? (a.N / 16 + 11) / 12 : ((int64_t)a.items + 5) / 6);
+      if (WNv != 3 || tiles3 > cus || p.us <= 8 + 1.9 * (double)(a.K / GM_BK)) return gemm_lds(a, g, fmt, 1, p, (float*)workspace, s);
     }
   }
   const bool pp = WNv != 0;
@@ -679,6 +670,17 @@ using namespace fh;
 extern "C" int fh_gemm_bfp(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t N, const void* w_mant,
                            const uint8_t* w_exps, int fmt, const fh_epilogue* ep, void* y, int y_dtype, int64_t ldy,
                            void* stream) {
+  return fh_gemm_bfp_ws(x, x_dtype, ldx, M, K, N, w_mant, w_exps, fmt, ep, y, y_dtype, ldy, nullptr, 0, stream);
+}
+
+extern "C" size_t fh_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
+  if (M <= 64 || K < 64 || K % 64 || N < 16 || N % 16) return 0;
+  return gemm_lds_bytes(gemm_lds_plan(M, K, N, 0, true), M, N);
+}
+
+extern "C" int fh_gemm_bfp_ws(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t N, const void* w_mant,
+                              const uint8_t* w_exps, int fmt, const fh_epilogue* ep, void* y, int y_dtype, int64_t ldy,
+                              void* workspace, size_t ws_bytes, void* stream) {
   if (!x || !w_mant || !w_exps || !y) return fail(FH_EINVAL, "fh_gemm_bfp: null pointer");
   if (M < 1 || K < 32 || K % 32 || N < 16 || N % 16)
     return fail(FH_EINVAL, "fh_gemm_bfp: need M >= 1, K a multiple of 32, N a multiple of 16");
@@ -693,6 +695,8 @@ extern "C" int fh_gemm_bfp(const void* x, int x_dtype, int64_t ldx, int64_t M, i
   a.mant = (const uint8_t*)w_mant; a.exps = w_exps; a.K = K; a.N = N; a.M = M;
   a.y = y; a.y_bf16 = y_dtype != FH_F32; a.y_tiles = y_dtype == FH_BF16_T16; a.ldy = ldy;
   if (int rc = epilogue_args("fh_gemm_bfp", ep, K, N, y_dtype, ldy, a)) return rc;
+  // (a program that only copies the sum, what a lazy matmul with nothing on top of it carries, is a plain store)
+  if (a.kind == FH_EP_PROGRAM && a.prog.n_ops == 1 && a.prog.op[0] == FH_OP_COPY && a.prog.a[0] == FH_OPND_ACC) a.kind = FH_EP_STORE;
   if (a.y_tiles && ldy % 8) return fail(FH_EINVAL, "fh_gemm_bfp: FH_BF16_T16 y needs ldy a multiple of 8");
   hipStream_t s = as_stream(stream);
   if (M <= 64 && K % 64 == 0) {  // a few rows: the skinny kernel (K split among waves, as the GEMV splits it)
@@ -702,6 +706,7 @@ extern "C" int fh_gemm_bfp(const void* x, int x_dtype, int64_t ldx, int64_t M, i
   if (a.x_tiles || a.y_tiles || a.copy_tiles)
     return fail(FH_EUNSUP, "fh_gemm_bfp: FH_BF16_T16 rows (and copy_tiles) are for up to 64 rows with K a multiple of 64");
   const SkinnyMoe none = {};
-  if (int rc = gemm_tiles(a, none, fmt, 1, s)) return rc;
+  if (workspace && ((uintptr_t)workspace & 15)) return fail(FH_EINVAL, "fh_gemm_bfp_ws: a workspace at 16-byte alignment");
+  if (int rc = gemm_tiles(a, none, fmt, 1, workspace, ws_bytes, s)) return rc;
   return check_launch("fh_gemm_bfp");
 }

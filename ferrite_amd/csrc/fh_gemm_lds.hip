@@ -1,0 +1,468 @@
+// The tiled matmul by a block-float weight for bf16 rows whose K is whole steps of 64 (a prompt's matmuls, a mixture's
+// gathered experts): x straight from memory into LDS, the weight converted on its way there.
+//
+// A workgroup of 2 WR waves takes 32 WR TM rows by 128 columns (8 runs of 16, or 4 runs and their RoPE / SiLU·gate
+// partners), each wave 32 TM rows by two blocks of 32 columns, the second 64 columns after the first: a pair's two runs,
+// so that a lane holds both of a pair's sums and the epilogue runs on the accumulators where they are. K steps of 64:
+// x's rows go into a ring of two or three LDS stages by global_load_lds_dwordx4 (no registers, no LDS write instructions; each
+// lane's address places its 16 bytes in the swizzled row). The weight's rows come in registers,
+// three steps ahead (a lane a run's row: 16 bytes of bfp8, 8 of bfp4, and its exponent; a wave's loads 1 KiB or 512 B in
+// one piece), and go as 16 bf16 values, row-major as they lie, into one of two stages while the matrix cores work on
+// the other; ds_read_b64_tr_b16 reads them K-contiguous (fh_skinny.hip's read), so nothing is transposed on the way in.
+// A row's 16-byte pieces are XOR-swizzled by the row so that 16 rows' writes, and a transposed read's four, meet no bank
+// twice. One workgroup barrier a step.
+//
+// The products are gemm_kernel's, in its order: the same bits. Split (K in parts, for tiles that do not fill the CUs): a
+// workgroup adds up its part and leaves the sums, as its lanes hold them, in the workspace; split_sum_kernel adds a
+// tile's parts in order and runs the epilogue.
+#include "fh_gemm.h"
+
+namespace fh {
+
+constexpr int GL_BK = 64, GL_BN = 128, GL_RUNS = GL_BN / 16;
+
+typedef short gl_short4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) gl_short4* gl_lds_short4;
+typedef const __attribute__((address_space(1))) uint32_t* gl_global;
+typedef __attribute__((address_space(3))) uint32_t* gl_lds;
+
+// A wave's 16 rows m0 .. by two blocks of 32 columns (columns wc and 64 + wc of the tile) through a's epilogue, from cs
+// (LDS, this wave's own: [16][GL_LDC], a row's two blocks side by side). rs: the rows' 1/rms, or null for 1. Short loops,
+// not unrolled rows: a workgroup runs this once, at the pace its instructions arrive (unrolled over the accumulators the
+// kernel was 90 KB of code, and a call of one K step took 13 us).
+constexpr int GL_LDC = 68;
+__device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe& g, const float* cs, int tn, int wc, int64_t m0,
+                                               int64_t M, int64_t ybase, int lane, const float* rs) {
+  const int kind = a.kind;
+  if (a.P == 1) {  // a lane 4 columns of a row, 4 rows a pass
+    const int q = lane & 15, c = 4 * q, lc = wc + (c & 31);
+    const int64_t run = tile_run<GL_RUNS>(a, tn, 4 * (q >> 3) + (lc >> 4)), col = run * 16 + (lc & 15);
+    const bool res = kind == FH_EP_RESIDUAL;
+    const bool vec = !(a.ldy & 3) && !((uintptr_t)a.y & 15) && !(res && ((uintptr_t)a.residual & 15));
+    float4 old[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // (the rows' loads before the first store, which may alias them)
+      const float* p = a.residual + (ybase + min(m0 + (lane >> 4) + 4 * i, M - 1)) * a.ldy + col;
+      old[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (res && run >= 0) old[i] = vec ? *(const float4*)p : make_float4(p[0], p[1], p[2], p[3]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = (lane >> 4) + 4 * i;
+      const int64_t m = m0 + r, at = (ybase + m) * a.ldy + col;
+      const bool ok = m < M && run >= 0;
+      float4 v = *(const float4*)(cs + r * GL_LDC + c);
+      if (rs) { v.x *= rs[r]; v.y *= rs[r]; v.z *= rs[r]; v.w *= rs[r]; }
+      if (res) { v.x += old[i].x; v.y += old[i].y; v.z += old[i].z; v.w += old[i].w; }
+      if (ok) {
+        if (vec && !a.y_bf16) *(float4*)((float*)a.y + at) = v;
+        else if (vec) *(uint2*)((uint16_t*)a.y + at) = make_uint2(bf16_rne_f(v.x) | bf16_rne_f(v.y) << 16, bf16_rne_f(v.z) | bf16_rne_f(v.w) << 16);
+        else { store_out(a.y, a.y_bf16, at, v.x); store_out(a.y, a.y_bf16, at + 1, v.y); store_out(a.y, a.y_bf16, at + 2, v.z); store_out(a.y, a.y_bf16, at + 3, v.w); }
+      }
+      if (res && a.copy_bf16 && ok) { put_copy(a, m, col, v.x); put_copy(a, m, col + 1, v.y); put_copy(a, m, col + 2, v.z); put_copy(a, m, col + 3, v.w); }
+      if (res && a.ssq_out) {  // (a run is 4 lanes' 4 columns: the pairs 8, 4, 2 and 1 columns apart, in that order)
+        float s[4] = {v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { s[k] += __shfl_xor(s[k], 2, 64); s[k] += __shfl_xor(s[k], 1, 64); }
+        if (ok && !(q & 3)) a.ssq_out[m * (a.N / 16) + run] = (s[0] + s[2]) + (s[1] + s[3]);
+      }
+      if (kind == FH_EP_STORE && a.argmax_parts) {
+        float bv = v.x;
+        int bc = (int)col;
+        if (v.y > bv) { bv = v.y; bc = (int)col + 1; }
+        if (v.z > bv) { bv = v.z; bc = (int)col + 2; }
+        if (v.w > bv) { bv = v.w; bc = (int)col + 3; }
+#pragma unroll
+        for (int k = 2; k >= 1; k >>= 1) {
+          const float ov = __shfl_xor(bv, k, 64);
+          const int oc = __shfl_xor(bc, k, 64);
+          if (ov > bv || (ov == bv && oc < bc)) { bv = ov; bc = oc; }
+        }
+        if (ok && !(q & 3)) a.argmax_parts[m * (a.N / 16) + run] = make_int2(__float_as_int(bv), bc);
+      }
+    }
+    return;
+  }
+  // the pairs: a lane a column of the first run (its partner in the second block), 2 rows a pass; a run is 16 lanes
+  const int c = lane & 31, j = lane & 15;
+  const int64_t run = tile_run<GL_RUNS>(a, tn, (wc + c) >> 4), c0 = run * 16 + j;
+  if (kind == FH_EP_SILU_GATE) {
+    float sc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sc[i] = g.scale_rows ? g.row_w[ybase + min(m0 + (lane >> 5) + 2 * i, M - 1)] : 1.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = (lane >> 5) + 2 * i;
+      const float s = rs ? rs[r] : 1.f;
+      if (m0 + r < M && run >= 0)
+        store_out(a.y, a.y_bf16, (ybase + m0 + r) * a.ldy + c0, silu(cs[r * GL_LDC + c] * s) * (cs[r * GL_LDC + 32 + c] * s) * sc[i]);
+    }
+    return;
+  }
+  const int hd = a.head_dim, h = (int)c0 / hd, d = (int)c0 % hd, d1 = d + hd / 2;  // (c0 < N < 2^31)
+  const bool turn = h < a.heads + a.kv_heads;  // q's and k's heads turn: x cos + (-x2, x1) sin (models/llama.py:92-93)
+  for (int i0 = 0; i0 < 8; i0 += 4) {
+    float cs0[4], cs1[4], sn0[4], sn1[4];
+    int32_t crow[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t m = min(m0 + (lane >> 5) + 2 * (i0 + u), M - 1);
+      crow[u] = a.cache_rows[m];
+      cs0[u] = cs1[u] = 1.f;
+      sn0[u] = sn1[u] = 0.f;
+      if (turn) {
+        const int64_t place = rope_place(a, a.places[m]);
+        cs0[u] = a.cos_tab[place * hd + d]; cs1[u] = a.cos_tab[place * hd + d1];
+        sn0[u] = a.sin_tab[place * hd + d]; sn1[u] = a.sin_tab[place * hd + d1];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = (lane >> 5) + 2 * (i0 + u);
+      const int64_t m = m0 + r;
+      if (m >= M || run < 0) continue;
+      const float s = rs ? rs[r] : 1.f;
+      float x0 = cs[r * GL_LDC + c] * s, x1 = cs[r * GL_LDC + 32 + c] * s;
+      if (turn) {
+        const float t0 = x0 * cs0[u] - x1 * sn0[u], t1 = x1 * cs1[u] + x0 * sn1[u];
+        x0 = t0; x1 = t1;
+      }
+      if (h < a.heads) {
+        float* q = (float*)a.y + m * a.ldy + (int64_t)h * hd;
+        q[d] = x0; q[d1] = x1;
+      } else {
+        cache_put(a, h - a.heads, crow[u], d, d1, j, x0, x1);
+      }
+    }
+  }
+}
+
+// A wave's blocks' values of 16 rows (values r = 8 half .. + 7 of each block: rows 16 half .. + 15) into cs
+__device__ __forceinline__ void block_to_lds(float* cs, const floatx16 (&v)[2], int half, int lane) {
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh)
+    if (hh == half)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) cs[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * GL_LDC + 32 * j + (lane & 31)] = v[j][8 * hh + r];
+}
+
+// 1/rms of rows m0 .. m0 + n - 1 into rs (LDS), from the sums of squares their maker left by runs of 16, two of the
+// workgroup's threads a row
+__device__ __forceinline__ void row_scales(const MatArgs& a, float* rs, int n, int64_t m0, int t, int threads) {
+  for (int r = t >> 1; r < n; r += threads >> 1) {
+    float s = 0.f;
+    if (m0 + r < a.M) {
+      const float* q = a.ssq_in + (m0 + r) * a.ssq_parts;
+      for (int i = t & 1; i < a.ssq_parts; i += 2) s += q[i];
+    }
+    s += __shfl_xor(s, 1, 64);
+    if (!(t & 1)) rs[r] = 1.0f / sqrtf(s / (float)a.K + a.eps);
+  }
+}
+
+template <bool FOUR, int WR, int TM, bool SPLIT>
+__global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits,
+                                                                                  float* parts) {
+  constexpr int NW = 2 * WR, BM = 32 * WR * TM, NS = TM == 2 || SPLIT ? 2 : 3;
+  constexpr int AB = BM * GL_BK * 2, BB = GL_BK * GL_BN * 2;
+  constexpr int IA = AB / 1024 / NW;           // a wave's loads of x a step (1 KiB, 8 rows each)
+  constexpr int UPT = (GL_RUNS + NW - 1) / NW;  // runs a wave takes, a lane a row of the step
+  constexpr int WL = 2 * (GL_RUNS / NW);        // at least so many loads of the weight a step
+  constexpr int RB = FOUR ? 8 : 16;
+  using Row = typename std::conditional<FOUR, uint2, uint4>::type;
+  __shared__ __attribute__((aligned(16))) char a0[AB];
+  __shared__ __attribute__((aligned(16))) char a1[AB];
+  __shared__ __attribute__((aligned(16))) char a2[NS == 3 ? AB : 16];
+  __shared__ __attribute__((aligned(16))) char b0[BB];
+  __shared__ __attribute__((aligned(16))) char b1[BB];
+
+  // this workgroup's expert, part of K and tile: tiles (a part's one after another) go to the XCDs in contiguous ranges,
+  // in groups of 8 row tiles
+  int64_t M = a.M, ybase = 0;
+  const uint8_t* wmant = a.mant;
+  const uint8_t* wexps = a.exps;
+  int id = blockIdx.x, tiles = tiles_m * tiles_n, at = 0;
+  if (g.counts) {
+    const int e = blockIdx.y;
+    at = e * tiles * splits;  // (its place among the partial sums)
+    M = min((int64_t)g.counts[e], a.M);
+    ybase = (int64_t)e * a.M;
+    wmant += e * g.expert_mant;
+    wexps += e * g.expert_exps;
+    tiles_m = (int)((M + BM - 1) / BM);
+    tiles = tiles_m * tiles_n;
+    const int q = (tiles * splits + 7) / 8;
+    if (id >= 8 * q) return;
+    id = (id % 8) * q + id / 8;
+    if (id >= tiles * splits) return;
+  } else if (tiles * splits % 8 == 0) {
+    id = (id % 8) * (tiles * splits / 8) + id / 8;
+  }
+  const int part = SPLIT ? id / tiles : 0;
+  if (SPLIT) id -= part * tiles;
+  const int per_group = 8 * tiles_n, first_m = id / per_group * 8, gm = min(tiles_m - first_m, 8);
+  const int tm = first_m + (id % per_group) % gm, tn = (id % per_group) / gm;
+  const int64_t m0 = (int64_t)tm * BM;
+  const int all = (int)(a.K / GL_BK);
+  const int first = SPLIT ? (int)((int64_t)all * part / splits) : 0;
+  const int steps = (SPLIT ? (int)((int64_t)all * (part + 1) / splits) : all) - first;
+
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  // x: load i of this wave fills rows 8 (wave IA + i) .. + 7 of a stage, lane l the l-th 16 bytes: row l / 8, piece l % 8,
+  // which holds piece (l % 8) ^ (row / 2 % 8) of the row (rows past M read the last one)
+  const uint16_t* px[IA];
+#pragma unroll
+  for (int i = 0; i < IA; ++i) {
+    const int r = 8 * (wave * IA + i) + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    const int64_t m = min(m0 + r, M - 1);
+    const int64_t row = g.counts ? (g.x_rows ? (int64_t)g.x_rows[ybase + m] : ybase + m) : m;
+    px[i] = (const uint16_t*)a.x + row * a.ldx + (int64_t)first * GL_BK + 8 * c;
+  }
+  auto load_x = [&](char* s, int step) {
+#pragma unroll
+    for (int i = 0; i < IA; ++i)
+      __builtin_amdgcn_global_load_lds((gl_global)(px[i] + (int64_t)min(step, steps - 1) * GL_BK), (gl_lds)(s + (wave * IA + i) * 1024), 16, 0, 0);
+  };
+  // the weight: run wave + NW i of the tile, row `lane` of the step (a run past the weight reads the first; its columns
+  // are not stored)
+  const uint8_t* pm[UPT];
+  const uint8_t* pe[UPT];
+#pragma unroll
+  for (int i = 0; i < UPT; ++i) {
+    const int lr = wave + NW * i;
+    const int64_t nb = lr < GL_RUNS ? tile_run<GL_RUNS>(a, tn, lr) : 0;
+    const int64_t k = (nb < 0 ? 0 : nb) * a.K + (int64_t)first * GL_BK + lane;
+    pm[i] = wmant + k * RB;
+    pe[i] = wexps + k;
+  }
+  Row wm[2][UPT];
+  uint32_t we[2][UPT];
+  auto load_w = [&](int step, int set) {
+    const int64_t k = (int64_t)min(step, steps - 1) * GL_BK;
+#pragma unroll
+    for (int i = 0; i < UPT; ++i) {
+      if (GL_RUNS % NW && wave + NW * i >= GL_RUNS) continue;
+      wm[set][i] = *(const Row*)(pm[i] + k * RB);
+      we[set][i] = pe[i][k];
+    }
+  };
+  auto swz = [](int k) { return 4 * (k & 3) + ((k >> 2) & 3); };  // row k's XOR on a piece's place
+  auto store_w = [&](char* s, int set) {
+#pragma unroll
+    for (int i = 0; i < UPT; ++i) {
+      const int lr = wave + NW * i;
+      if (GL_RUNS % NW && lr >= GL_RUNS) continue;
+      float f[16];
+      magnitudes(wm[set][i], f);
+      const float sc = ldexpf(1.f, (int)we[set][i] - 133);
+      uint32_t w[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w[q] = pack_bf16_exact(f[2 * q] * sc, f[2 * q + 1] * sc);
+      char* row = s + lane * GL_BN * 2;
+      *(uint4*)(row + ((2 * lr ^ swz(lane)) << 4)) = make_uint4(w[0], w[1], w[2], w[3]);
+      *(uint4*)(row + (((2 * lr + 1) ^ swz(lane)) << 4)) = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+  };
+
+  floatx16 acc[TM][2];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  const int wr = (wave >> 1) * 32 * TM, wc = (wave & 1) * 32;
+  const bool live = m0 + wr < M;  // (else none of this wave's rows are there: it only loads for the others)
+  const int fr = lane & 31, fh8 = lane >> 5;
+  const int rm = (lane >> 2) & 3, rq = lane & 3, rg = (lane >> 4) & 1;
+  auto compute = [&](const char* sa, const char* sb) {
+    if (TM == 1 && !live) return;
+#pragma unroll
+    for (int kk = 0; kk < GL_BK; kk += 16) {
+      bf16x8 fa[TM], fb[2];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int r = wr + 32 * i + fr;
+        fa[i] = *(const bf16x8*)(sa + r * GL_BK * 2 + (((kk / 8 + fh8) ^ ((r >> 1) & 7)) << 4));
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int k = kk + 8 * fh8 + rm, c = (64 * j + wc + 16 * rg + 4 * rq) >> 3;
+        union { gl_short4 s[2]; bf16x8 v; } u;
+        u.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gl_lds_short4)(sb + k * GL_BN * 2 + ((c ^ swz(k)) << 4) + 8 * (rq & 1)));
+        u.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gl_lds_short4)(sb + (k + 4) * GL_BN * 2 + ((c ^ swz(k + 4)) << 4) + 8 * (rq & 1)));
+        fb[j] = u.v;
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+    }
+  };
+
+  // Step s: wait for this wave's loads of x's stage s (issued after them, with two stages: the weight of s + 2; with three:
+  // the weight of s + 1, x of s + 1 and the weight of s + 2), for its LDS writes and its reads of the last step, meet the
+  // others; then x of s + NS - 1 goes out, the weight of s + 1 into its stage, the weight of s + 3 out, and the products
+  // (the compiler interleaves the conversion with them). Past the last step the loads read it again, into stages and
+  // registers that nobody reads.
+#define GL_A(i) ((i) % NS == 0 ? a0 : (i) % NS == 1 ? a1 : a2)
+#define GL_B(i) ((i) % 2 == 0 ? b0 : b1)
+  load_x(a0, 0);
+  load_w(0, 0);
+  asm volatile("" ::: "memory");
+  if (NS == 3) load_x(a1, 1);
+  asm volatile("" ::: "memory");
+  load_w(1, 1);
+  store_w(b0, 0);
+  load_w(2, 0);
+  constexpr int TURN = NS == 2 ? 2 : 6;  // (both stage counts divide it)
+  for (int q = 0; q < steps; q += TURN) {
+#pragma unroll
+    for (int i = 0; i < TURN; ++i) {
+      if (q + i >= steps) break;
+      constexpr int W = NS == 3 ? IA + 2 * WL : WL;  // vmcnt(W) lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0x0070 | (W & 15) | (W >> 4) << 14);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      load_x(GL_A(i + NS - 1), q + i + NS - 1);
+      asm volatile("" ::: "memory");
+      store_w(GL_B(i + 1), (i + 1) & 1);
+      load_w(q + i + 3, (i + 1) & 1);
+      compute(GL_A(i), GL_B(i));
+    }
+  }
+#undef GL_A
+#undef GL_B
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070);  // (no load into LDS outlives its workgroup)
+  if (SPLIT) {
+    if (!live) return;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      float* p = parts + (((int64_t)(at + part * tiles + id) * NW + wave) * TM + i) * 2048 + lane;
+      if (m0 + wr + 32 * i < M)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) p[(16 * j + r) * 64] = acc[i][j][r];
+    }
+    return;
+  }
+  __syncthreads();  // the stages are free: each wave's outputs, 16 rows at a time, in a part of x's of its own
+  constexpr int CW = 16 * GL_LDC * 4, WPA = AB / CW;
+  static_assert(SPLIT || 5 * WPA >= NW, "the outputs' place");
+  float* cs = (float*)((wave < WPA ? a0 : wave < 2 * WPA ? a1 : NS == 3 ? a2 : b1) + wave % WPA * CW);
+  float* rs_s = (float*)b0 + wave * 32 * TM;
+  if (a.ssq_in) row_scales(a, rs_s, 32 * TM, m0 + wr, lane, 64);  // (each wave its own rows' 1/rms, where the weight was)
+  for (int u = 0; u < 2 * TM && m0 + wr + 16 * u < M; ++u) {
+#pragma unroll
+    for (int ii = 0; ii < TM; ++ii)  // (the accumulators' indices stay constants)
+      if (ii == u >> 1) block_to_lds(cs, acc[ii], u & 1, lane);
+    block_epilogue(a, g, cs, tn, wc, m0 + wr + 16 * u, M, ybase, lane, a.ssq_in ? rs_s + 16 * u : nullptr);
+  }
+}
+
+// The split tiles' sums: a wave 16 rows by 2 x 32 columns of a tile (half of a wave's block there), its parts added in order,
+// four parts' loads in flight at a time, then the epilogue. Bound by reading the parts once (splits x 4 bytes an output).
+template <int WR, int TM>
+__global__ __launch_bounds__(256) void split_sum_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits, const float* parts) {
+  constexpr int NW = 2 * WR, BM = 32 * WR * TM;
+  __shared__ float rs_s[4][16];
+  __shared__ __attribute__((aligned(16))) float cs_s[4][16 * GL_LDC];
+  int64_t M = a.M, ybase = 0;
+  int tiles = tiles_m * tiles_n, at = 0;
+  if (g.counts) {
+    const int e = blockIdx.y;
+    at = e * tiles * splits;
+    M = min((int64_t)g.counts[e], a.M);
+    ybase = (int64_t)e * a.M;
+    tiles_m = (int)((M + BM - 1) / BM);
+    tiles = tiles_m * tiles_n;
+  }
+  const int lane = threadIdx.x & 63, u = blockIdx.x * 4 + (threadIdx.x >> 6);  // unit u: (tile, wave, i, half)
+  const int half = u & 1, i = (u >> 1) % TM, wave = (u >> 1) / TM % NW, id = (u >> 1) / (TM * NW);
+  if (id >= tiles) return;
+  const int per_group = 8 * tiles_n, first_m = id / per_group * 8, gm = min(tiles_m - first_m, 8);
+  const int tm = first_m + (id % per_group) % gm, tn = (id % per_group) / gm;
+  const int64_t m0 = (int64_t)tm * BM + ((wave >> 1) * TM + i) * 32 + 16 * half;
+  if (m0 >= M) return;
+  float* rs = rs_s[threadIdx.x >> 6];
+  float* cs = cs_s[threadIdx.x >> 6];
+  if (a.ssq_in) row_scales(a, rs, 16, m0, lane, 64);  // (this wave's own rows)
+  const int64_t stride = (int64_t)tiles * NW * TM * 2048;
+  const float* p = parts + (((int64_t)(at + id) * NW + wave) * TM + i) * 2048 + 512 * half + lane;
+  float acc[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  for (int s = 0; s < splits; s += 4) {
+    float v[4][16];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[k][r] = p[min(s + k, splits - 1) * stride + (r & 7) * 64 + (r >> 3) * 1024];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] += s + k < splits ? v[k][r] : 0.f;
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) cs[(8 * ((r & 7) >> 2) + 4 * (lane >> 5) + (r & 3)) * GL_LDC + 32 * (r >> 3) + (lane & 31)] = acc[r];
+  block_epilogue(a, g, cs, tn, (wave & 1) * 32, m0, M, ybase, lane, a.ssq_in ? rs : nullptr);
+}
+
+bool gemm_lds_takes(const MatArgs& a) {
+  return a.kind != FH_EP_PROGRAM && a.x_bf16 && !a.x_tiles && !a.y_tiles && !a.copy_tiles && !a.norm_w && a.K % GL_BK == 0 && !((uintptr_t)a.x & 15) && a.ldx % 8 == 0;
+}
+
+// Rows a tile and K's parts: the least of a model of the call's time in us, its constants measured at the 8B shapes (bfp8
+// and bfp4 alike): 8 a launch; a step of a 256-row tile 1.0 with a workgroup a CU, 1.15 a round of them with the chip
+// full; of a 128-row tile 0.8 alone on a CU, 1.38 two a CU; K in parts, 6 more for the second launch and the parts written
+// and read back at 6.5 TB/s. (Measured, 200 rows after 1 part -> the plan's: o 4096 x 4096 75 -> 29 us in 8, down
+// 14336 x 4096 203 -> 48 in 8, qkv 4096 x 6144 67 -> 31 in 4; 1024 rows: o 72 -> 53 and down 214 -> 133 in 2; at 2048
+// rows every shape is fastest in one part.) A gathered matmul (experts > 0), whose rows an expert the host does not know,
+// takes 128-row tiles in one part.
+GemmPlan gemm_lds_plan(int64_t M, int64_t K, int64_t N, int experts, bool may_split) {
+  if (experts > 0) return {128, 1, 0};
+  GemmPlan best = {};
+  double cost = 0;
+  for (int bm = 256; bm >= 128; bm /= 2) {
+    const int64_t tiles = (M + bm - 1) / bm * ((N + GL_BN - 1) / GL_BN), all = K / GL_BK;
+    for (int s = 1; s <= (may_split ? 16 : 1) && (s == 1 || all / s >= 4); ++s) {
+      const int64_t t = tiles * s;
+      double step;
+      if (bm == 256) step = t <= 256 ? 1.0 : 1.15 * ((t + 255) / 256);
+      else step = 1.38 * (t / 512) + (t % 512 == 0 ? 0 : t % 512 <= 256 ? 0.8 : 1.38);
+      const double us = 8 + (all + s - 1) / s * step + (s > 1 ? 6 + 8.0 * s * M * N / 6.5e6 : 0);
+      if (cost == 0 || us < cost) { cost = us; best = {bm, s, us}; }
+    }
+  }
+  return best;
+}
+
+size_t gemm_lds_bytes(const GemmPlan& p, int64_t M, int64_t N) {
+  return p.splits < 2 ? 0 : (size_t)p.splits * ((M + p.bm - 1) / p.bm) * ((N + GL_BN - 1) / GL_BN) * p.bm * GL_BN * 4;
+}
+
+int gemm_lds(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, const GemmPlan& p, float* parts, hipStream_t s) {
+  const int64_t tm = (a.M + p.bm - 1) / p.bm, tn = a.P == 1 ? (a.N / 16 + 7) / 8 : ((int64_t)a.items + 3) / 4;
+  if (tm * tn * p.splits >= 1LL << 22) return fail(FH_EUNSUP, "fh_gemm_bfp: too many tiles");
+  const int64_t n = g.counts ? (tm * tn * p.splits + 7) / 8 * 8 : tm * tn * p.splits;
+  const dim3 grid((unsigned)n, g.counts ? experts : 1);
+#define GL(F, WR, TM) do { \
+    if (p.splits < 2) hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, false>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, 1, parts); \
+    else { \
+      hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, true>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
+      hipLaunchKernelGGL((split_sum_kernel<WR, TM>), dim3((unsigned)(tm * tn * WR * TM), g.counts ? experts : 1), dim3(256), 0, s, a, g, (int)tm, (int)tn, p.splits, (const float*)parts); \
+    } } while (0)
+#define GL_F(WR, TM) do { if (fmt == FH_BFP4) GL(true, WR, TM); else GL(false, WR, TM); } while (0)
+  if (p.bm == 256) GL_F(4, 2);
+  else GL_F(4, 1);
+#undef GL_F
+#undef GL
+  return check_launch("fh_gemm_bfp");
+}
+
+}  // namespace fh

@@ -382,7 +382,7 @@ extern "C" int fh_moe_experts(const float* x, int64_t ldx, int rows, int64_t dim
     SkinnyMoe moe = {};
     moe.expert_mant = (int64_t)mb; moe.expert_exps = (int64_t)eb; moe.experts = experts; moe.scale_rows = 1;
     moe.counts = counts; moe.x_rows = rows_of; moe.row_w = row_w;
-    if (int rc = n > 64 ? gemm_tiles(a, moe, gu_fmt, experts, s) : skinny_matmul(a, moe, gu_fmt, experts, s)) return rc;
+    if (int rc = n > 64 ? gemm_tiles(a, moe, gu_fmt, experts, nullptr, 0, s) : skinny_matmul(a, moe, gu_fmt, experts, s)) return rc;
     // down, each expert on its own rows of g
     MatArgs d = {};
     fh_epilogue de = {};
@@ -395,7 +395,7 @@ extern "C" int fh_moe_experts(const float* x, int64_t ldx, int rows, int64_t dim
     SkinnyMoe dm = {};
     dm.expert_mant = (int64_t)dmb; dm.expert_exps = (int64_t)deb; dm.experts = experts; dm.scale_rows = 0;
     dm.counts = counts;
-    if (int rc = n > 64 ? gemm_tiles(d, dm, down_fmt, experts, s) : skinny_matmul(d, dm, down_fmt, experts, s)) return rc;
+    if (int rc = n > 64 ? gemm_tiles(d, dm, down_fmt, experts, nullptr, 0, s) : skinny_matmul(d, dm, down_fmt, experts, s)) return rc;
     hipLaunchKernelGGL(moe_sum_kernel, dim3(n, (unsigned)((dim + 255) / 256)), dim3(256), 0, s, parts, slot, experts, n,
                        (int)dim, residual ? residual + (int64_t)r0 * dim : nullptr, y + (int64_t)r0 * dim,
                        ssq_out ? ssq_out + (int64_t)r0 * (dim / 16) : nullptr);

@@ -50,6 +50,8 @@ SIGNATURES = {
   "fh_gemv_bfp": ([P, I, L, I, L, L, P, P, I, ctypes.POINTER(Epilogue), P, I, L, P], I),
   "fh_gemv_bfp_k": ([P, I, L, I, L, L, P, P, I, ctypes.POINTER(Epilogue), P, I, L, P], I),
   "fh_gemm_bfp": ([P, I, L, L, L, L, P, P, I, ctypes.POINTER(Epilogue), P, I, L, P], I),
+  "fh_gemm_workspace_bytes": ([L, L, L], S),
+  "fh_gemm_bfp_ws": ([P, I, L, L, L, L, P, P, I, ctypes.POINTER(Epilogue), P, I, L, P, S, P], I),
   "fh_matmul": ([P, I, L, L, P, I, L, L, L, L, L, L, ctypes.POINTER(Program), P, I, L, L, P], I),
   "fh_embed_rows": ([P, I, L, L, P, I, P, P, P], I),
   "fh_attention_workspace_bytes": ([I, I, I, L], S),

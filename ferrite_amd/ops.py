@@ -1,7 +1,7 @@
 """The hot path's operations on torch tensors resident on the GPU: shape and dtype checks on the host, then one call
 into libferrite_hip.so on torch's current stream. torch is the buffer and stream provider only; every computation is
 a HIP kernel of the library, and a missing library raises (ferrite_amd.lib.load)."""
-import ctypes
+import ctypes, functools
 from dataclasses import dataclass
 import torch
 from ferrite_amd import lib
@@ -178,9 +178,20 @@ def _matmul(entry, x, bw, ep, out, out_dtype):
     dev = x.data.device if isinstance(x, Tiles16) else x.device
     out = torch.empty(rows, cols, dtype=out_dtype, device=dev)
   yp, ydt, ldy, _ = _layout(out)
-  lib.call(entry, xp, xdt, ldx, rows, bw.K, bw.N, _ptr(bw.mant), _ptr(bw.exps),
-           lib.DTYPES[bw.fmt], ctypes.byref(ep) if ep is not None else None, yp, ydt, ldy, _stream())
+  args = (xp, xdt, ldx, rows, bw.K, bw.N, _ptr(bw.mant), _ptr(bw.exps), lib.DTYPES[bw.fmt],
+          ctypes.byref(ep) if ep is not None else None, yp, ydt, ldy)
+  n = _gemm_workspace_bytes(rows, bw.K, bw.N) if entry == "fh_gemm_bfp" and rows > 64 else 0
+  if n:  # (freed as this returns: torch's allocator hands it only to later work on this stream)
+    ws = torch.empty(n, dtype=torch.uint8, device=x.device)
+    lib.call("fh_gemm_bfp_ws", *args, _ptr(ws), n, _stream())
+  else:
+    lib.call(entry, *args, _stream())
   return out
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_workspace_bytes(rows, K, N):
+  return lib.load().fh_gemm_workspace_bytes(rows, K, N)
 
 
 def gemv(x, bw, ep=None, out=None, out_dtype=torch.float32):

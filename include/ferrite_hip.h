@@ -189,6 +189,15 @@ int fh_gemv_bfp_k(const void* x, int x_dtype, int64_t ldx, int batch, int64_t K,
  * depend on timing. */
 int fh_gemm_bfp(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t N, const void* w_mant,
                 const uint8_t* w_exps, int fmt, const fh_epilogue* ep, void* y, int y_dtype, int64_t ldy, void* stream);
+/* The same with a workspace (16-byte aligned, fh_gemm_workspace_bytes bytes, no clearing): a matmul of few tiles, a short
+ * prompt's, whose K is cut into parts that different workgroups sum (a call of 65 to ~1000 rows by an 8B model's weights;
+ * 0 bytes where one part is the fastest). The parts are added in order: the same bits every time. With no workspace, or
+ * one too small, K stays whole. */
+size_t fh_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N);
+int fh_gemm_bfp_ws(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t N, const void* w_mant,
+                   const uint8_t* w_exps, int fmt, const fh_epilogue* ep, void* y, int y_dtype, int64_t ldy,
+                   void* workspace, size_t ws_bytes, void* stream);
+
 
 /* ---- the rest of a decode step ------------------------------------------------------------------------------- */
 

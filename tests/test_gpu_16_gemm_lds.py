@@ -1,0 +1,84 @@
+"""The tiled matmul of bf16 rows whose x goes straight into LDS (fh_gemm_lds.hip): every epilogue at the edges of its
+tiles, in one part of K against the kernel that fp32 rows take (the same bf16 products in the same order: the same bits),
+and with K in parts within fp32 summation's error of that. Rows past M of x's buffer hold NaN: none may reach a sum."""
+import ctypes
+import pytest
+import torch
+from ferrite_amd import llama as G
+
+pytestmark = pytest.mark.gpu
+HD = 64
+
+
+def both(ops, lib, x, bw, make, out_shape, dtype, ws_bytes):
+  """The call on fp32 rows (values of bf16), on bf16 rows with K whole, and on bf16 rows with a workspace."""
+  got = []
+  for rows, n in ((x.float(), 0), (x, 0), (x, ws_bytes)):
+    out = torch.full(out_shape, float("nan"), dtype=dtype, device="cuda")
+    ep, state = make(out)
+    ws = torch.full((max(n, 16),), 0xFF, dtype=torch.uint8, device="cuda")
+    lib.call("fh_gemm_bfp_ws", ops._ptr(rows), ops._TORCH[rows.dtype], rows.stride(0), rows.shape[0], bw.K, bw.N, ops._ptr(bw.mant),
+             ops._ptr(bw.exps), lib.DTYPES[bw.fmt], ctypes.byref(ep) if ep is not None else None, ops._ptr(out), ops._TORCH[dtype],
+             out.stride(0), ops._ptr(ws) if n else None, n, ops._stream())
+    torch.cuda.synchronize()
+    got.append([out, *state])
+  return got
+
+
+@pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
+@pytest.mark.parametrize("M,K,N", [(65, 64, 16), (96, 192, 144), (127, 1536, 576), (128, 4096, 128), (129, 320, 2064),
+                                   (200, 4096, 1024), (257, 576, 960), (300, 1024, 4096), (1000, 512, 6144)])
+def test_every_epilogue_at_tile_edges(cuda, fmt, M, K, N):
+  from ferrite_amd import lib, ops
+  g = torch.Generator(device="cuda").manual_seed(M + 3 * K + 7 * N)
+  rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+  x = torch.full((M + 8, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+  x[:M] = rand(M, K)
+  x = x[:M]
+  n = lib.load().fh_gemm_workspace_bytes(M, K, N)
+
+  def check(bw, make, shape, dtype, bound, what):
+    old, one, split = both(ops, lib, x, bw, make, shape, dtype, n)
+    for a, b in zip(old, one): assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), what
+    for a, b in zip(old, split):
+      if not n: assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), what
+      elif a.dtype in (torch.float32, torch.bfloat16): assert ((a.double() - b.double()).abs() <= bound(a.double())).all(), what
+
+  w = rand(K, N) * 0.02
+  bw = ops.pack(w, fmt)
+  mag = (x.double().abs() @ ops.dequant(bw).double().abs())
+  near = 2 ** -21 * mag  # sums of exact products in another order: at most K / 16 roundings of 2^-24 of sum |x w|, K <= 4096 twice over
+  def store(out):
+    parts = torch.zeros(M, N // 16, dtype=torch.int64, device="cuda")
+    return ops.epilogue(lib.EP_STORE, argmax_parts=parts), [parts]
+  check(bw, store, (M, N), torch.float32, lambda a: near, "store")
+  # (bf16 on both sides: each rounding moves its sum by half a bf16 step, at most 2^-8 of it, so 2^-7 between the two)
+  check(bw, lambda out: (None, []), (M, N), torch.bfloat16, lambda a: near + 2 ** -7 * a.abs(), "store bf16")
+  res, cw = rand(M, N), rand(N)
+  def residual(out):
+    ssq, cp = torch.zeros(M, N // 16, device="cuda"), torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+    return ops.epilogue(lib.EP_RESIDUAL, residual=res, ssq_out=ssq, copy_bf16=cp, copy_w=cw), [ssq, cp]
+  def residual_bound(a):
+    if a.shape[1] != N: return 1e-4 * a + 1e-4  # the sums of squares: twice a value's error times the value, 16 of them
+    return near * (1 + cw.abs()) + 2 ** -7 * a.abs()  # (the copy: two bf16 roundings, as above)
+  check(bw, residual, (M, N), torch.float32, residual_bound, "residual")
+  # 1/rms from the rows' own sums of squares
+  ssq_in = x.float().square().reshape(M, K // 16, 16).sum(-1)
+  check(bw, lambda out: (ops.epilogue(lib.EP_STORE, ssq_in=ssq_in, eps=1e-5), []), (M, N), torch.float32, lambda a: near, "1/rms")
+  if N % 32 == 0:
+    check(bw, lambda out: (ops.epilogue(lib.EP_SILU_GATE, split=N // 2), []), (M, N // 2), torch.bfloat16,
+          lambda a: 2 ** -7 * a.abs() + 1e-5 * mag[:, :N // 2] * (1 + mag[:, N // 2:]), "silu")
+  if N % (6 * HD) == 0:  # heads of 64: 4 of q's to each of k's and v's
+    kv = N // (6 * HD)
+    cos, sin = (torch.from_numpy(t).cuda() for t in G.rotary_tables(G.model(dim=HD, heads=1, theta=1e4), 64))
+    places = torch.randint(0, 64, (M,), generator=g, device="cuda", dtype=torch.int32)
+    rows = torch.randperm(M + 9, generator=g, device="cuda")[:M].to(torch.int32)
+    for kind in ("fp32", "bfp8", "bfp4"):
+      def rope(out):
+        cache = ops.kv_cache(2 * kv, M + 9, HD, kind, "cuda")
+        data, dt, length = ops.cache_fields(cache)
+        ep = ops.epilogue(lib.EP_ROPE_KV, heads=4 * kv, kv_heads=kv, head_dim=HD, cos_tab=cos, sin_tab=sin, rope_rows=64, places=places,
+                          cache_rows=rows, cache=data, cache_dtype=dt, cache_len=length)
+        return ep, [data]
+      big = 2 * near.max()
+      check(bw, rope, (M, 4 * kv * HD), torch.float32, lambda a: big + 0 * a, f"rope {kind}")
