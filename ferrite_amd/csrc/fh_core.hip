@@ -210,6 +210,24 @@ extern "C" int fh_embed_rows(const void* table, int table_dtype, int64_t vocab, 
   return check_launch("fh_embed_rows");
 }
 
+// ---- a step's few integers from the host: they travel as kernel arguments, so nothing waits for a copy ------------------
+constexpr int PI_N = 960;  // 3840 bytes of a launch's arguments
+struct PutInts { int32_t v[PI_N]; };
+__global__ __launch_bounds__(PI_N) void put_i32_kernel(PutInts a, int n, int32_t* __restrict__ out) {
+  if ((int)threadIdx.x < n) out[threadIdx.x] = a.v[threadIdx.x];
+}
+
+extern "C" int fh_put_i32(const int32_t* values, int64_t n, int32_t* out, void* stream) {
+  if (!values || !out || n < 1) return fail(FH_EINVAL, "fh_put_i32: need values, out and n >= 1");
+  PutInts a;
+  for (int64_t i = 0; i < n; i += PI_N) {
+    const int m = (int)(n - i < PI_N ? n - i : PI_N);
+    memcpy(a.v, values + i, (size_t)m * 4);
+    hipLaunchKernelGGL(put_i32_kernel, dim3(1), dim3((m + 63) / 64 * 64), 0, as_stream(stream), a, m, out + i);
+  }
+  return check_launch("fh_put_i32");
+}
+
 // ---- argmax of each row: one workgroup a row, the first of equal maxima ------------------------------------------
 __global__ __launch_bounds__(1024) void argmax_kernel(const float* __restrict__ x, int64_t n, int32_t* __restrict__ ids) {
   const float* row = x + (int64_t)blockIdx.x * n;

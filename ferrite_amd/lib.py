@@ -53,6 +53,7 @@ SIGNATURES = {
   "fh_gemm_workspace_bytes": ([L, L, L], S),
   "fh_gemm_bfp_ws": ([P, I, L, L, L, L, P, P, I, ctypes.POINTER(Epilogue), P, I, L, P, S, P], I),
   "fh_matmul": ([P, I, L, L, P, I, L, L, L, L, L, L, ctypes.POINTER(Program), P, I, L, L, P], I),
+  "fh_put_i32": ([P, L, P, P], I),
   "fh_embed_rows": ([P, I, L, L, P, I, P, P, P], I),
   "fh_attention_workspace_bytes": ([I, I, I, L], S),
   "fh_kv_cache_bytes": ([I, I, L, I], S),

@@ -30,6 +30,9 @@ import torch
 from ferrite_amd import lib, ops
 
 
+PUT_MAX = 4096  # a prompt's tokens that go to the GPU as launches' arguments (5 launches); more by copies
+
+
 def model(**c):
   """A config: dim, heads, kv, layers, eps, theta, vocab, ffn, places (RoPE rows), head_dim, rope (Llama 3's scaling),
   tied (output layer = embedding), centered (RMSNorm by 1 + w), as models/llama.py:541-543 keeps them."""
@@ -144,10 +147,10 @@ class Decoder:
     # a step's buffers, fixed so a step replays as a graph
     B = batch
     z = lambda *s: torch.zeros(*s, dtype=torch.float32, device=self.device)
-    self.ids = torch.zeros(B, dtype=torch.int32, device=self.device)
-    self.places = torch.zeros(B, dtype=torch.int32, device=self.device)
-    self.rows = torch.zeros(B, dtype=torch.int32, device=self.device)       # cache row of each row's token
-    self.first = torch.zeros(B, dtype=torch.int32, device=self.device)      # its sequence's first cache row
+    # each row's token, place, its sequence's first cache row and the cache row of its token: one buffer, so that a
+    # step's values from the host go in by one launch
+    self._int = torch.zeros(4, B, dtype=torch.int32, device=self.device)
+    self.ids, self.places, self.first, self.rows = self._int
     self.x, self.ssq = z(B, c.dim), z(B, c.dim // 16)
     self.q, self.att = z(B, c.heads * hd), z(B, c.heads * hd)
     self.h = z(B, c.ffn)
@@ -174,12 +177,32 @@ class Decoder:
 
   def set_rows(self, places, slots=None):
     """Each row's place, and the cache rows: slot s's sequence keeps rows s * context .. (models/llama.py:429-452)."""
+    self._put(places=places, slots=slots)
+
+  def _put(self, ids=None, places=None, slots=None):
+    """The rows' tokens, and their places and slots where places is given: what the host holds by one launch whose
+    arguments they are (ops.put_i32), tensors on the GPU by copies on the stream."""
+    if ids is not None:
+      ids = torch.as_tensor(ids, dtype=torch.int32)
+      if places is None or ids.is_cuda or ids.shape != (self.batch,):
+        if ids.is_cuda or ids.shape != (self.batch,): self.ids.copy_(ids)
+        else: ops.put_i32(ids.numpy(), self.ids)
+        ids = None
+    if places is None: return
     places = torch.as_tensor(places, dtype=torch.int32)
     slots = torch.zeros_like(places) if slots is None else torch.as_tensor(slots, dtype=torch.int32)
     if places.shape != (self.batch,) or slots.shape != (self.batch,): raise ValueError(f"set_rows: {self.batch} places and slots")
-    if (places < 0).any() or (places >= min(self.context, self.c.places)).any(): raise ValueError("a place past the cache or RoPE's tables")
-    if (slots < 0).any() or (slots >= self.slots).any(): raise ValueError(f"a slot outside 0..{self.slots - 1}")
-    self.top = int(places.max())  # (the largest place, kept on the host for advance's check)
+    host = not (places.is_cuda or slots.is_cuda)
+    p, s = (places.numpy(), slots.numpy()) if host else (places, slots)
+    if (p < 0).any() or (p >= min(self.context, self.c.places)).any(): raise ValueError("a place past the cache or RoPE's tables")
+    if (s < 0).any() or (s >= self.slots).any(): raise ValueError(f"a slot outside 0..{self.slots - 1}")
+    self.top = int(p.max())  # (the largest place, kept on the host for advance's check)
+    if host:
+      first = s * np.int32(self.part)
+      v = [p, first, first + p]
+      ops.put_i32(np.concatenate(v if ids is None else [ids.numpy(), *v]), self._int[1 if ids is None else 0:])
+      return
+    if ids is not None: ops.put_i32(ids.numpy(), self.ids)
     self.places.copy_(places)
     self.first.copy_(slots * self.part)
     self.rows.copy_(slots * self.part + places)
@@ -274,9 +297,11 @@ class Decoder:
     P = self._prefill_buffers(T)
     ids_t, places, rows = P.ids[:T], P.places[:T], P.rows[:T]
     x, ssq, xn, q, att, h = P.x[:T], P.ssq[:T], P.xn[:T], P.q[:T], P.att[:T], P.h[:T]
-    ids_t.copy_(torch.as_tensor(ids, dtype=torch.int32))
-    places.copy_(torch.arange(p0, p0 + T, dtype=torch.int32))
-    rows.copy_(places + slot * self.part)
+    at = np.arange(p0, p0 + T, dtype=np.int32)
+    if T <= PUT_MAX:
+      for v, out in ((ids, ids_t), (at, places), (at + np.int32(slot * self.part), rows)): ops.put_i32(v, out)
+    else:
+      for v, out in ((ids, ids_t), (at, places), (at + np.int32(slot * self.part), rows)): out.copy_(torch.as_tensor(v, dtype=torch.int32))
     ops.embed_rows(self.embed, ids_t, x, ssq)
     # (each RMSNorm a pass of its own here: at 2048 rows the tiled kernel's per-tile sums of the rows' squares cost
     # more than fh_rms_rows; the batched decode takes the residual epilogues' scaled copies instead)
@@ -298,8 +323,7 @@ class Decoder:
   def step(self, ids=None, places=None, slots=None, replay=True):
     """One step: the logits (fp32, [batch][vocab]) and picks for tokens ids at places. With replay, the step runs as
     a HIP graph captured on the first call (every later step launches the same kernels: places are data)."""
-    if ids is not None: self.ids.copy_(torch.as_tensor(ids, dtype=torch.int32))
-    if places is not None: self.set_rows(places, slots)
+    if ids is not None or places is not None: self._put(ids, places, slots)
     if not replay:
       self._step()
     else:

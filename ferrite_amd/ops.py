@@ -3,6 +3,7 @@ into libferrite_hip.so on torch's current stream. torch is the buffer and stream
 a HIP kernel of the library, and a missing library raises (ferrite_amd.lib.load)."""
 import ctypes, functools
 from dataclasses import dataclass
+import numpy as np
 import torch
 from ferrite_amd import lib
 
@@ -226,6 +227,16 @@ def matmul(a, b, program=None, out=None, out_dtype=torch.float32):
   sb = b.stride(0) if b.shape[0] > 1 else 0
   lib.call("fh_matmul", _ptr(a), _TORCH[a.dtype], sa, a.stride(1), _ptr(b), _TORCH[b.dtype], sb, b.stride(1), batch, M, K, N,
            ctypes.byref(program) if program is not None else None, _ptr(out), _DT_OUT[out.dtype], out.stride(0), out.stride(1), _stream())
+  return out
+
+
+def put_i32(values, out):
+  """out (a contiguous int32 tensor on the GPU) from as many integers of the host's, in stream order and with no copy
+  (fh_put_i32): values a list, or an int32 array or CPU tensor."""
+  _dev(out)
+  v = np.ascontiguousarray(values, np.int32)
+  if out.dtype != torch.int32 or not out.is_contiguous() or v.size != out.numel(): raise ValueError(f"put_i32: {v.size} integers into {tuple(out.shape)} {out.dtype}")
+  lib.call("fh_put_i32", v.ctypes.data, v.size, _ptr(out), _stream())
   return out
 
 

@@ -119,3 +119,30 @@ def test_read_probe_reads_every_byte(cuda):
     assert got == np.bitwise_xor.reduce(data), (words, blocks)
   with pytest.raises(ValueError):
     lib.call("fh_read_probe", src.data_ptr(), 10, sink.data_ptr(), blocks, None)
+
+
+@pytest.mark.parametrize("n", [1, 64, 959, 960, 961, 1920, 2500])
+def test_put_i32_from_the_host(cuda, n):
+  """Integers of the host into device memory as launch arguments (fh_put_i32): every value, in place, none past the end,
+  the host's buffer free to change once the call has returned; a Decoder's rows from lists and from GPU tensors the same."""
+  from ferrite_amd import ops
+  out = torch.full((n + 64,), -7, dtype=torch.int32, device="cuda")
+  v = np.random.default_rng(n).integers(-2**31, 2**31, n, dtype=np.int64).astype(np.int32)
+  keep = v.copy()
+  ops.put_i32(v, out[:n])
+  v[:] = 0
+  got = out.cpu().numpy()
+  assert np.array_equal(got[:n], keep) and (got[n:] == -7).all()
+
+
+def test_decoder_rows_from_host_and_gpu(cuda):
+  from ferrite_amd import llama as G
+  c = G.model(dim=64, heads=1, kv=1, layers=1, eps=1e-5, theta=1e4, vocab=64, ffn=64, places=32, tied=True)
+  dec = G.Decoder(c, G.random_weights(c), batch=3, context=32, slots=4)
+  ids, places, slots = [5, 9, 63], [0, 31, 7], [2, 0, 3]
+  want = [ids, places, [64, 0, 96], [64, 31, 103]]
+  gpu = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+  for i, p, s in ((ids, places, slots), (gpu(ids), gpu(places), gpu(slots)), (gpu(ids), places, slots), (ids, gpu(places), gpu(slots))):
+    for t in (dec.ids, dec.places, dec.first, dec.rows): t.fill_(1)
+    dec.step(i, p, s, replay=False)
+    assert [t.tolist() for t in (dec.ids, dec.places, dec.first, dec.rows)] == want and dec.top == 31
