@@ -100,9 +100,8 @@ def load():
 
 def call(name, *args):
   """Calls an entry point that returns a status; a negative one raises with fh_last_error()'s message."""
-  lib = load()
-  rc = getattr(lib, name)(*args)
-  if rc < 0: raise ERRORS.get(rc, RuntimeError)(lib.fh_last_error().decode())
+  rc = getattr(_lib or load(), name)(*args)
+  if rc < 0: raise ERRORS.get(rc, RuntimeError)(_lib.fh_last_error().decode())
   return rc
 
 

@@ -10,12 +10,13 @@ from ferrite_amd import lib
 _TORCH = {torch.float32: lib.F32, torch.bfloat16: lib.BF16}
 
 
-def _ptr(t):
-  return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+def _ptr(t):  # (a pointer argument takes a plain integer)
+  return t.data_ptr() if t is not None else None
 
 
 def _stream():
-  return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+  """The current device's current stream, raw (what torch.cuda.current_stream().cuda_stream is, without the objects)."""
+  return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(*ts):
@@ -160,8 +161,8 @@ def _layout(t):
   if isinstance(t, Tiles16):
     _dev(t.data)
     return t.data.data_ptr(), lib.BF16_T16, t.cols, t.rows
-  _dev(t)
-  return _ptr(t), _TORCH[t.dtype], t.stride(0), t.shape[0]
+  if not t.is_cuda: _dev(t)
+  return t.data_ptr(), _TORCH[t.dtype], t.stride(0), t.shape[0]
 
 
 def _matmul(entry, x, bw, ep, out, out_dtype):
