@@ -70,28 +70,39 @@ __device__ inline uint4 raw_bf16x8(const CacheRaw& r) {
   }
 }
 
-template <int HD, int CF>
-__global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefArgs a) {
+// KS 1: as above. KS 4, for a prompt of few rows: a workgroup takes 32 query rows, its four waves every fourth key tile,
+// each staging its own (one buffer a wave, no workgroup barrier) and keeping a softmax of its own; the four partial
+// outputs meet in LDS at the end. Four times the workgroups, each a quarter of the key tiles long: what a short prompt
+// waits for is one workgroup's chain of tiles (200 rows after 824, 32 heads of 128: 30.4 -> 20.1 us, 64 workgroups of 16
+// tiles before, 224 of 4 now; 9 heads of 64: 20.6 -> 10.9).
+template <int HD, int CF, int KS>
+__global__ __launch_bounds__(256, KS == 1 ? 2 : 1) void attention_prefill_kernel(PrefArgs a) {
   constexpr int KLD = HD + 8;        // K tile row in LDS (bf16): 16-byte aligned, banks spread
   constexpr int VLD = PA_BK + 8;     // V^T tile row (bf16)
-  __shared__ __attribute__((aligned(16))) uint16_t Ks2[2][PA_BK * KLD];  // two buffers: a tile's arithmetic reads
-  __shared__ __attribute__((aligned(16))) uint16_t Vt2[2][HD * VLD];     // one while the next tile is stored in the other
+  constexpr int BQ = KS == 1 ? PA_BQ : 32;  // the workgroup's query rows
+  constexpr int NB = KS == 1 ? 2 : KS;      // buffers: two, a tile's arithmetic reading one while the next is stored in
+                                            // the other; or one a wave
+  __shared__ __attribute__((aligned(16))) uint16_t Ks2[NB][PA_BK * KLD];
+  __shared__ __attribute__((aligned(16))) uint16_t Vt2[NB][HD * VLD];
 
-  const int ntiles = (a.T + PA_BQ - 1) / PA_BQ;
+  const int ntiles = (a.T + BQ - 1) / BQ;
   // the longest tiles first; the second half of the heads shortest first, so that the two workgroups a CU holds
   // (blocks b and b + half the grid) together walk about the same number of key tiles whatever b is
   const bool flip = (int)blockIdx.y >= ((int)gridDim.y + 1) / 2;
   const int qt = flip ? (int)blockIdx.x : ntiles - 1 - (int)blockIdx.x, h = blockIdx.y;
   const int kvh = h / (a.heads / a.kv_heads);
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int t = KS == 1 ? (int)threadIdx.x : lane;          // this thread among those that load a tile
+  constexpr int TT = KS == 1 ? 256 : 64;
   const int ql = lane & 31, hh = lane >> 5;
-  const int qrow = qt * PA_BQ + wave * 32 + ql;            // this lane's query row
+  const int row0 = qt * BQ + (KS == 1 ? wave * 32 : 0);    // the wave's first query row
+  const int qrow = row0 + ql;                              // this lane's
   const int qr = min(qrow, a.T - 1);
   const int64_t qplace = a.p0 + qr;
-  const int64_t last_key = a.p0 + min(qt * PA_BQ + PA_BQ, a.T) - 1;  // the workgroup's last key (its last row's place)
+  const int64_t last_key = a.p0 + min(qt * BQ + BQ, a.T) - 1;  // the workgroup's last key (its last row's place)
   const int nkt = (int)(last_key / PA_BK) + 1;
   // the wave's first row's place: a key tile wholly at or before it is visible to every row of the wave (no mask)
-  const int64_t wave_first = a.p0 + min(qt * PA_BQ + wave * 32, a.T - 1);
+  const int64_t wave_first = a.p0 + min(row0, a.T - 1);
   // scores kept in base 2 (scale times log2 e): the softmax's exponentials are then the chip's exp2 alone
   const float scale2 = a.scale * 1.44269504088896341f;
 
@@ -119,20 +130,23 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefArgs a) {
   const int64_t vrow = (int64_t)(a.kv_heads + kvh) * a.cache_len + a.slot_row;
 
   // a tile's loads: K, 64 rows x HD, a thread NK pieces of 8; V, a thread (past NVT threads none) 4 keys x 8 dimensions
-  constexpr int NK = PA_BK * HD / 8 / 256, NVT = (PA_BK / 4) * (HD / 8);
-  static_assert(NK * 256 == PA_BK * HD / 8 && NVT <= 256, "tile pieces a thread");
-  CacheRaw kraw[NK], vraw[4];
+  constexpr int NK = PA_BK * HD / 8 / TT, NVT = (PA_BK / 4) * (HD / 8), NV = (NVT + TT - 1) / TT;
+  static_assert(NK * TT == PA_BK * HD / 8 && (NVT <= TT || NVT % TT == 0), "tile pieces a thread");
+  CacheRaw kraw[NK], vraw[NV][4];
   auto load_tile = [&](int kt) {
     const int64_t k0 = (int64_t)kt * PA_BK;
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
-      const int i = t + 256 * j, r = i / (HD / 8), c = (i % (HD / 8)) * 8;
+      const int i = t + TT * j, r = i / (HD / 8), c = (i % (HD / 8)) * 8;
       kraw[j] = cache_raw<HD, CF>(a, krow + min(k0 + r, last_key), c);
     }
-    if (t < NVT) {
-      const int kq = t % (PA_BK / 4), dg = t / (PA_BK / 4);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) vraw[j] = cache_raw<HD, CF>(a, vrow + min(k0 + 4 * kq + j, last_key), 8 * dg);
+    for (int v = 0; v < NV; ++v) {
+      const int u = t + TT * v;
+      if (u >= NVT) break;
+      const int kq = u % (PA_BK / 4), dg = u / (PA_BK / 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vraw[v][j] = cache_raw<HD, CF>(a, vrow + min(k0 + 4 * kq + j, last_key), 8 * dg);
     }
   };
   // a tile's loads, as bf16, into buffer b: K rows; V^T, a thread's 4 keys x 8 dimensions as 8 rows of 4 keys. In a
@@ -144,15 +158,18 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefArgs a) {
     uint16_t* Vt = Vt2[b];
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
-      const int i = t + 256 * j, r = i / (HD / 8), c = (i % (HD / 8)) * 8;
+      const int i = t + TT * j, r = i / (HD / 8), c = (i % (HD / 8)) * 8;
       *(uint4*)(Ks + r * KLD + c) = raw_bf16x8<CF>(kraw[j]);
     }
-    if (t < NVT) {
-      const int kq = t % (PA_BK / 4), dg = t / (PA_BK / 4);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int u = t + TT * v;
+      if (u >= NVT) break;
+      const int kq = u % (PA_BK / 4), dg = u / (PA_BK / 4);
       uint32_t lo[4][4];  // [key][pair of dims]
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const uint4 w = raw_bf16x8<CF>(vraw[j]);
+        const uint4 w = raw_bf16x8<CF>(vraw[v][j]);
         lo[j][0] = w.x; lo[j][1] = w.y; lo[j][2] = w.z; lo[j][3] = w.w;
       }
 #pragma unroll
@@ -164,14 +181,23 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefArgs a) {
       }
     }
   };
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-  for (int kt = 0; kt < nkt; ++kt) {
+  const int kt0 = KS == 1 ? 0 : wave;  // this wave's first tile (with KS 4 it may have none)
+  if (kt0 < nkt) {
+    load_tile(kt0);
+    if (KS == 1) store_tile(0);
+  }
+  if (KS == 1) __syncthreads();
+  for (int kt = kt0; kt < nkt; kt += KS) {
     const int64_t k0 = (int64_t)kt * PA_BK;
-    const uint16_t* Ks = Ks2[kt & 1];
-    const uint16_t* Vt = Vt2[kt & 1];
-    if (kt + 1 < nkt) load_tile(kt + 1);  // the next tile's loads in flight during this one's arithmetic
+    const uint16_t* Ks = Ks2[KS == 1 ? kt & 1 : wave];
+    const uint16_t* Vt = Vt2[KS == 1 ? kt & 1 : wave];
+    if (KS > 1) {  // (the wave's own buffer: its reads of the last tile were done before these writes in its order)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      store_tile(wave);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (kt + KS < nkt) load_tile(kt + KS);  // the next tile's loads in flight during this one's arithmetic
 
     // S^T for the tile's two blocks of 32 keys: block kb's value r of lane (ql, hh) is key 32 kb + 8 (r / 4) + 4 hh +
     // r % 4, query ql
@@ -212,12 +238,14 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefArgs a) {
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
     const float mn = fmaxf(m, mt == PA_MASKED ? PA_MASKED : mt * scale2);
     const float alpha = __builtin_amdgcn_exp2f(m - mn);
+    // (KS 4: a wave's tiles so far may all lie past a row's place, its max still the mask: then every exponent is 0)
+    const float shift = KS > 1 && mn == PA_MASKED ? 0.f : mn;
     float rsum = 0.f;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(s[kb][r], scale2, -mn));
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[kb][r], scale2, -shift));
         s[kb][r] = p;
         rsum += p;
       }
@@ -244,8 +272,59 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefArgs a) {
           acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)&vv, pf, acc[d], 0, 0, 0);
         }
       }
-    if (kt + 1 < nkt) store_tile((kt + 1) & 1);  // (the other buffer: its last readers passed the previous barrier)
+    if (KS == 1) {
+      if (kt + 1 < nkt) store_tile((kt + 1) & 1);  // (the other buffer: its last readers passed the previous barrier)
+      __syncthreads();
+    }
+  }
+
+  if constexpr (KS > 1) {
+    // the waves' parts meet: each leaves its sums, its max and its exponents' sum in LDS (where the tiles were); wave w
+    // then adds block w of the dimensions over the parts, in order, each part times 2^(its max - the largest)
+    __shared__ float ml[KS][2][64];
+    constexpr int PB = HD / 32;  // blocks of 32 dimensions
+    float* parts = (float*)Ks2;
+    constexpr int IN = (int)(sizeof(Ks2) / (16 * 64 * 4));  // blocks that fit where K was; the rest where V was
+    auto part = [&](int w, int d) { const int i = w * PB + d; return (i < IN ? parts + i * 1024 : (float*)Vt2 + (i - IN) * 1024) + lane; };
+    static_assert((KS * PB - IN) * 4096 <= (int)sizeof(Vt2), "the parts' place");
     __syncthreads();
+#pragma unroll
+    for (int d = 0; d < PB; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part(wave, d)[64 * r] = acc[d][r];
+    ml[wave][0][lane] = m;
+    ml[wave][1][lane] = l;
+    __syncthreads();
+    if (wave >= PB) return;
+    float top = PA_MASKED;
+#pragma unroll
+    for (int w = 0; w < KS; ++w) top = fmaxf(top, ml[w][0][lane]);
+    float f[KS];
+    l = 0.f;
+#pragma unroll
+    for (int w = 0; w < KS; ++w) {
+      f[w] = __builtin_amdgcn_exp2f(ml[w][0][lane] - top);  // (0 for a part that saw no key: its max is the mask)
+      l = fmaf(f[w], ml[w][1][lane], l);
+    }
+    if (qrow < a.T) {
+      const float inv = 1.f / l;
+      const int64_t base = (int64_t)qrow * a.ldo + (int64_t)h * HD;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float x = 0.f;
+#pragma unroll
+          for (int w = 0; w < KS; ++w) x = fmaf(f[w], part(w, wave)[64 * (4 * g + i)], x);
+          v[i] = x * inv;
+        }
+        const int dim = 32 * wave + 8 * g + 4 * hh;
+        if (a.o_bf16) *(uint2*)((uint16_t*)a.o + base + dim) = make_uint2(pack2_rne(v[0], v[1]), pack2_rne(v[2], v[3]));
+        else *(float4*)((float*)a.o + base + dim) = make_float4(v[0], v[1], v[2], v[3]);
+      }
+    }
+    return;
   }
 
   // o[row][h * HD + dim]: block d's value r of lane (ql, hh) is dimension 32 d + 8 (r / 4) + 4 hh + r % 4
@@ -337,13 +416,13 @@ __global__ __launch_bounds__(256) void rms_rows_kernel(const float* x, int64_t l
   for (int i = threadIdx.x; i < dim; i += 256) put(i, xr[i], rs);
 }
 
-template <int HD>
+template <int HD, int KS>
 static void launch_prefill(int cf, dim3 g, dim3 b, hipStream_t s, const PrefArgs& a) {
   switch (cf) {
-    case FH_F32: hipLaunchKernelGGL((attention_prefill_kernel<HD, FH_F32>), g, b, 0, s, a); break;
-    case FH_BF16: hipLaunchKernelGGL((attention_prefill_kernel<HD, FH_BF16>), g, b, 0, s, a); break;
-    case FH_BFP8: hipLaunchKernelGGL((attention_prefill_kernel<HD, FH_BFP8>), g, b, 0, s, a); break;
-    default: hipLaunchKernelGGL((attention_prefill_kernel<HD, FH_BFP4>), g, b, 0, s, a); break;
+    case FH_F32: hipLaunchKernelGGL((attention_prefill_kernel<HD, FH_F32, KS>), g, b, 0, s, a); break;
+    case FH_BF16: hipLaunchKernelGGL((attention_prefill_kernel<HD, FH_BF16, KS>), g, b, 0, s, a); break;
+    case FH_BFP8: hipLaunchKernelGGL((attention_prefill_kernel<HD, FH_BFP8, KS>), g, b, 0, s, a); break;
+    default: hipLaunchKernelGGL((attention_prefill_kernel<HD, FH_BFP4, KS>), g, b, 0, s, a); break;
   }
 }
 
@@ -369,10 +448,25 @@ extern "C" int fh_attention_prefill(const float* q, int64_t ldq, const void* cac
   a.cache_exps = (const uint8_t*)cache + kv_exps_at(cache_dtype, kv_heads, cache_len, head_dim);
   a.T = T; a.heads = heads; a.kv_heads = kv_heads; a.scale = 1.0f / sqrtf((float)head_dim);
   a.p0 = p0; a.slot_row = slot_row; a.o = o; a.ldo = ldo; a.o_bf16 = o_dtype == FH_BF16;
-  const dim3 g((T + PA_BQ - 1) / PA_BQ, heads), b(256);
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    return n;
+  }();
   hipStream_t s = as_stream(stream);
-  if (head_dim == 128) launch_prefill<128>(cache_dtype, g, b, s, a);
-  else launch_prefill<64>(cache_dtype, g, b, s, a);
+  // the keys split among a workgroup's waves where its tiles of 32 rows are still one round of a workgroup a CU and there
+  // is more than one key tile (32 heads of 128: 100 rows 9.0 -> 7.5 us, 64 after 1900 51 -> 30; past one round it loses:
+  // 300 rows 13 -> 18, 512 19 -> 24; one key tile 5.2 -> 7.1)
+  const bool split = (int64_t)((T + 31) / 32) * heads <= cus && p0 + T > PA_BK;
+  const int bq = split ? 32 : PA_BQ;
+  const dim3 g((T + bq - 1) / bq, heads), b(256);
+  if (split) {
+    if (head_dim == 128) launch_prefill<128, 4>(cache_dtype, g, b, s, a);
+    else launch_prefill<64, 4>(cache_dtype, g, b, s, a);
+  } else {
+    if (head_dim == 128) launch_prefill<128, 1>(cache_dtype, g, b, s, a);
+    else launch_prefill<64, 1>(cache_dtype, g, b, s, a);
+  }
   return check_launch("fh_attention_prefill");
 }
 
