@@ -112,6 +112,9 @@ struct SkinnyMoe {
   // grid's third dimension
   const int32_t* counts; const int32_t* x_rows; const float* row_w;
   int row0;
+  // K in `splits` parts (0: whole), part p's outputs split_y elements after part p - 1's: a store of fp32 sums that
+  // the reader adds up (gemm_tiles' 128-row tiles only)
+  int splits; int64_t split_y;
 };
 
 // x @ W for up to 64 rows a pass on the matrix cores (fh_skinny.hip); a's epilogue already checked

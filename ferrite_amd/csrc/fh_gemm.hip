@@ -616,7 +616,11 @@ int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void*
   // faster (the Mixtral layer at 1000 tokens: 1168 us against 1279; at 300 even, at 100 616 against 485)
   if (gemm_lds_takes(a)) {
     if (g.counts) {
-      if (a.M <= 512) return gemm_lds(a, g, fmt, experts, gemm_lds_plan(a.M, a.K, a.N, experts, false), nullptr, s);
+      if (a.M <= 512) {
+        GemmPlan p = gemm_lds_plan(a.M, a.K, a.N, experts, false);
+        if (g.splits > 1) p.splits = g.splits;
+        return gemm_lds(a, g, fmt, experts, p, nullptr, s);
+      }
     } else {
       GemmPlan p = gemm_lds_plan(a.M, a.K, a.N, 0, workspace != nullptr);
       if (gemm_lds_bytes(p, a.M, a.N) > ws_bytes) p = gemm_lds_plan(a.M, a.K, a.N, 0, false);
@@ -624,6 +628,7 @@ int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void*
       if (WNv != 3 || tiles3 > cus || p.us <= 8 + 1.9 * (double)(a.K / GM_BK)) return gemm_lds(a, g, fmt, 1, p, (float*)workspace, s);
     }
   }
+  if (g.splits > 1) return fail(FH_EUNSUP, "gathered GEMM: K in parts for up to 512 bf16 rows whose K is a multiple of 64");
   const bool pp = WNv != 0;
   const int TMv = (pp || (!g.counts && tiles2 <= cus)) ? 2 : 1;
   const int64_t tiles_m = (a.M + GM_BM * TMv - 1) / (GM_BM * TMv);

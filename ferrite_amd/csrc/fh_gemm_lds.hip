@@ -32,13 +32,13 @@ typedef __attribute__((address_space(3))) uint32_t* gl_lds;
 // kernel was 90 KB of code, and a call of one K step took 13 us).
 constexpr int GL_LDC = 68;
 __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe& g, const float* cs, int tn, int wc, int64_t m0,
-                                               int64_t M, int64_t ybase, int lane, const float* rs) {
+                                               int64_t M, int64_t ybase, int lane, const float* rs, int64_t y0 = 0) {
   const int kind = a.kind;
   if (a.P == 1) {  // a lane 4 columns of a row, 4 rows a pass
     const int q = lane & 15, c = 4 * q, lc = wc + (c & 31);
     const int64_t run = tile_run<GL_RUNS>(a, tn, 4 * (q >> 3) + (lc >> 4)), col = run * 16 + (lc & 15);
     const bool res = kind == FH_EP_RESIDUAL;
-    const bool vec = !(a.ldy & 3) && !((uintptr_t)a.y & 15) && !(res && ((uintptr_t)a.residual & 15));
+    const bool vec = !((a.ldy | y0) & 3) && !((uintptr_t)a.y & 15) && !(res && ((uintptr_t)a.residual & 15));
     float4 old[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {  // (the rows' loads before the first store, which may alias them)
@@ -49,7 +49,7 @@ __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = (lane >> 4) + 4 * i;
-      const int64_t m = m0 + r, at = (ybase + m) * a.ldy + col;
+      const int64_t m = m0 + r, at = y0 + (ybase + m) * a.ldy + col;
       const bool ok = m < M && run >= 0;
       float4 v = *(const float4*)(cs + r * GL_LDC + c);
       if (rs) { v.x *= rs[r]; v.y *= rs[r]; v.z *= rs[r]; v.w *= rs[r]; }
@@ -162,9 +162,12 @@ __device__ __forceinline__ void row_scales(const MatArgs& a, float* rs, int n, i
   }
 }
 
-template <bool FOUR, int WR, int TM, bool SPLIT>
+// MODE 0: K whole; 1: a part of K, its sums left in `parts`; 2: a part of K whose outputs go g.split_y elements after the
+// part before's (a store's only: whoever reads them adds them up)
+template <bool FOUR, int WR, int TM, int MODE>
 __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits,
                                                                                   float* parts) {
+  constexpr bool SPLIT = MODE != 0;
   constexpr int NW = 2 * WR, BM = 32 * WR * TM, NS = TM == 2 || SPLIT ? 2 : 3;
   constexpr int AB = BM * GL_BK * 2, BB = GL_BK * GL_BN * 2;
   constexpr int IA = AB / 1024 / NW;           // a wave's loads of x a step (1 KiB, 8 rows each)
@@ -278,7 +281,7 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
   const int fr = lane & 31, fh8 = lane >> 5;
   const int rm = (lane >> 2) & 3, rq = lane & 3, rg = (lane >> 4) & 1;
   auto compute = [&](const char* sa, const char* sb) {
-    if (TM == 1 && !live) return;
+    if (TM == 1 && MODE != 1 && !live) return;  // (an expert's 128-row tile is often a third empty)
 #pragma unroll
     for (int kk = 0; kk < GL_BK; kk += 16) {
       bf16x8 fa[TM], fb[2];
@@ -338,7 +341,7 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
 #undef GL_B
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0x0070);  // (no load into LDS outlives its workgroup)
-  if (SPLIT) {
+  if (MODE == 1) {
     if (!live) return;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -353,15 +356,15 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
   }
   __syncthreads();  // the stages are free: each wave's outputs, 16 rows at a time, in a part of x's of its own
   constexpr int CW = 16 * GL_LDC * 4, WPA = AB / CW;
-  static_assert(SPLIT || 5 * WPA >= NW, "the outputs' place");
-  float* cs = (float*)((wave < WPA ? a0 : wave < 2 * WPA ? a1 : NS == 3 ? a2 : b1) + wave % WPA * CW);
-  float* rs_s = (float*)b0 + wave * 32 * TM;
+  static_assert(MODE == 1 || (NS + 2) * WPA >= NW, "the outputs' place");
+  float* cs = (float*)((wave < WPA ? a0 : wave < 2 * WPA ? a1 : wave < 3 * WPA ? (NS == 3 ? a2 : b1) : b0) + wave % WPA * CW);
+  float* rs_s = (float*)(b0 + BB) - 32 * TM * (wave + 1);
   if (a.ssq_in) row_scales(a, rs_s, 32 * TM, m0 + wr, lane, 64);  // (each wave its own rows' 1/rms, where the weight was)
   for (int u = 0; u < 2 * TM && m0 + wr + 16 * u < M; ++u) {
 #pragma unroll
     for (int ii = 0; ii < TM; ++ii)  // (the accumulators' indices stay constants)
       if (ii == u >> 1) block_to_lds(cs, acc[ii], u & 1, lane);
-    block_epilogue(a, g, cs, tn, wc, m0 + wr + 16 * u, M, ybase, lane, a.ssq_in ? rs_s + 16 * u : nullptr);
+    block_epilogue(a, g, cs, tn, wc, m0 + wr + 16 * u, M, ybase, lane, a.ssq_in ? rs_s + 16 * u : nullptr, MODE == 2 ? part * g.split_y : 0);
   }
 }
 
@@ -452,9 +455,10 @@ int gemm_lds(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, const G
   const int64_t n = g.counts ? (tm * tn * p.splits + 7) / 8 * 8 : tm * tn * p.splits;
   const dim3 grid((unsigned)n, g.counts ? experts : 1);
 #define GL(F, WR, TM) do { \
-    if (p.splits < 2) hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, false>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, 1, parts); \
+    if (p.splits < 2) hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, 0>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, 1, parts); \
+    else if (TM == 1 && g.split_y) hipLaunchKernelGGL((gemm_lds_kernel<F, WR, 1, 2>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
     else { \
-      hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, true>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
+      hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, 1>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
       hipLaunchKernelGGL((split_sum_kernel<WR, TM>), dim3((unsigned)(tm * tn * WR * TM), g.counts ? experts : 1), dim3(256), 0, s, a, g, (int)tm, (int)tn, p.splits, (const float*)parts); \
     } } while (0)
 #define GL_F(WR, TM) do { if (fmt == FH_BFP4) GL(true, WR, TM); else GL(false, WR, TM); } while (0)

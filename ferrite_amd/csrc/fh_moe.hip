@@ -16,6 +16,7 @@
 // expert's own fp32 rows; a last kernel adds each row's experts in expert order (no atomics: the result does not
 // depend on timing) onto the residual. An expert no row picked reads no weight.
 #include <math.h>
+#include <algorithm>
 #include "fh_epilogue.h"
 
 namespace fh {
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(256) void moe_prep_kernel(const float* x, int64_t l
 // y[row] = residual[row] + the row's experts' outputs (parts: each expert's own rows) in expert order, and y's sums of
 // squares by 16 columns; a workgroup 256 columns of a row
 __global__ __launch_bounds__(256) void moe_sum_kernel(const float* parts, const int32_t* slot, int experts, int n, int dim,
-                                                      const float* residual, float* y, float* ssq_out) {
+                                                      const float* residual, float* y, float* ssq_out, int splits) {
   const int64_t row = blockIdx.x;
   const int c = blockIdx.y * 256 + threadIdx.x;
   float v = 0.f;
@@ -260,7 +261,10 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const float* parts, const 
     v = residual ? residual[row * dim + c] : 0.f;
     for (int e = 0; e < experts; ++e) {
       const int sl = slot[row * experts + e];
-      if (sl >= 0) v += parts[((int64_t)e * n + sl) * dim + c];
+      if (sl < 0) continue;
+      float p = parts[((int64_t)e * n + sl) * dim + c];
+      for (int s = 1; s < splits; ++s) p += parts[((int64_t)(s * experts + e) * n + sl) * dim + c];  // (K's parts, in order)
+      v += p;
     }
     y[row * dim + c] = v;
   }
@@ -272,8 +276,16 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const float* parts, const 
 }
 
 // A pass's workspace (n rows, E experts): counts [E], rows_of [E][n], row_w [E][n], slot [n][E], xn [n][dim] bf16,
-// g [E][n][ffn] bf16, parts [E][n][dim] fp32, each region 256-byte aligned
-struct MoeSpace { size_t counts, rows_of, row_w, slot, xn, g, parts, total; };
+// g [E][n][ffn] bf16, parts [splits][E][n][dim] fp32, each region 256-byte aligned
+struct MoeSpace { size_t counts, rows_of, row_w, slot, xn, g, parts, total; int splits; };
+// down's K in parts where a prompt's few rows an expert leave its tiles of 128 x 128 one a CU or fewer (a tile an expert
+// for every 128 columns): two or more workgroups a CU then share its long K (the Mixtral layer at 300 tokens: 256 tiles
+// of 224 steps, down 270 -> 190 us), moe_sum adding the parts
+static int moe_splits(int64_t n, int64_t E, int64_t ffn, int64_t dim) {
+  if (n <= 64 || n > 512 || ffn % 64 || dim % 64) return 1;
+  const int64_t tiles = E * ((dim + 127) / 128), s = 512 / tiles;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(s, 4), ffn / 64 / 16));
+}
 static MoeSpace moe_space(int64_t n, int64_t E, int64_t ffn, int64_t dim) {
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   MoeSpace m;
@@ -284,7 +296,8 @@ static MoeSpace moe_space(int64_t n, int64_t E, int64_t ffn, int64_t dim) {
   m.xn = m.slot + up(n * E * 4);
   m.g = m.xn + up(n * dim * 2);
   m.parts = m.g + up(E * n * ffn * 2);
-  m.total = m.parts + up(E * n * dim * 4);
+  m.splits = moe_splits(n, E, ffn, dim);
+  m.total = m.parts + up(m.splits * E * n * dim * 4);
   return m;
 }
 
@@ -334,7 +347,8 @@ extern "C" size_t fh_moe_workspace_bytes(int rows, int experts, int64_t ffn, int
   const int64_t pass = moe_pass(rows, experts, ffn, dim);
   const int64_t r = rows < pass ? rows : pass;  // a pass's rows
   if (r < 1 || experts < 1 || ffn < 1 || dim < 1) return 0;
-  return moe_space(r, experts, ffn, dim).total;
+  // (the last pass's fewer rows may have down's K in parts, and so take more than a whole pass's)
+  return std::max(moe_space(r, experts, ffn, dim).total, rows > pass && rows % pass ? moe_space(rows % pass, experts, ffn, dim).total : 0);
 }
 
 extern "C" int fh_moe_experts(const float* x, int64_t ldx, int rows, int64_t dim, const float* norm_w, const float* ssq_in,
@@ -395,10 +409,11 @@ extern "C" int fh_moe_experts(const float* x, int64_t ldx, int rows, int64_t dim
     SkinnyMoe dm = {};
     dm.expert_mant = (int64_t)dmb; dm.expert_exps = (int64_t)deb; dm.experts = experts; dm.scale_rows = 0;
     dm.counts = counts;
+    if (m.splits > 1) { dm.splits = m.splits; dm.split_y = (int64_t)experts * n * dim; }
     if (int rc = n > 64 ? gemm_tiles(d, dm, down_fmt, experts, nullptr, 0, s) : skinny_matmul(d, dm, down_fmt, experts, s)) return rc;
     hipLaunchKernelGGL(moe_sum_kernel, dim3(n, (unsigned)((dim + 255) / 256)), dim3(256), 0, s, parts, slot, experts, n,
                        (int)dim, residual ? residual + (int64_t)r0 * dim : nullptr, y + (int64_t)r0 * dim,
-                       ssq_out ? ssq_out + (int64_t)r0 * (dim / 16) : nullptr);
+                       ssq_out ? ssq_out + (int64_t)r0 * (dim / 16) : nullptr, m.splits);
     if (int rc = check_launch("fh_moe_experts")) return rc;
   }
   return FH_OK;
