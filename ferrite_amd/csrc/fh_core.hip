@@ -23,48 +23,122 @@ int check_launch(const char* kernel) {
   return FH_OK;
 }
 
-// ---- packing: one thread a block of 16 ---------------------------------------------------------------------------
+// ---- packing: one thread a block of 16 (or four) ------------------------------------------------------------------
 // A block is (outer, inner): outer = the run of 16 (N/16 of them for FH_AXIS_N, K/16 for FH_AXIS_K), inner = the other
 // axis's index. Its value j sits at src[inner * s_inner + outer * s_outer + j * s_elem]; its bytes go to
 // mant[(outer * n_inner + inner) * (16 or 8)] and its exponent to exps[outer * n_inner + inner].
-template <bool FOUR, bool BF16>
+
+// 16 bf16 values' magnitudes under their largest exponent, as stored: 16 bytes (bfp8) or the first 8 (bfp4)
+template <bool FOUR>
+__device__ inline void pack_block(const uint32_t (&bits)[16], uint32_t& top, uint32_t (&w)[4]) {
+  top = 0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const uint32_t e = (bits[j] >> 7) & 255u;
+    top = e > top ? e : top;
+  }
+  w[0] = w[1] = w[2] = w[3] = 0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const uint32_t q = bfp_magnitude(bits[j], top, FOUR);
+    const int32_t sq = (bits[j] >> 15) && q ? -(int32_t)q : (int32_t)q;  // no sign on a zero
+    if (FOUR) w[j / 8] |= ((uint32_t)sq & 15u) << (4 * (j % 8));
+    else w[j / 4] |= ((uint32_t)sq & 255u) << (8 * (j % 4));
+  }
+}
+__device__ inline uint32_t pack_load(const void* src, bool bf16, int64_t at) {
+  return bf16 ? ((const uint16_t*)src)[at] : bf16_rne(((const uint32_t*)src)[at]);
+}
+
+// A thread IN neighbouring blocks. Along K (a run down 16 rows) lanes lie along the columns, so every load of a wave is
+// whole lines; bound by the read and the write (14336 x 4096: 4.9 TB/s of bf16 into bfp8, 5.8 of fp32, a column a
+// thread). IN 4, one 8-byte load a row for four columns: bf16 into bfp4 only, whose instructions are the most a byte
+// (4096 x 28672 80.4 -> 66.6 us; into bfp8 77 -> 79, fp32 104 -> 112, 576 x 1536 3.0 -> 4.6).
+template <bool FOUR, bool BF16, int IN>
 __global__ __launch_bounds__(256) void pack_kernel(const void* __restrict__ src, int64_t n_outer, int64_t n_inner,
                                                    int64_t s_outer, int64_t s_inner, int64_t s_elem,
                                                    uint8_t* __restrict__ mant, uint8_t* __restrict__ exps) {
-  int64_t blk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t blk = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * IN;
   if (blk >= n_outer * n_inner) return;
-  int64_t outer = blk / n_inner, inner = blk % n_inner;
+  const int64_t outer = blk / n_inner, inner = blk % n_inner;
   const int64_t base = inner * s_inner + outer * s_outer;
-  uint32_t bits[16];
-  uint32_t top = 0;
+  uint32_t bits[IN][16];
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    uint32_t b;
-    if (BF16) b = ((const uint16_t*)src)[base + j * s_elem];
-    else b = bf16_rne(((const uint32_t*)src)[base + j * s_elem]);
-    bits[j] = b;
-    uint32_t e = (b >> 7) & 255u;
-    top = e > top ? e : top;
+    if constexpr (IN == 1) {
+      bits[0][j] = pack_load(src, BF16, base + j * s_elem);
+    } else {
+      static_assert(BF16 && IN == 4, "four bf16 columns a load");
+      const uint2 v = *(const uint2*)((const uint16_t*)src + base + j * s_elem);
+      bits[0][j] = v.x & 0xFFFFu; bits[1][j] = v.x >> 16; bits[2][j] = v.y & 0xFFFFu; bits[3][j] = v.y >> 16;
+    }
   }
-  exps[blk] = (uint8_t)top;
-  if (!FOUR) {
-    uint32_t w[4] = {0, 0, 0, 0};
+  uint32_t e4 = 0;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      uint32_t q = bfp_magnitude(bits[j], top, false);
-      int32_t sq = (bits[j] >> 15) && q ? -(int32_t)q : (int32_t)q;  // no sign on a zero
-      w[j / 4] |= ((uint32_t)sq & 255u) << (8 * (j % 4));
-    }
-    *(uint4*)(mant + blk * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-  } else {
-    uint32_t w[2] = {0, 0};
+  for (int i = 0; i < IN; ++i) {
+    uint32_t top, w[4];
+    pack_block<FOUR>(bits[i], top, w);
+    e4 |= top << (8 * i);
+    if (FOUR) *(uint2*)(mant + (blk + i) * 8) = make_uint2(w[0], w[1]);
+    else *(uint4*)(mant + (blk + i) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+  if constexpr (IN == 1) exps[blk] = (uint8_t)e4;
+  else {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      uint32_t q = bfp_magnitude(bits[j], top, true);
-      int32_t sq = (bits[j] >> 15) && q ? -(int32_t)q : (int32_t)q;
-      w[j / 8] |= ((uint32_t)sq & 15u) << (4 * (j % 8));
+    for (int i = 0; i < IN; ++i) exps[blk + i] = (uint8_t)(e4 >> (8 * i));
+  }
+}
+
+// Along N (a run along a row): a workgroup 64 rows by 16 runs, its reads along the rows (512 bytes of bf16 a row in one
+// piece), the packed blocks met in LDS so that a run's 64 rows go out as the 1 KiB (512 B) they are in the layout. A
+// thread a block, straight from memory, takes 32 bytes a row a lane and each line from several XCDs: 4096 x 28672 of bf16
+// into bfp8 259 us that way, 81 this (fp32 289 -> 130). vec: rows at 16-byte alignment.
+template <bool FOUR, bool BF16>
+__global__ __launch_bounds__(256) void pack_rows_kernel(const void* __restrict__ src, int64_t K, int64_t runs, int64_t ld, int vec,
+                                                        uint8_t* __restrict__ mant, uint8_t* __restrict__ exps) {
+  constexpr int RB = FOUR ? 8 : 16, RS = 64 * RB + 16;  // a run's rows in LDS (16 bytes more: the runs' banks apart)
+  __shared__ __attribute__((aligned(16))) uint8_t ms[16 * RS];
+  __shared__ uint8_t es[16][64];
+  const int64_t k0 = (int64_t)blockIdx.y * 64, o0 = (int64_t)blockIdx.x * 16;
+  const int t = threadIdx.x, run = t & 15;
+  if (o0 + run < runs) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (t >> 4) + 16 * i;
+      if (k0 + row >= K) break;
+      const int64_t at = (k0 + row) * ld + (o0 + run) * 16;
+      uint32_t bits[16];
+      if (vec) {
+#pragma unroll
+        for (int q = 0; q < (BF16 ? 2 : 4); ++q) {
+          const uint4 v = ((const uint4*)((const char*)src + at * (BF16 ? 2 : 4)))[q];
+          const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if (BF16) { bits[(8 * q + 2 * j) & 15] = u[j] & 0xFFFFu; bits[(8 * q + 2 * j + 1) & 15] = u[j] >> 16; }
+            else bits[4 * q + j] = bf16_rne(u[j]);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) bits[j] = pack_load(src, BF16, at + j);
+      }
+      uint32_t top, w[4];
+      pack_block<FOUR>(bits, top, w);
+      es[run][row] = (uint8_t)top;
+      if (FOUR) *(uint2*)(ms + run * RS + row * 8) = make_uint2(w[0], w[1]);
+      else *(uint4*)(ms + run * RS + row * 16) = make_uint4(w[0], w[1], w[2], w[3]);
     }
-    *(uint2*)(mant + blk * 8) = make_uint2(w[0], w[1]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // a wave a run's 64 rows
+    const int r = (t >> 6) + 4 * i, row = t & 63;
+    if (o0 + r >= runs || k0 + row >= K) continue;
+    const int64_t blk = (o0 + r) * K + k0 + row;
+    if (FOUR) *(uint2*)(mant + blk * 8) = *(const uint2*)(ms + r * RS + row * 8);
+    else *(uint4*)(mant + blk * 16) = *(const uint4*)(ms + r * RS + row * 16);
+    exps[blk] = es[r][row];
   }
 }
 
@@ -136,17 +210,30 @@ extern "C" int fh_bfp_pack(const void* src, int src_dtype, int64_t K, int64_t N,
   if (!src || !mant || !exps) return fail(FH_EINVAL, "fh_bfp_pack: null pointer");
   if (src_dtype != FH_F32 && src_dtype != FH_BF16) return fail(FH_EINVAL, "fh_bfp_pack: src is FH_F32 or FH_BF16");
   if (fmt != FH_BFP8 && fmt != FH_BFP4) return fail(FH_EINVAL, "fh_bfp_pack: fmt is FH_BFP8 or FH_BFP4");
-  int64_t blocks = g.n_outer * g.n_inner;
-  dim3 grid((unsigned)((blocks + 255) / 256)), block(256);
+  const bool four = fmt == FH_BFP4, bf = src_dtype == FH_BF16;
+  const int64_t blocks = g.n_outer * g.n_inner;
   hipStream_t s = as_stream(stream);
   auto m = (uint8_t*)mant;
-  if (fmt == FH_BFP8) {
-    if (src_dtype == FH_F32) hipLaunchKernelGGL((pack_kernel<false, false>), grid, block, 0, s, src, g.n_outer, g.n_inner, g.s_outer, g.s_inner, g.s_elem, m, exps);
-    else hipLaunchKernelGGL((pack_kernel<false, true>), grid, block, 0, s, src, g.n_outer, g.n_inner, g.s_outer, g.s_inner, g.s_elem, m, exps);
-  } else {
-    if (src_dtype == FH_F32) hipLaunchKernelGGL((pack_kernel<true, false>), grid, block, 0, s, src, g.n_outer, g.n_inner, g.s_outer, g.s_inner, g.s_elem, m, exps);
-    else hipLaunchKernelGGL((pack_kernel<true, true>), grid, block, 0, s, src, g.n_outer, g.n_inner, g.s_outer, g.s_inner, g.s_elem, m, exps);
+  const dim3 block(256);
+  // (past ~2 MB of values; 576 x 1536 takes 4.5 us a thread a block, 4.9 in these tiles)
+  if (axis == FH_AXIS_N && blocks >= 131072 && (K + 63) / 64 <= 65535) {
+    const int vec = !((uintptr_t)src & 15) && ld % (bf ? 8 : 4) == 0;
+    const dim3 grid((unsigned)((g.n_outer + 15) / 16), (unsigned)((K + 63) / 64));
+#define PK_ROWS(F, B) hipLaunchKernelGGL((pack_rows_kernel<F, B>), grid, block, 0, s, src, K, g.n_outer, ld, vec, m, exps)
+    if (four) { if (bf) PK_ROWS(true, true); else PK_ROWS(true, false); }
+    else { if (bf) PK_ROWS(false, true); else PK_ROWS(false, false); }
+#undef PK_ROWS
+    return check_launch("fh_bfp_pack");
   }
+  // (four columns a thread where the rows' pieces are whole and aligned and the chip stays full)
+  const bool wide = axis == FH_AXIS_K && bf && four && blocks >= (1 << 20) && N % 4 == 0 && ld % 4 == 0 && !((uintptr_t)src & 7);
+  const int64_t threads = wide ? blocks / 4 : blocks;
+  const dim3 grid((unsigned)((threads + 255) / 256));
+#define PK(F, B, IN) hipLaunchKernelGGL((pack_kernel<F, B, IN>), grid, block, 0, s, src, g.n_outer, g.n_inner, g.s_outer, g.s_inner, g.s_elem, m, exps)
+  if (wide) PK(true, true, 4);
+  else if (four) { if (bf) PK(true, true, 1); else PK(true, false, 1); }
+  else { if (bf) PK(false, true, 1); else PK(false, false, 1); }
+#undef PK
   return check_launch("fh_bfp_pack");
 }
 

@@ -58,3 +58,33 @@ def test_prefill_attention_of_few_rows(cuda, kind, heads, kv, hd, T, p0):
     s = (qb[:, h] @ k.T.contiguous()) / hd ** 0.5
     want = torch.softmax(s.masked_fill(late, -torch.inf), -1) @ v
     assert ((got[:, h] - want).abs() <= 2 ** -8 * v.abs().max()).all(), h
+
+
+@pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("K,N,pad,off", [(16, 16, 0, 0), (63, 272, 0, 0), (64, 256, 8, 0), (65, 240, 4, 0), (128, 4112, 0, 0), (80, 64, 1, 0), (96, 48, 0, 1),
+                                         (2064, 1040, 0, 0), (1104, 2064, 2, 0), (2048, 1072, 8, 1), (4096, 4112, 0, 0), (4112, 4104, 4, 0)])
+def test_packing_at_every_stride(cuda, fmt, dtype, K, N, pad, off):
+  """fh_bfp_pack along both axes, in its wide and its narrow loads (whole tiles and ragged ones, row strides and bases at
+  odd alignments), against the oracle's blocks: magnitudes and exponents bit for bit, as gpt2.bfp makes them."""
+  import numpy as np
+  from ferrite_amd import lib, ops
+  from oracle import bfp as O
+  rng = np.random.default_rng(K + N + pad)
+  w = (rng.normal(0, 1, (K, N)) * np.exp(rng.normal(0, 3, (K, N)))).astype(np.float32)
+  w[rng.random((K, N)) < 0.05] = 0
+  buf = torch.full((off + K * (N + pad),), float("nan"), dtype=dtype, device="cuda")
+  x = buf[off:].view(K, N + pad)[:, :N]
+  x.copy_(torch.from_numpy(w))
+  vals = x.float().cpu().numpy()
+  for axis in (lib.AXIS_N, lib.AXIS_K):
+    if (K if axis == lib.AXIS_K else N) % 16: continue
+    bw = ops.pack(x, fmt, axis)
+    q, top = O.bfp_parts(vals if axis == lib.AXIS_N else vals.T, fmt)  # [inner][outer * 16], [inner][outer]
+    assert np.array_equal(bw.exps.cpu().numpy().reshape(top.shape[1], top.shape[0]), top.T), axis
+    m = bw.mant.cpu().numpy().reshape(top.shape[1], top.shape[0], -1)
+    if fmt == "bfp8": got = m.view(np.int8).astype(np.int32)
+    else:
+      got = np.stack([m & 15, m >> 4], -1).reshape(*m.shape[:2], 16).astype(np.int32)
+      got = np.where(got > 7, got - 16, got)
+    assert np.array_equal(got, q.reshape(q.shape[0], -1, 16).transpose(1, 0, 2)), axis
