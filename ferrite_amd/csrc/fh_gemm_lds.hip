@@ -181,7 +181,7 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
   __shared__ __attribute__((aligned(16))) char b0[BB];
   __shared__ __attribute__((aligned(16))) char b1[BB];
 
-  // this workgroup's expert, part of K and tile: tiles (a part's one after another) go to the XCDs in contiguous ranges,
+  // this workgroup's expert, part of K and tile: tiles (each its parts one after another) go to the XCDs in contiguous ranges,
   // in groups of 8 row tiles
   int64_t M = a.M, ybase = 0;
   const uint8_t* wmant = a.mant;
@@ -203,8 +203,8 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
   } else if (tiles * splits % 8 == 0) {
     id = (id % 8) * (tiles * splits / 8) + id / 8;
   }
-  const int part = SPLIT ? id / tiles : 0;
-  if (SPLIT) id -= part * tiles;
+  const int part = SPLIT ? id % splits : 0;  // (a tile's parts on one XCD: their sums meet in its L2)
+  if (SPLIT) id /= splits;
   const int per_group = 8 * tiles_n, first_m = id / per_group * 8, gm = min(tiles_m - first_m, 8);
   const int tm = first_m + (id % per_group) % gm, tn = (id % per_group) / gm;
   const int64_t m0 = (int64_t)tm * BM;
@@ -369,7 +369,9 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
 }
 
 // The split tiles' sums: a wave 16 rows by 2 x 32 columns of a tile (half of a wave's block there), its parts added in order,
-// four parts' loads in flight at a time, then the epilogue. Bound by reading the parts once (splits x 4 bytes an output).
+// four parts' loads in flight at a time, then the epilogue. Bound by reading the parts once (splits x 4 bytes an output),
+// from the L2 of the XCD that wrote them (o at 200 rows in bfp4, both launches: 30.6 -> 24.7 us against parts dealt to
+// the XCDs part by part).
 template <int WR, int TM>
 __global__ __launch_bounds__(256) void split_sum_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits, const float* parts) {
   constexpr int NW = 2 * WR, BM = 32 * WR * TM;
@@ -385,7 +387,9 @@ __global__ __launch_bounds__(256) void split_sum_kernel(MatArgs a, SkinnyMoe g, 
     tiles_m = (int)((M + BM - 1) / BM);
     tiles = tiles_m * tiles_n;
   }
-  const int lane = threadIdx.x & 63, u = blockIdx.x * 4 + (threadIdx.x >> 6);  // unit u: (tile, wave, i, half)
+  // (workgroups dealt to the XCDs in contiguous ranges, as the tiles' were: a tile's parts are in this XCD's L2)
+  const int nb = gridDim.x, blk = nb % 8 == 0 ? (int)(blockIdx.x % 8) * (nb / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
+  const int lane = threadIdx.x & 63, u = blk * 4 + (threadIdx.x >> 6);  // unit u: (tile, wave, i, half)
   const int half = u & 1, i = (u >> 1) % TM, wave = (u >> 1) / TM % NW, id = (u >> 1) / (TM * NW);
   if (id >= tiles) return;
   const int per_group = 8 * tiles_n, first_m = id / per_group * 8, gm = min(tiles_m - first_m, 8);
@@ -423,8 +427,8 @@ bool gemm_lds_takes(const MatArgs& a) {
 // Rows a tile and K's parts: the least of a model of the call's time in us, its constants measured at the 8B shapes (bfp8
 // and bfp4 alike): 8 a launch; a step of a 256-row tile 1.0 with a workgroup a CU, 1.15 a round of them with the chip
 // full; of a 128-row tile 0.8 alone on a CU, 1.38 two a CU; K in parts, 6 more for the second launch and the parts written
-// and read back at 6.5 TB/s. (Measured, 200 rows after 1 part -> the plan's: o 4096 x 4096 75 -> 29 us in 8, down
-// 14336 x 4096 203 -> 48 in 8, qkv 4096 x 6144 67 -> 31 in 4; 1024 rows: o 72 -> 53 and down 214 -> 133 in 2; at 2048
+// and read back at 6.5 TB/s. (Measured, 200 rows, 1 part -> the plan's: o 4096 x 4096 75 -> 26 us in 8, down
+// 14336 x 4096 203 -> 45 in 8, qkv 4096 x 6144 67 -> 30 in 5; 1024 rows: o 72 -> 53 and down 214 -> 133 in 2; at 2048
 // rows every shape is fastest in one part.) A gathered matmul (experts > 0), whose rows an expert the host does not know,
 // takes 128-row tiles in one part.
 GemmPlan gemm_lds_plan(int64_t M, int64_t K, int64_t N, int experts, bool may_split) {

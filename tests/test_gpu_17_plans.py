@@ -88,3 +88,23 @@ def test_packing_at_every_stride(cuda, fmt, dtype, K, N, pad, off):
       got = np.stack([m & 15, m >> 4], -1).reshape(*m.shape[:2], 16).astype(np.int32)
       got = np.where(got > 7, got - 16, got)
     assert np.array_equal(got, q.reshape(q.shape[0], -1, 16).transpose(1, 0, 2)), axis
+
+
+@pytest.mark.parametrize("M,K,N", [(200, 64, 33600), (200, 96, 51200), (300, 64, 51200), (65, 96, 640), (2048, 96, 6144)])
+def test_gemm_program_tiles(cuda, M, K, N):
+  """A fused elementwise program on bf16 rows' matmul (the kernels that fh_gemm_lds.hip's does not replace: programs, and a
+  K that is not whole steps of 64), in each of their tile widths, against float64: exact products, fp32 sums."""
+  import ctypes
+  from ferrite_amd import lib, ops
+  g = torch.Generator(device="cuda").manual_seed(M + N)
+  x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+  bw = ops.pack(torch.randn(K, N, generator=g, device="cuda") * 0.02, "bfp8")
+  wv = ops.dequant(bw).double()
+  mag, want = x.double().abs() @ wv.abs(), x.double() @ wv
+  p = lib.Program()
+  p.n_ops, p.op[0], p.a[0], p.b[0], p.imm[0] = 1, lib.OP["mul"], lib.OPND_ACC, lib.OPND_IMM, 0.5
+  for program, scale in ((p, 0.5), (None, 1.0)):
+    ep = ops.epilogue(lib.EP_PROGRAM if program is not None else lib.EP_STORE)
+    if program is not None: ep.program = ctypes.pointer(program)
+    got = ops.gemm(x, bw, ep)
+    assert ((got.double() - scale * want).abs() <= 2 ** -21 * mag + 1e-30).all()
