@@ -126,12 +126,13 @@ __global__ __launch_bounds__(skinny_threads(XBF16, MB)) void skinny_kernel(MatAr
       erun[j] = exps + run * a.K;
     }
     // x: row 16 b + lane % 16, k 8 (lane / 16) .. + 7 of each 32 k. In rows, a wave's 16-byte loads take 16 rows'
-    // 64 bytes each (rows past M read row M - 1); in tiles of 16 rows (FH_BF16_T16, bf16), 1 KiB in a piece
+    // 64 bytes each (rows past M read row M - 1); in tiles of 16 rows (FH_BF16_T16, bf16), 1 KiB in a piece (a block past
+    // the rows' last tile reads that tile: 33 to 48 rows take the kernel of 4 blocks, and their buffer holds 3)
     const bool tiles = XBF16 && a.x_tiles;
     const char* xp[MB];
 #pragma unroll
     for (int b = 0; b < MB; ++b)
-      xp[b] = tiles ? (const char*)a.x + ((int64_t)16 * b * a.ldx + 8 * lane) * 2
+      xp[b] = tiles ? (const char*)a.x + ((int64_t)16 * min(b, (M - 1) >> 4) * a.ldx + 8 * lane) * 2
                     : (const char*)a.x + (xrow(min(16 * b + (lane & 15), M - 1)) * a.ldx + (int64_t)e * moe.expert_xcols + 8 * (lane >> 4)) * (XBF16 ? 2 : 4);
     const int xk = tiles ? 32 : XBF16 ? 2 : 4;  // bytes a column of k moves the loads on
     const int last = r1 - SK_BK;  // (r1 - r0 is a multiple of 64: K is)

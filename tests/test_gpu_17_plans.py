@@ -108,3 +108,15 @@ def test_gemm_program_tiles(cuda, M, K, N):
     if program is not None: ep.program = ctypes.pointer(program)
     got = ops.gemm(x, bw, ep)
     assert ((got.double() - scale * want).abs() <= 2 ** -21 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("M", [33, 36, 47, 48, 49])
+@pytest.mark.parametrize("K,N", [(64, 48), (576, 960), (1536, 576)])
+def test_tile_rows_between_block_counts(cuda, M, K, N):
+  """Rows in tiles of 16 where the kernel's blocks (4) are more than the rows' tiles (3 for 33 to 48 rows): the tiles past
+  the last are not read (the buffer ends there), and the outputs are the plain rows', bit for bit."""
+  from ferrite_amd import ops
+  g = torch.Generator(device="cuda").manual_seed(M + K)
+  x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+  bw = ops.pack(torch.randn(K, N, generator=g, device="cuda") * 0.02, "bfp8")
+  assert torch.equal(ops.gemm(ops.to_tiles16(x, float("nan")), bw), ops.gemm(x, bw))
