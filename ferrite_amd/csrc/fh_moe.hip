@@ -286,7 +286,9 @@ static int moe_splits(int64_t n, int64_t E, int64_t ffn, int64_t dim) {
   const int64_t tiles = E * ((dim + 127) / 128), s = 512 / tiles;
   return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(s, 4), ffn / 64 / 16));
 }
-static MoeSpace moe_space(int64_t n, int64_t E, int64_t ffn, int64_t dim) {
+// (as many parts of down's K as fit `bytes`; one, whatever it takes: a workspace sized for more rows, whose passes have K
+// whole, may be smaller than fewer rows' in parts, and holds them in fewer parts)
+static MoeSpace moe_space(int64_t n, int64_t E, int64_t ffn, int64_t dim, size_t bytes) {
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   MoeSpace m;
   m.counts = 0;
@@ -296,9 +298,10 @@ static MoeSpace moe_space(int64_t n, int64_t E, int64_t ffn, int64_t dim) {
   m.xn = m.slot + up(n * E * 4);
   m.g = m.xn + up(n * dim * 2);
   m.parts = m.g + up(E * n * ffn * 2);
-  m.splits = moe_splits(n, E, ffn, dim);
-  m.total = m.parts + up(m.splits * E * n * dim * 4);
-  return m;
+  for (m.splits = moe_splits(n, E, ffn, dim);; --m.splits) {
+    m.total = m.parts + up(m.splits * E * n * dim * 4);
+    if (m.splits == 1 || m.total <= bytes) return m;
+  }
 }
 
 }  // namespace fh
@@ -338,7 +341,7 @@ constexpr int64_t MOE_BUDGET = (int64_t)1 << 30;
 static int64_t moe_pass(int64_t rows, int64_t experts, int64_t ffn, int64_t dim) {
   if (rows <= 64) return 64;
   int64_t p = 2048;
-  while (p > 128 && (int64_t)moe_space(p, experts, ffn, dim).total > MOE_BUDGET) p /= 2;
+  while (p > 128 && (int64_t)moe_space(p, experts, ffn, dim, 0).total > MOE_BUDGET) p /= 2;
   return p;
 }
 
@@ -346,9 +349,9 @@ extern "C" size_t fh_moe_workspace_bytes(int rows, int experts, int64_t ffn, int
   if (rows < 1 || experts < 1 || ffn < 1 || dim < 1) return 0;
   const int64_t pass = moe_pass(rows, experts, ffn, dim);
   const int64_t r = rows < pass ? rows : pass;  // a pass's rows
-  if (r < 1 || experts < 1 || ffn < 1 || dim < 1) return 0;
   // (the last pass's fewer rows may have down's K in parts, and so take more than a whole pass's)
-  return std::max(moe_space(r, experts, ffn, dim).total, rows > pass && rows % pass ? moe_space(rows % pass, experts, ffn, dim).total : 0);
+  return std::max(moe_space(r, experts, ffn, dim, MOE_BUDGET).total,
+                  rows > pass && rows % pass ? moe_space(rows % pass, experts, ffn, dim, MOE_BUDGET).total : 0);
 }
 
 extern "C" int fh_moe_experts(const float* x, int64_t ldx, int rows, int64_t dim, const float* norm_w, const float* ssq_in,
@@ -362,17 +365,17 @@ extern "C" int fh_moe_experts(const float* x, int64_t ldx, int rows, int64_t dim
   if (experts < 1 || experts > 256) return fail(FH_EUNSUP, "fh_moe_experts: at most 256 experts");
   if ((gu_fmt != FH_BFP8 && gu_fmt != FH_BFP4) || (down_fmt != FH_BFP8 && down_fmt != FH_BFP4)) return fail(FH_EINVAL, "fh_moe_experts: weights are FH_BFP8 or FH_BFP4");
   if (norm_w && !ssq_in) return fail(FH_EINVAL, "fh_moe_experts: the RMSNorm prologue needs ssq_in");
-  if (ws_bytes < fh_moe_workspace_bytes(rows, experts, ffn, dim)) return fail(FH_EINVAL, "fh_moe_experts: workspace too small");
+  const int pass = (int)moe_pass(rows, experts, ffn, dim);
+  if (ws_bytes < moe_space(rows < pass ? rows : pass, experts, ffn, dim, 0).total) return fail(FH_EINVAL, "fh_moe_experts: workspace too small");
   hipStream_t s = as_stream(stream);
   const int64_t gu_n = 2 * ffn;
   size_t mb, eb;
   if (int rc = fh_bfp_bytes(dim, gu_n, gu_fmt, FH_AXIS_N, &mb, &eb)) return rc;
   size_t dmb, deb;
   if (int rc = fh_bfp_bytes(ffn, dim, down_fmt, FH_AXIS_N, &dmb, &deb)) return rc;
-  const int pass = (int)moe_pass(rows, experts, ffn, dim);
   for (int r0 = 0; r0 < rows; r0 += pass) {
     const int n = rows - r0 < pass ? rows - r0 : pass;
-    const MoeSpace m = moe_space(n, experts, ffn, dim);
+    const MoeSpace m = moe_space(n, experts, ffn, dim, std::min(ws_bytes, (size_t)MOE_BUDGET));
     char* w = (char*)workspace;
     int32_t* counts = (int32_t*)(w + m.counts);
     int32_t* rows_of = (int32_t*)(w + m.rows_of);

@@ -285,7 +285,8 @@ int fh_moe_route(const float* x, int64_t ldx, int rows, int64_t dim, const float
  * down: the experts' [ffn][dim] weights packed one after another. An expert no row picked reads no weight. residual
  * NULL: y is the sum alone; ssq_out: y's sums of squares by 16 columns. On the matrix cores, x and the SwiGLU outputs
  * in bf16 (fh_gemm_bfp's arithmetic); the experts' outputs summed in expert order. dim and ffn multiples of 64.
- * Workspace: fh_moe_workspace_bytes (a pass of 64 rows' gate_up and down outputs). */
+ * Workspace: fh_moe_workspace_bytes (a pass's gate_up and down outputs; one sized for more rows serves fewer, down's K then
+ * in the parts that fit it). */
 size_t fh_moe_workspace_bytes(int rows, int experts, int64_t ffn, int64_t dim);
 int fh_moe_experts(const float* x, int64_t ldx, int rows, int64_t dim, const float* norm_w, const float* ssq_in, float eps,
                    int centered, int experts, int64_t ffn, const void* gu_mant, const uint8_t* gu_exps, int gu_fmt,

@@ -120,3 +120,27 @@ def test_tile_rows_between_block_counts(cuda, M, K, N):
   x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
   bw = ops.pack(torch.randn(K, N, generator=g, device="cuda") * 0.02, "bfp8")
   assert torch.equal(ops.gemm(ops.to_tiles16(x, float("nan")), bw), ops.gemm(x, bw))
+
+
+@pytest.mark.parametrize("rows,sized", [(512, 513), (512, 600), (300, 513), (129, 257)])
+def test_moe_in_a_workspace_sized_for_more_rows(cuda, rows, sized):
+  """down's K goes in parts for 65 to 512 rows only, so more rows' workspace can be the smaller one: it still serves fewer
+  rows (in the parts that fit), with the larger workspace's results but for the order of fp32 sums of its 4096 products."""
+  from ferrite_amd import lib, ops
+  E, dim, ffn = 2, 256, 4096
+  g = torch.Generator(device="cuda").manual_seed(rows)
+  gu, dn = (torch.randn(*s, generator=g, device="cuda") * 0.05 for s in ((E, dim, 2 * ffn), (E, ffn, dim)))
+  ex = ops.pack_experts(gu, dn, "bfp8")
+  x = torch.randn(rows, dim, generator=g, device="cuda")
+  dense = torch.rand(rows, E, generator=g, device="cuda")
+  want = ops.moe_experts(x, ex, dense)
+  need, have = lib.load().fh_moe_workspace_bytes(rows, E, ffn, dim), lib.load().fh_moe_workspace_bytes(sized, E, ffn, dim)
+  ws, got = torch.empty(have, dtype=torch.uint8, device="cuda"), torch.empty(rows, dim, device="cuda")
+  lib.call("fh_moe_experts", x.data_ptr(), dim, rows, dim, None, None, 1e-5, 0, E, ffn, ex.gate_up.mant.data_ptr(), ex.gate_up.exps.data_ptr(),
+           lib.DTYPES["bfp8"], ex.down.mant.data_ptr(), ex.down.exps.data_ptr(), lib.DTYPES["bfp8"], dense.data_ptr(), got.data_ptr(),
+           None, None, ws.data_ptr(), have, torch.cuda.current_stream().cuda_stream)
+  if sized == 513 and rows == 512: assert need > have
+  # (4096 products an expert summed in fp32 in 16s on the matrix cores: fewer than 2^9 roundings of 2^-24 of the sum of
+  # their magnitudes in each order; twice that sum as plain fp32 has it covers the rounding of h and the weights)
+  mag = sum(dense[:, e:e + 1] * ((torch.nn.functional.silu(x @ gu[e, :, :ffn]) * (x @ gu[e, :, ffn:])).abs() @ dn[e].abs()) for e in range(E))
+  assert ((got - want).abs() <= 2 * 2 * 2 ** -15 * mag).all()
