@@ -182,7 +182,7 @@ def _matmul(entry, x, bw, ep, out, out_dtype):
   yp, ydt, ldy, _ = _layout(out)
   args = (xp, xdt, ldx, rows, bw.K, bw.N, _ptr(bw.mant), _ptr(bw.exps), lib.DTYPES[bw.fmt],
           ctypes.byref(ep) if ep is not None else None, yp, ydt, ldy)
-  n = _gemm_workspace_bytes(rows, bw.K, bw.N) if entry == "fh_gemm_bfp" and rows > 64 else 0
+  n = _gemm_workspace_bytes(rows, bw.K, bw.N) if entry == "fh_gemm_bfp" and rows > 64 and xdt == lib.BF16 else 0
   if n:  # (freed as this returns: torch's allocator hands it only to later work on this stream)
     ws = torch.empty(n, dtype=torch.uint8, device=x.device)
     lib.call("fh_gemm_bfp_ws", *args, _ptr(ws), n, _stream())

@@ -131,6 +131,9 @@ def test_tiles_refused_past_64_rows(cuda):
   xt = ops().tiles16(65, 256)
   with pytest.raises(NotImplementedError, match="FH_BF16_T16"):
     ops().gemm(xt, bw)
+  wide = ops().pack(torch.from_numpy(rng.normal(0, 0.02, (4096, 64)).astype(np.float32)).cuda(), "bfp8")
+  with pytest.raises(NotImplementedError, match="FH_BF16_T16"):  # (a shape whose K bf16 rows would have in parts)
+    ops().gemm(ops().tiles16(65, 4096), wide)
   with pytest.raises(NotImplementedError, match="FH_BF16_T16"):
     ops().gemm(torch.zeros(65, 256, device="cuda"), bw, out=ops().tiles16(65, 64))
   with pytest.raises(ValueError):  # (the GEMV writes rows only)
