@@ -21,6 +21,12 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 // fp32 to bf16 bits, rounded to nearest even (models/gpt2.py:16-18 without packer)
 __host__ __device__ inline uint32_t bf16_rne(uint32_t b) { return (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16; }
 __device__ inline uint32_t bf16_rne_f(float f) { return bf16_rne(__float_as_uint(f)); }
+// between a wave's writes to LDS and its other lanes' reads of them, or reads and the next writes: the wave's LDS accesses
+// run in order, so this holds the compiler to that order and emits nothing
+__device__ inline void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 __device__ inline float bf16_to_f(uint32_t h) { return __uint_as_float(h << 16); }
 // FH_BF16_T16: element (r, c) of bf16 rows of length ld in tiles of 16 rows, 8 columns of the 16 rows together
 __host__ __device__ inline int64_t tile16_at(int64_t r, int64_t c, int64_t ld) {

@@ -417,6 +417,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(MatArgs a, SkinnyMoe g, 
   }
 #pragma unroll
   for (int r = 0; r < 16; ++r) cs[(8 * ((r & 7) >> 2) + 4 * (lane >> 5) + (r & 3)) * GL_LDC + 32 * (r >> 3) + (lane & 31)] = acc[r];
+  wave_lds_order();
   block_epilogue(a, g, cs, tn, (wave & 1) * 32, m0, M, ybase, lane, a.ssq_in ? rs : nullptr);
 }
 
@@ -439,6 +440,8 @@ GemmPlan gemm_lds_plan(int64_t M, int64_t K, int64_t N, int experts, bool may_sp
     const int64_t tiles = (M + bm - 1) / bm * ((N + GL_BN - 1) / GL_BN), all = K / GL_BK;
     for (int s = 1; s <= (may_split ? 16 : 1) && (s == 1 || all / s >= 4); ++s) {
       const int64_t t = tiles * s;
+      // (parts of at most 256 MB: past it the tiles are over a thousand already, and parts save the last round's rest alone)
+      if (s > 1 && t * bm * GL_BN * 4 > (int64_t)256 << 20) break;
       double step;
       if (bm == 256) step = t <= 256 ? 1.0 : 1.15 * ((t + 255) / 256);
       else step = 1.38 * (t / 512) + (t % 512 == 0 ? 0 : t % 512 <= 256 ? 0.8 : 1.38);

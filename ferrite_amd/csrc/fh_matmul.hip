@@ -106,6 +106,7 @@ __device__ inline void matmul_epilogue(const MmArgs& m, const fh_program& p, con
   // value r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of a block
   const int64_t cbase = bi * m.sc;
   for (int i = 0; i < TM; ++i) {
+    wave_lds_order();
 #pragma unroll
     for (int ii = 0; ii < TM; ++ii) {  // (the accumulators' indices stay constants)
       if (ii != i) continue;
@@ -114,6 +115,7 @@ __device__ inline void matmul_epilogue(const MmArgs& m, const fh_program& p, con
 #pragma unroll
         for (int r = 0; r < 16; ++r) cs[(8 * (r >> 2) + 4 * fh8 + (r & 3)) * CLD + 32 * j + fr] = acc[ii][j][r];
     }
+    wave_lds_order();
     const int64_t row0 = r0 + 32 * i;
     const bool inside = row0 + 32 <= m.M && col0 + 32 * TN <= m.N;
     if (!PROG && m.cvec && inside && m.c_dtype != FH_I32) {
