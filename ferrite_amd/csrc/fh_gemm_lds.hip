@@ -364,7 +364,9 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
 #pragma unroll
     for (int ii = 0; ii < TM; ++ii)  // (the accumulators' indices stay constants)
       if (ii == u >> 1) block_to_lds(cs, acc[ii], u & 1, lane);
+    wave_lds_order();
     block_epilogue(a, g, cs, tn, wc, m0 + wr + 16 * u, M, ybase, lane, a.ssq_in ? rs_s + 16 * u : nullptr, MODE == 2 ? part * g.split_y : 0);
+    wave_lds_order();
   }
 }
 
