@@ -17,7 +17,7 @@ __device__ inline uint32_t pack_bf16_rne(float lo, float hi) { return bf16_rne_f
 // the run a tile's local run lr (0 .. RUNS - 1) stands for, or -1 past the weight: RUNS runs of 16 columns a tile, or
 // RUNS / 2 pairs (the first runs, then their partners)
 template <int RUNS = 8>
-__device__ inline int64_t tile_run(const MatArgs& a, int tn, int lr) {
+__host__ __device__ inline int64_t tile_run(const MatArgs& a, int tn, int lr) {
   if (a.P == 1) {
     const int64_t nb = (int64_t)tn * RUNS + lr;
     return nb < a.N / 16 ? nb : -1;

@@ -113,8 +113,7 @@ __device__ inline void gemm_epilogue(const MatArgs& a, const SkinnyMoe& g, const
     const int64_t c0 = run * 16 + j;
     const bool rope = kind == FH_EP_ROPE_KV;
     const int hd = rope ? a.head_dim : 1;
-    const int h = (int)c0 / hd, d = (int)c0 % hd, d1 = d + hd / 2;  // (c0 < N < 2^31)
-    const bool turn = rope && h < a.heads + a.kv_heads;  // q's and k's heads turn: x cos + (-x2, x1) sin (models/llama.py:92-93)
+    const auto [h, d, d1, turn] = rope ? rope_pair(a, run, j) : RopePair{};  // (turn: x cos + (-x2, x1) sin, models/llama.py:92-93)
     constexpr int S = NT / H, RB = 8;
     for (int rb = t / H; rb < BM; rb += RB * S) {
       float cs0[RB], cs1[RB], sn0[RB], sn1[RB], sc[RB];

@@ -99,8 +99,8 @@ __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe
     }
     return;
   }
-  const int hd = a.head_dim, h = (int)c0 / hd, d = (int)c0 % hd, d1 = d + hd / 2;  // (c0 < N < 2^31)
-  const bool turn = h < a.heads + a.kv_heads;  // q's and k's heads turn: x cos + (-x2, x1) sin (models/llama.py:92-93)
+  const int hd = a.head_dim;
+  const auto [h, d, d1, turn] = rope_pair(a, run, j);  // (turn: x cos + (-x2, x1) sin, models/llama.py:92-93)
   for (int i0 = 0; i0 < 8; i0 += 4) {
     float cs0[4], cs1[4], sn0[4], sn1[4];
     int32_t crow[4];

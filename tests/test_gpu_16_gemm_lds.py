@@ -82,3 +82,52 @@ def test_every_epilogue_at_tile_edges(cuda, fmt, M, K, N):
         return ep, [data]
       big = 2 * near.max()
       check(bw, rope, (M, 4 * kv * HD), torch.float32, lambda a: big + 0 * a, f"rope {kind}")
+
+
+def cache_parts(data, kind, rows):
+  """A cache's values in 64 bits and the step its values lie on (a block float's run; 0 elsewhere), [rows][HD]."""
+  if kind in ("fp32", "bf16"): return data.double().reshape(rows, HD), 0 * data.double().reshape(rows, HD)
+  mags, e = data[:rows * HD // (1 if kind == "bfp8" else 2)], data[data.numel() - rows * HD // 16:].double()
+  q, bias = (mags.view(torch.int8).double(), 133) if kind == "bfp8" else (torch.stack([mags.to(torch.int16) & 15, mags.to(torch.int16) >> 4], -1).double(), 129)
+  if kind == "bfp4": q = torch.where(q > 7, q - 16, q)
+  step = torch.exp2(e - bias)[:, None].expand(-1, 16)
+  return (q.reshape(-1, 16) * step).reshape(rows, HD), step.reshape(rows, HD)
+
+
+@pytest.mark.parametrize("kind", ["fp32", "bf16", "bfp8", "bfp4"])
+@pytest.mark.parametrize("M,K,heads,kv", [(65, 64, 1, 1), (130, 576, 9, 3), (200, 576, 4, 1), (96, 4096, 5, 2), (300, 4096, 9, 3)])
+def test_rope_where_the_pairs_end_inside_a_tile(cuda, kind, M, K, heads, kv):
+  """A qkv matmul whose pairs of runs are no whole tiles (SmolLM's 30 in tiles of 4 among them), rows at place 0 among
+  the others, on fp32 rows, on bf16 rows with K whole (the same bits) and with K in parts (fp32 sums in another order; the
+  cache's values each rounded to its format, so a step of each run's more)."""
+  from ferrite_amd import lib, ops
+  N = (heads + 2 * kv) * HD
+  g = torch.Generator(device="cuda").manual_seed(M + K + heads)
+  x = torch.full((M + 8, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+  x[:M] = torch.randn(M, K, generator=g, device="cuda")
+  x = x[:M]
+  bw = ops.pack(torch.randn(K, N, generator=g, device="cuda") * 0.02, "bfp8")
+  cos, sin = (torch.from_numpy(t).cuda() for t in G.rotary_tables(G.model(dim=HD, heads=1, theta=1e4), 64))
+  places = torch.arange(M, dtype=torch.int32, device="cuda") % 64
+  rows = torch.randperm(M + 9, generator=g, device="cuda")[:M].to(torch.int32)
+  def rope(out):
+    cache = ops.kv_cache(2 * kv, M + 9, HD, kind, "cuda")
+    data, dt, length = ops.cache_fields(cache)
+    return ops.epilogue(lib.EP_ROPE_KV, heads=heads, kv_heads=kv, head_dim=HD, cos_tab=cos, sin_tab=sin, rope_rows=64, places=places,
+                        cache_rows=rows, cache=data, cache_dtype=dt, cache_len=length), [data]
+  old, one, split = both(ops, lib, x, bw, rope, (M, heads * HD), torch.float32, lib.load().fh_gemm_workspace_bytes(M, K, N))
+  for a, b in zip(old, one): assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+  # against 64 bits: q turned by its row's place, k turned and v as they are in the cache rows
+  y = (x.double() @ ops.dequant(bw).double()).reshape(M, -1, HD)
+  turn = y[:, :heads + kv]
+  c, s = cos[places].double()[:, None], sin[places].double()[:, None]
+  y[:, :heads + kv] = turn * c + torch.cat([-turn[..., HD // 2:], turn[..., :HD // 2]], -1) * s
+  # (sums of exact products in fp32, 2^-21 of sum |x w| as above, and a turn's two products and sum: of the two sums together)
+  near = 4 * 2 ** -21 * (x.double().abs() @ ops.dequant(bw).double().abs()).max()
+  for got in (one, split):
+    assert ((got[0].double().reshape(M, heads, HD) - y[:, :heads]).abs() <= near).all()
+    v, step = cache_parts(got[1], kind, 2 * kv * (M + 9))
+    v, step = (t.reshape(2 * kv, M + 9, HD)[:, rows.long()].permute(1, 0, 2) for t in (v, step))
+    want = y[:, heads:]
+    # (bf16's rounding, then at most a whole step of a run's block float: the largest magnitudes saturate)
+    assert ((v - want).abs() <= near + (0 if kind == "fp32" else 2 ** -8 * want.abs()) + step).all()
