@@ -373,9 +373,11 @@ extern "C" int fh_moe_experts(const float* x, int64_t ldx, int rows, int64_t dim
   if (int rc = fh_bfp_bytes(dim, gu_n, gu_fmt, FH_AXIS_N, &mb, &eb)) return rc;
   size_t dmb, deb;
   if (int rc = fh_bfp_bytes(ffn, dim, down_fmt, FH_AXIS_N, &dmb, &deb)) return rc;
+  // (down's K in parts is fh_gemm_lds.hip's alone, which reads g's rows 16-byte aligned: in a workspace that is not, K whole)
+  const size_t room = ((uintptr_t)workspace & 15) ? 0 : std::min(ws_bytes, (size_t)MOE_BUDGET);
   for (int r0 = 0; r0 < rows; r0 += pass) {
     const int n = rows - r0 < pass ? rows - r0 : pass;
-    const MoeSpace m = moe_space(n, experts, ffn, dim, std::min(ws_bytes, (size_t)MOE_BUDGET));
+    const MoeSpace m = moe_space(n, experts, ffn, dim, room);
     char* w = (char*)workspace;
     int32_t* counts = (int32_t*)(w + m.counts);
     int32_t* rows_of = (int32_t*)(w + m.rows_of);

@@ -144,3 +144,25 @@ def test_moe_in_a_workspace_sized_for_more_rows(cuda, rows, sized):
   # their magnitudes in each order; twice that sum as plain fp32 has it covers the rounding of h and the weights)
   mag = sum(dense[:, e:e + 1] * ((torch.nn.functional.silu(x @ gu[e, :, :ffn]) * (x @ gu[e, :, ffn:])).abs() @ dn[e].abs()) for e in range(E))
   assert ((got - want).abs() <= 2 * 2 * 2 ** -15 * mag).all()
+
+
+@pytest.mark.parametrize("rows", [65, 300, 512, 513])
+def test_moe_in_a_workspace_at_8_bytes(cuda, rows):
+  """A workspace that is not 16-byte aligned serves too: down's K whole there, whatever the rows (fh_gemm_lds.hip, which
+  takes K in parts, reads 16-byte aligned rows), the results as in an aligned one but for the order of fp32 sums."""
+  from ferrite_amd import lib, ops
+  E, dim, ffn = 2, 256, 2048
+  g = torch.Generator(device="cuda").manual_seed(rows)
+  gu, dn = (torch.randn(*s, generator=g, device="cuda") * 0.05 for s in ((E, dim, 2 * ffn), (E, ffn, dim)))
+  ex = ops.pack_experts(gu, dn, "bfp4")
+  x = torch.randn(rows, dim, generator=g, device="cuda")
+  dense = torch.rand(rows, E, generator=g, device="cuda")
+  need = lib.load().fh_moe_workspace_bytes(rows, E, ffn, dim)
+  want = ops.moe_experts(x, ex, dense, ws=torch.empty(need, dtype=torch.uint8, device="cuda"))
+  ws = torch.full((need + 16,), 0xFF, dtype=torch.uint8, device="cuda")[8:]
+  assert ws.data_ptr() % 16 == 8
+  got = ops.moe_experts(x, ex, dense, ws=ws)
+  # (2048 products an expert summed in fp32 16 at a time: fewer than 2^8 roundings of 2^-24 of the sum of their magnitudes
+  # in each order; twice that sum, as above)
+  mag = sum(dense[:, e:e + 1] * ((torch.nn.functional.silu(x @ gu[e, :, :ffn]) * (x @ gu[e, :, ffn:])).abs() @ dn[e].abs()) for e in range(E))
+  assert ((got - want).abs() <= 2 * 2 * 2 ** -16 * mag).all()
