@@ -12,17 +12,10 @@
 // (about 60 a lane at batch 1) keep ~32 waves on every CU, each with its loads in flight: a decode GEMV is a
 // latency-bound stream, and that is what hides the latency. Nothing crosses workgroups: no atomics, no fences.
 #include <math.h>
-#include <algorithm>
 #include <type_traits>
-#include "fh_epilogue.h"
+#include "fh_gemv.h"
 
 namespace fh {
-
-// rows a lane has in flight at once, by format and batch rows (about 4 KiB of weight a wave and run at batch 1)
-__host__ __device__ constexpr int gemv_group(bool four, int b, int p) { return (b <= 2 ? 4 : b <= 4 ? 2 : 1) * (four ? 2 : 1) + 0 * p; }
-
-// threads a workgroup at most: 16 waves for one row, 8 for more (whose partial sums need the registers)
-__host__ __device__ constexpr int gemv_threads(int b) { return b == 1 ? 1024 : 512; }
 
 // The first arguments are what the stream's first loads need, passed apart from MatArgs so that they arrive in
 // SGPRs with the wave (kernel-argument preloading, -amdgpu-kernarg-preload-count): the loads go out without waiting
@@ -164,18 +157,21 @@ __global__ __launch_bounds__(gemv_threads(B)) void gemv_kernel(const uint8_t* __
   __syncthreads();
   if (slice != 0) return;  // wave 0 adds the slices in order and runs the epilogue
   // (in 64 bits, rounded once, four slices' reads in flight: a chain of fp32 sums over more and shorter slices loses what
-  // the lanes' shorter chains gain. 576 x 1536 in bfp8, error against 64 bits: 8.4e-8 in 3 slices, 8.7e-8
-  // in 5, 7.8e-8 in 5 this way; no slower: SmolLM's step 741-744 us both ways)
+  // the lanes' shorter chains gain. Error against 64 bits in bfp8, fp32 sums of the slices -> these: 576 x 1536 in 3 slices
+  // 8.5e-8 -> 8.1e-8, 1536 x 576 in 6 9.6e-8 -> 8.8e-8, 2048 x 2048 in 8 9.5e-8 -> 8.2e-8, at the same time within 0.1 us)
   for (int i = lane; i < V; i += 64) {
     double t = red[0][i];
-    for (int w = 1; w < W; w += 4) {
-      float v[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = red[min(w + k, W - 1)][i];
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (w + k < W) t += v[k];
+    int w = 1;
+    for (; w + 4 <= W; w += 4) {
+      const float v0 = red[w][i], v1 = red[w + 1][i], v2 = red[w + 2][i], v3 = red[w + 3][i];
+      t += v0; t += v1; t += v2; t += v3;
     }
+    if (w + 2 <= W) {
+      const float v0 = red[w][i], v1 = red[w + 1][i];
+      t += v0; t += v1;
+      w += 2;
+    }
+    if (w < W) t += red[w][i];
     fin[i] = (float)t;
   }
   // each batch row's 1 / rms, from the sums of squares its maker left by runs of 16
@@ -297,37 +293,6 @@ static int dispatch_batch(const MatArgs& a, int batch, int items, int W, hipStre
   return FH_OK;
 }
 
-// The K slices: W waves a workgroup, the least power of 2 giving about 16384 waves in all (64 a CU on 256 CUs, in
-// turns), at most one a group of U loads of 64 rows a lane, at most 8 for more than one row (their launch bound is 512
-// threads, so that the rows' partial sums stay in registers: bound to 1024 threads they spilled, and batch 8 of an 8B
-// step took 35.6 ms instead of 6.5), and at most 16 for bfp4 and 8 for bfp8 at one row: a bfp8 wave needs
-// ~100 registers at two runs an item, so a 16-wave workgroup fills a CU alone and the grid runs in lock-step rounds
-// (on MI355X: the 8B shapes' bfp8 gate_up 31.7 us at 16, 25.9 at 8; bfp4's down 11.0 at 16, 11.4 at 8).
-struct Plan { int W, rows, P, most, items; };
-static Plan plan(int64_t K, int64_t N, int fmt, int kind, int batch) {
-  Plan p;
-  p.P = (kind == FH_EP_SILU_GATE || kind == FH_EP_ROPE_KV) ? 2 : 1;  // as epilogue_args sets MatArgs::P
-  p.most = p.P == 1 ? 8 : 4;
-  p.items = (int)(N / 16 / p.P);
-  const int b = batch < p.most ? batch : p.most;
-  const int unit = 64 * gemv_group(fmt == FH_BFP4, b, p.P);
-  int64_t units = (K + unit - 1) / unit;
-  // (few items leave most of the chip idle, and a call takes what one wave's chain takes: then a wave as few as 64 rows.
-  // SmolLM's step: qkv 5.6 -> 5.2 us, gate_up 5.3 -> 4.7, o 4.7 -> 3.9, down 4.5 -> 3.9, the step 768 -> 744. The line is
-  // where all waves fit the chip at once, 4 a CU)
-  if (units * p.items < 1024) units = (K + 63) / 64;
-  const int64_t most = std::min<int64_t>(fmt == FH_BFP4 ? 16 : 8, gemv_threads(b) / 64);  // (measured: bfp8's 16-wave
-                                                                                           // workgroups run in lock-step rounds)
-  int64_t W = 1;
-  while (W < most && W * p.items < 16384) W *= 2;
-  while (W > 1 && W > units) W /= 2;
-  int64_t rows = (K + W - 1) / W;
-  rows = (rows + 63) / 64 * 64;
-  p.W = (int)((K + rows - 1) / rows);
-  p.rows = (int)rows;
-  return p;
-}
-
 }  // namespace fh
 
 using namespace fh;
@@ -347,7 +312,7 @@ extern "C" int fh_gemv_bfp(const void* x, int x_dtype, int64_t ldx, int batch, i
   a.mant = (const uint8_t*)w_mant; a.exps = w_exps; a.K = K; a.N = N; a.M = batch;
   a.y = y; a.y_bf16 = y_dtype == FH_BF16; a.ldy = ldy;
   if (int rc = epilogue_args("fh_gemv_bfp", ep, K, N, y_dtype, ldy, a)) return rc;
-  const Plan p = plan(K, N, fmt, a.kind, batch);
+  const GemvPlan p = gemv_plan(K, N, fmt, a.kind, batch);
   a.rows = p.rows;
   hipStream_t s = as_stream(stream);
   const bool four = fmt == FH_BFP4;

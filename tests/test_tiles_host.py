@@ -1,4 +1,4 @@
-"""The tiled matmul kernels' index rules, compiled for the host from the headers the kernels include (no GPU needed)."""
+"""The matmul kernels' index rules and plans, compiled for the host from the headers the kernels include (no GPU needed)."""
 import subprocess
 import pytest
 from ferrite_amd import build
@@ -32,13 +32,16 @@ int main(int, char** v) {
 '''
 
 
-@pytest.fixture(scope="module")
-def ragged(tmp_path_factory):
-  d = tmp_path_factory.mktemp("tiles")
-  (d / "t.hip").write_text(RAGGED)
+def program(d, text):
+  (d / "t.hip").write_text(text)
   subprocess.run([build.hipcc(), "-x", "hip", "--offload-host-only", "-std=c++17", "-O1", "-w", "-I", str(build.CSRC),
                   "-I", str(build.HERE.parent / "include"), str(d / "t.hip"), "-o", str(d / "t")], check=True)
   return d / "t"
+
+
+@pytest.fixture(scope="module")
+def ragged(tmp_path_factory):
+  return program(tmp_path_factory.mktemp("tiles"), RAGGED)
 
 
 @pytest.mark.parametrize("heads,kv,hd", [(9, 3, 64), (1, 1, 32), (4, 1, 32), (5, 2, 64), (1, 1, 96), (3, 1, 160), (32, 8, 128)])
@@ -49,3 +52,33 @@ def test_rope_pairs_past_the_weight_read_no_table(ragged, heads, kv, hd):
   assert r.returncode == 0, r.stdout
   pairs = (heads + 2 * kv) * hd // 32
   assert [int(x) for x in r.stdout.split()] == [-pairs % 4, -pairs % 6, -pairs % 8]
+
+
+GEMV = r'''
+#include "fh_gemv.h"
+#include <cstdio>
+int main() {
+  for (int fmt : {FH_BFP8, FH_BFP4})
+    for (int kind : {FH_EP_STORE, FH_EP_SILU_GATE})
+      for (int batch : {1, 2, 3, 4, 5, 8, 9})
+        for (int64_t K : {1, 63, 64, 65, 256, 257, 512, 576, 1024, 1025, 1536, 2048, 2816, 4096, 14336})
+          for (int64_t N : {32, 576, 960, 4096, 49152, 1 << 22}) {
+            const fh::GemvPlan p = fh::gemv_plan(K, N, fmt, kind, batch);
+            printf("%d %d %d %ld %ld %d %d %d %d %d\n", fmt, kind, batch, (long)K, (long)N, p.W, p.rows, p.P, p.most, p.items);
+          }
+}
+'''
+
+
+def test_gemv_slices_are_whole_load_groups(tmp_path):
+  """The GEMV's K slices cover K once, in whole 64 rows, none empty, within its workgroups' waves, and never more of them
+  than the groups of loads a wave keeps in flight: shorter ones made bfp4 calls of few items up to twice as slow."""
+  from ferrite_amd import lib
+  lines = [list(map(int, l.split())) for l in subprocess.run([str(program(tmp_path, GEMV))], capture_output=True, text=True, check=True).stdout.splitlines()]
+  assert len(lines) == 2 * 2 * 7 * 15 * 6
+  for fmt, kind, batch, K, N, W, rows, P, most, items in lines:
+    b = min(batch, most)
+    assert P == (2 if kind == lib.EP_SILU_GATE else 1) and items == N // 16 // P
+    assert rows % 64 == 0 and (W - 1) * rows < K <= W * rows and 1 <= W <= (16 if b == 1 and fmt == lib.BFP4 else 8)
+    group = 64 * (4 if b <= 2 else 2 if b <= 4 else 1) * (2 if fmt == lib.BFP4 else 1)
+    assert W <= -(-K // group), (fmt, kind, batch, K, N, W)
