@@ -1,7 +1,7 @@
 // Errors, block-float packing and unpacking, embedding rows and argmax: the small kernels of libferrite_hip.so.
 #include <stdarg.h>
 #include <string.h>
-#include "fh_common.h"
+#include "fh_pack.h"
 
 namespace fh {
 
@@ -215,8 +215,7 @@ extern "C" int fh_bfp_pack(const void* src, int src_dtype, int64_t K, int64_t N,
   hipStream_t s = as_stream(stream);
   auto m = (uint8_t*)mant;
   const dim3 block(256);
-  // (past ~2 MB of values; 576 x 1536 takes 4.5 us a thread a block, 4.9 in these tiles)
-  if (axis == FH_AXIS_N && blocks >= 131072 && (K + 63) / 64 <= 65535) {
+  if (axis == FH_AXIS_N && pack_in_tiles(K, g.n_outer)) {
     const int vec = !((uintptr_t)src & 15) && ld % (bf ? 8 : 4) == 0;
     const dim3 grid((unsigned)((g.n_outer + 15) / 16), (unsigned)((K + 63) / 64));
 #define PK_ROWS(F, B) hipLaunchKernelGGL((pack_rows_kernel<F, B>), grid, block, 0, s, src, K, g.n_outer, ld, vec, m, exps)

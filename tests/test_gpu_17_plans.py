@@ -63,7 +63,7 @@ def test_prefill_attention_of_few_rows(cuda, kind, heads, kv, hd, T, p0):
 @pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("K,N,pad,off", [(16, 16, 0, 0), (63, 272, 0, 0), (64, 256, 8, 0), (65, 240, 4, 0), (128, 4112, 0, 0), (80, 64, 1, 0), (96, 48, 0, 1),
-                                         (2064, 1040, 0, 0), (1104, 2064, 2, 0), (2048, 1072, 8, 1), (4096, 4112, 0, 0), (4112, 4104, 4, 0)])
+                                         (2064, 1040, 0, 0), (1, 2097152, 0, 0), (7, 299600, 0, 0), (8, 262160, 8, 0), (9, 240000, 2, 0), (1104, 2064, 2, 0), (2048, 1072, 8, 1), (4096, 4112, 0, 0), (4112, 4104, 4, 0)])
 def test_packing_at_every_stride(cuda, fmt, dtype, K, N, pad, off):
   """fh_bfp_pack along both axes, in its wide and its narrow loads (whole tiles and ragged ones, row strides and bases at
   odd alignments), against the oracle's blocks: magnitudes and exponents bit for bit, as gpt2.bfp makes them."""

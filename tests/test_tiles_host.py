@@ -82,3 +82,23 @@ def test_gemv_slices_are_whole_load_groups(tmp_path):
     assert rows % 64 == 0 and (W - 1) * rows < K <= W * rows and 1 <= W <= (16 if b == 1 and fmt == lib.BFP4 else 8)
     group = 64 * (4 if b <= 2 else 2 if b <= 4 else 1) * (2 if fmt == lib.BFP4 else 1)
     assert W <= -(-K // group), (fmt, kind, batch, K, N, W)
+
+
+PACK = r'''
+#include "fh_pack.h"
+#include <cstdio>
+int main() {
+  for (int64_t K : {1, 4, 7, 8, 15, 16, 64, 4096, 4194240, 4194241})
+    for (int64_t runs : {1ll, 8192ll, 16384ll, 131072ll, 1ll << 26, (1ll << 28) - 1, 1ll << 28, 1ll << 29})
+      printf("%ld %ld %d\n", (long)K, (long)runs, fh::pack_in_tiles(K, runs));
+}
+'''
+
+
+def test_packing_in_tiles_where_it_is_the_faster(tmp_path):
+  """Packing along N in tiles of 64 rows: not of fewer than 8 rows, whose tiles are mostly idle threads (1 row 1.8 times as
+  slow as a thread a block), and never past what a grid holds, which a thread a block takes (2^32 blocks)."""
+  out = subprocess.run([str(program(tmp_path, PACK))], capture_output=True, text=True, check=True).stdout.splitlines()
+  got = {(int(k), int(r)): t == "1" for k, r, t in (l.split() for l in out)}
+  for (K, runs), tiles in got.items():
+    assert tiles == (K >= 8 and K * runs >= 131072 and (runs + 15) // 16 * 256 < 2 ** 32 and -(-K // 64) < 65536), (K, runs)
