@@ -182,13 +182,23 @@ def _matmul(entry, x, bw, ep, out, out_dtype):
   yp, ydt, ldy, _ = _layout(out)
   args = (xp, xdt, ldx, rows, bw.K, bw.N, _ptr(bw.mant), _ptr(bw.exps), lib.DTYPES[bw.fmt],
           ctypes.byref(ep) if ep is not None else None, yp, ydt, ldy)
-  n = _gemm_workspace_bytes(rows, bw.K, bw.N) if entry == "fh_gemm_bfp" and rows > 64 and xdt == lib.BF16 else 0
+  n = _gemm_workspace_bytes(rows, bw.K, bw.N) if entry == "fh_gemm_bfp" and rows > 64 and xdt == lib.BF16 and _in_parts(xp, ep) else 0
   if n:  # (freed as this returns: torch's allocator hands it only to later work on this stream)
-    ws = torch.empty(n, dtype=torch.uint8, device=x.device)
-    lib.call("fh_gemm_bfp_ws", *args, _ptr(ws), n, _stream())
-  else:
-    lib.call(entry, *args, _stream())
+    try: ws = torch.empty(n, dtype=torch.uint8, device=x.device)
+    except torch.OutOfMemoryError: n = 0  # (K whole, which needs none)
+  if n: lib.call("fh_gemm_bfp_ws", *args, _ptr(ws), n, _stream())
+  else: lib.call(entry, *args, _stream())
   return out
+
+
+def _in_parts(xp, ep):
+  """Whether a matmul of bf16 rows at xp with epilogue ep is one whose kernel can take K in parts (fh_gemm_lds.hip): rows
+  16-byte aligned, no RMSNorm weight, and no program but the one that only copies the sum."""
+  if xp % 16: return False
+  if ep is None: return True
+  if ep.kind != lib.EP_PROGRAM: return not ep.norm_w
+  p = ep.program.contents if ep.program else None
+  return not ep.norm_w and p is not None and p.n_ops == 1 and p.op[0] == lib.OP["copy"] and p.a[0] == lib.OPND_ACC
 
 
 @functools.lru_cache(maxsize=1024)

@@ -166,3 +166,47 @@ def test_moe_in_a_workspace_at_8_bytes(cuda, rows):
   # in each order; twice that sum, as above)
   mag = sum(dense[:, e:e + 1] * ((torch.nn.functional.silu(x @ gu[e, :, :ffn]) * (x @ gu[e, :, ffn:])).abs() @ dn[e].abs()) for e in range(E))
   assert ((got - want).abs() <= 2 * 2 * 2 ** -16 * mag).all()
+
+
+def test_gemm_workspace_only_where_a_kernel_reads_it(cuda):
+  """ops.gemm takes memory for K's parts only for the calls whose kernel adds them: a fused program, a norm's weight and
+  rows off 16 bytes go to kernels that take K whole. A plain call takes the parts' bytes."""
+  import ctypes
+  from ferrite_amd import lib, ops
+  M, K, N = 200, 4096, 1024
+  g = torch.Generator(device="cuda").manual_seed(3)
+  rows = torch.randn(M, K + 8, generator=g, device="cuda").to(torch.bfloat16)
+  x, off = rows[:, :K], rows.view(-1)[4:4 + (M - 1) * (K + 8) + K].as_strided((M, K), (K + 8, 1))
+  bw = ops.pack(torch.randn(K, N, generator=g, device="cuda") * 0.02, "bfp8")
+  parts = lib.load().fh_gemm_workspace_bytes(M, K, N)
+  out = torch.empty(M, N, device="cuda")
+  assert parts > 1 << 20
+  def program(op):
+    p = lib.Program()
+    p.n_ops, p.op[0], p.a[0], p.b[0], p.imm[0] = 1, lib.OP[op], lib.OPND_ACC, lib.OPND_IMM, 0.5
+    ep = ops.epilogue(lib.EP_PROGRAM)
+    ep.program = ctypes.pointer(p)
+    return ep
+  ssq, w = x.float().square().reshape(M, K // 16, 16).sum(-1), torch.ones(K, device="cuda")
+  for rows_, ep, most in ((x, None, parts), (x, ops.epilogue(lib.EP_STORE, ssq_in=ssq, eps=1e-5), parts), (x, program("copy"), parts),
+                          (x, program("mul"), 0), (x, ops.epilogue(lib.EP_STORE, norm_w=w, ssq_in=ssq, eps=1e-5), 0), (off, None, 0)):
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    ops.gemm(rows_, bw, ep, out=out)
+    took = torch.cuda.max_memory_allocated() - before
+    assert took >= parts if most else took == 0, (took, most)
+
+
+def test_gemm_without_room_for_its_parts(cuda, monkeypatch):
+  """A card too full for K's parts: K whole, the bits of fh_gemm_bfp, which needs no workspace."""
+  from ferrite_amd import lib, ops
+  M, K, N = 200, 4096, 1024
+  g = torch.Generator(device="cuda").manual_seed(4)
+  x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+  bw = ops.pack(torch.randn(K, N, generator=g, device="cuda") * 0.02, "bfp4")
+  want = torch.empty(M, N, device="cuda")
+  lib.call("fh_gemm_bfp", x.data_ptr(), lib.BF16, K, M, K, N, bw.mant.data_ptr(), bw.exps.data_ptr(), lib.BFP4, None, want.data_ptr(),
+           lib.F32, N, torch.cuda.current_stream().cuda_stream)
+  monkeypatch.setattr(ops, "_gemm_workspace_bytes", lambda *a: 1 << 46)
+  assert torch.equal(ops.gemm(x, bw), want)
