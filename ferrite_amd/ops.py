@@ -391,8 +391,10 @@ def moe_experts(x, ex, dense, out=None, residual=None, ssq_out=None, norm_w=None
   _dev(x, dense, out, residual, ssq_out, norm_w, ssq_in)
   rows = x.shape[0]
   if out is None: out = torch.empty(rows, ex.dim, dtype=torch.float32, device=x.device)
-  n = lib.load().fh_moe_workspace_bytes(rows, ex.experts, ex.ffn, ex.dim)
-  if ws is None or ws.numel() < n: ws = torch.empty(max(n, 256), dtype=torch.uint8, device=x.device)
+  need = lambda r: lib.load().fh_moe_workspace_bytes(r, ex.experts, ex.ffn, ex.dim)
+  n = need(rows)
+  # (up to 512 rows down's K goes in as many parts as fit: a workspace for more rows, which has none of them, serves too)
+  if ws is None or ws.numel() < n and (rows > 512 or ws.numel() < need(513)): ws = torch.empty(max(n, 256), dtype=torch.uint8, device=x.device)
   lib.call("fh_moe_experts", _ptr(x), x.stride(0), rows, ex.dim, _ptr(norm_w), _ptr(ssq_in), eps, int(centered),
            ex.experts, ex.ffn, _ptr(ex.gate_up.mant), _ptr(ex.gate_up.exps), lib.DTYPES[ex.gate_up.fmt], _ptr(ex.down.mant),
            _ptr(ex.down.exps), lib.DTYPES[ex.down.fmt], _ptr(dense), _ptr(out), _ptr(residual), _ptr(ssq_out), _ptr(ws),

@@ -210,3 +210,22 @@ def test_gemm_without_room_for_its_parts(cuda, monkeypatch):
            lib.F32, N, torch.cuda.current_stream().cuda_stream)
   monkeypatch.setattr(ops, "_gemm_workspace_bytes", lambda *a: 1 << 46)
   assert torch.equal(ops.gemm(x, bw), want)
+
+
+def test_moe_experts_keeps_a_workspace_for_more_rows(cuda):
+  """ops.moe_experts runs in the workspace it is given where that is one for more rows than the call's, though fewer rows'
+  own, with its parts of down's K, would be larger; one for fewer rows it replaces."""
+  from ferrite_amd import lib, ops
+  E, dim, ffn = 2, 256, 4096
+  g = torch.Generator(device="cuda").manual_seed(5)
+  ex = ops.pack_experts(*(torch.randn(*s, generator=g, device="cuda") * 0.05 for s in ((E, dim, 2 * ffn), (E, ffn, dim))), "bfp8")
+  bytes_ = lambda rows: lib.load().fh_moe_workspace_bytes(rows, E, ffn, dim)
+  assert bytes_(512) > bytes_(513)
+  for rows, sized, more in ((512, 513, False), (65, 513, False), (512, 2048, False), (512, 512, False), (512, 65, True), (600, 513, True)):
+    x, dense, out = torch.randn(rows, dim, generator=g, device="cuda"), torch.rand(rows, E, generator=g, device="cuda"), torch.empty(rows, dim, device="cuda")
+    ws = torch.empty(bytes_(sized), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    ops.moe_experts(x, ex, dense, out=out, ws=ws)
+    assert (torch.cuda.max_memory_allocated() > before) == more, (rows, sized)
