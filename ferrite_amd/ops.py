@@ -243,8 +243,10 @@ def matmul(a, b, program=None, out=None, out_dtype=torch.float32):
 
 def put_i32(values, out):
   """out (a contiguous int32 tensor on the GPU) from as many integers of the host's, in stream order and with no copy
-  (fh_put_i32): values a list, or an int32 array or CPU tensor."""
+  (fh_put_i32): values a list, or an int32 array or CPU tensor. Refused while the stream is captured, as a copy from the
+  host is: every replay would put these values again, whatever the host holds then."""
   _dev(out)
+  if torch.cuda.is_current_stream_capturing(): raise RuntimeError("put_i32: the host's integers cannot be captured (a replay would put the same ones)")
   v = np.ascontiguousarray(values, np.int32)
   if out.dtype != torch.int32 or not out.is_contiguous() or v.size != out.numel(): raise ValueError(f"put_i32: {v.size} integers into {tuple(out.shape)} {out.dtype}")
   lib.call("fh_put_i32", v.ctypes.data, v.size, _ptr(out), _stream())

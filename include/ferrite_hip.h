@@ -203,7 +203,8 @@ int fh_gemm_bfp_ws(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K
 
 /* n integers of the host's memory into out (device memory), in stream order: they travel as kernel arguments (960 a
  * launch), so the call neither waits for the stream nor keeps `values` past its return, and a step's tokens, places and
- * cache rows reach the GPU without a copy (a blocking one of pageable memory costs ~40 us of an idle GPU each). */
+ * cache rows reach the GPU without a copy (a blocking one of pageable memory costs ~40 us of an idle GPU each). Captured
+ * into a graph, the values are the graph's: a replay puts the same ones. */
 int fh_put_i32(const int32_t* values, int64_t n, int32_t* out, void* stream);
 
 /* Rows ids[batch] of an embedding table [vocab][dim] (fp32 or bf16) into x[batch][dim] fp32, with the sums of

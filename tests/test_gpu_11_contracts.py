@@ -146,3 +146,24 @@ def test_decoder_rows_from_host_and_gpu(cuda):
     for t in (dec.ids, dec.places, dec.first, dec.rows): t.fill_(1)
     dec.step(i, p, s, replay=False)
     assert [t.tolist() for t in (dec.ids, dec.places, dec.first, dec.rows)] == want and dec.top == 31
+
+
+def test_host_integers_are_not_captured(cuda):
+  """A step or a prompt with tokens and places of the host's is refused inside a caller's capture (a graph would replay
+  those tokens for good); with the rows set before, the step is captured and replays what the buffers then hold."""
+  from ferrite_amd import llama as G
+  c = G.model(dim=64, heads=1, kv=1, layers=1, eps=1e-5, theta=1e4, vocab=64, ffn=64, places=32, tied=True)
+  dec = G.Decoder(c, G.random_weights(c), batch=2, context=32, slots=2)
+  dec.prefill([5, 9, 3])  # (its buffers made outside the capture)
+  want = [dec.step(ids, [0, 0], [0, 1], replay=False)[0].clone() for ids in ([5, 9], [7, 1])]
+  g = torch.cuda.CUDAGraph()
+  torch.cuda.synchronize()
+  with torch.cuda.graph(g):
+    for call in (lambda: dec.step([5, 9], [0, 0], [0, 1], replay=False), lambda: dec.step([5, 9], replay=False), lambda: dec.set_rows([0, 0], [0, 1]),
+                 lambda: dec.prefill([5, 9, 3])):
+      with pytest.raises(RuntimeError): call()
+    dec.step(replay=False)
+  for ids, logits in (([5, 9], want[0]), ([7, 1], want[1]), ([5, 9], want[0])):
+    dec.ids.copy_(torch.tensor(ids, dtype=torch.int32))
+    g.replay()
+    assert torch.equal(dec.logits, logits)
