@@ -460,7 +460,7 @@ size_t gemm_lds_bytes(const GemmPlan& p, int64_t M, int64_t N) {
 
 int gemm_lds(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, const GemmPlan& p, float* parts, hipStream_t s) {
   const int64_t tm = (a.M + p.bm - 1) / p.bm, tn = a.P == 1 ? (a.N / 16 + 7) / 8 : ((int64_t)a.items + 3) / 4;
-  if (tm * tn * p.splits >= 1LL << 22) return fail(FH_EUNSUP, "fh_gemm_bfp: too many tiles");
+  if (tm * tn * p.splits >= 1LL << 23) return fail(FH_EUNSUP, "fh_gemm_bfp: too many tiles");  // (a grid's threads along x stay below 2^32)
   const int64_t n = g.counts ? (tm * tn * p.splits + 7) / 8 * 8 : tm * tn * p.splits;
   const dim3 grid((unsigned)n, g.counts ? experts : 1);
 #define GL(F, WR, TM) do { \

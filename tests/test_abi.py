@@ -1,6 +1,6 @@
 """The C-ABI library builds, loads and exports every entry point include/ferrite_hip.h declares, and the ctypes
 binding knows each one (no GPU needed: nothing here computes)."""
-import ctypes, pathlib, re
+import ctypes, os, pathlib, re, subprocess, sys
 import pytest
 from ferrite_amd import lib
 
@@ -79,3 +79,21 @@ def test_tile_layout_and_its_refusals():
     lib.call("fh_rms_rows", p, 12, 2, 12, p, ctypes.c_float(1e-5), 0, p, lib.BF16_T16, 12, None)
   with pytest.raises(ValueError):
     lib.call("fh_read_probe", p, 10, p, 1, None)
+
+
+def test_gemm_takes_every_grid_a_launch_holds():
+  # a matmul of up to 2^23 - 1 tiles of 256 rows is launched, not refused (2^30 rows of K 64 and N 16 fit the card); with no
+  # GPU visible the launch itself fails, so the host's checks are all that runs
+  if not lib.PATH.exists(): pytest.skip("libferrite_hip.so not built")
+  code = """
+import ctypes
+from ferrite_amd import lib
+b = ctypes.create_string_buffer(4096)
+p = (ctypes.addressof(b) + 63) // 64 * 64
+for M in (65, 1 << 22, (1 << 30) - 256, 1 << 30, (1 << 31) - 256, 1 << 31):
+  try: lib.call("fh_gemm_bfp", p, lib.BF16, 64, M, 64, 16, p, p, lib.BFP8, None, p, lib.F32, 16, None)
+  except Exception as e: print(type(e).__name__)
+"""
+  env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", PYTHONPATH=str(HEADER.parent.parent))
+  r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env, check=True)
+  assert r.stdout.split() == ["RuntimeError"] * 5 + ["NotImplementedError"], r.stdout + r.stderr
