@@ -28,11 +28,49 @@ __host__ __device__ inline int64_t tile_run(const MatArgs& a, int tn, int lr) {
   return lr < RUNS / 2 ? nb0 : nb0 + a.pair_half;
 }
 
-// gemm_tiles' kernel for bf16 rows whose K is whole steps of 64 (fh_gemm_lds.hip)
+// gemm_tiles' kernel for bf16 rows whose K is whole steps of 64 (fh_gemm_lds.hip): tiles of 128 columns in K steps of 64
+constexpr int GL_BK = 64, GL_BN = 128;
 struct GemmPlan { int bm; int splits; double us; };  // rows a tile, K's parts, and the time expected of it
+
+// Rows a tile and K's parts: the least of a model of the call's time in us, its constants measured at the 8B shapes (bfp8
+// and bfp4 alike): 8 a launch; a step of a 256-row tile 1.0 with a workgroup a CU, 1.15 a round of them with the chip
+// full; of a 128-row tile 0.8 alone on a CU, 1.38 two a CU; K in parts, 6 more for the second launch and the parts written
+// and read back at 6.5 TB/s. (Measured, 200 rows, 1 part -> the plan's: o 4096 x 4096 75 -> 26 us in 8, down
+// 14336 x 4096 203 -> 45 in 8, qkv 4096 x 6144 67 -> 30 in 5; 1024 rows: o 72 -> 53 and down 214 -> 133 in 2; at 2048
+// rows every shape is fastest in one part.) A gathered matmul (experts > 0), whose rows an expert the host does not know,
+// takes 128-row tiles in one part.
+inline GemmPlan gemm_lds_plan(int64_t M, int64_t K, int64_t N, int experts, bool may_split) {
+  if (experts > 0) return {128, 1, 0};
+  GemmPlan best = {};
+  double cost = 0;
+  for (int bm = 256; bm >= 128; bm /= 2) {
+    const int64_t tiles = (M + bm - 1) / bm * ((N + GL_BN - 1) / GL_BN), all = K / GL_BK;
+    for (int s = 1; s <= (may_split ? 16 : 1) && (s == 1 || all / s >= 4); ++s) {
+      const int64_t t = tiles * s;
+      // (parts of at most 256 MB: past it the tiles are over a thousand already, and parts save the last round's rest alone)
+      if (s > 1 && t * bm * GL_BN * 4 > (int64_t)256 << 20) break;
+      double step;
+      if (bm == 256) step = t <= 256 ? 1.0 : 1.15 * ((t + 255) / 256);
+      else step = 1.38 * (t / 512) + (t % 512 == 0 ? 0 : t % 512 <= 256 ? 0.8 : 1.38);
+      const double us = 8 + (all + s - 1) / s * step + (s > 1 ? 6 + 8.0 * s * M * N / 6.5e6 : 0);
+      if (cost == 0 || us < cost) { cost = us; best = {bm, s, us}; }
+    }
+  }
+  return best;
+}
+
+inline size_t gemm_lds_bytes(const GemmPlan& p, int64_t M, int64_t N) {
+  return p.splits < 2 ? 0 : (size_t)p.splits * ((M + p.bm - 1) / p.bm) * ((N + GL_BN - 1) / GL_BN) * p.bm * GL_BN * 4;
+}
+
+// its workgroups over a's rows (one expert's, gathered), and whether a grid of them is one that a launch holds (512 threads
+// each, a grid's threads along x below 2^32)
+inline int64_t gemm_lds_grid(const MatArgs& a, const GemmPlan& p) {
+  return (a.M + p.bm - 1) / p.bm * (a.P == 1 ? (a.N / 16 + 7) / 8 : ((int64_t)a.items + 3) / 4) * p.splits;
+}
+inline bool gemm_lds_fits(const MatArgs& a, const GemmPlan& p) { return gemm_lds_grid(a, p) < 1LL << 23; }
+
 bool gemm_lds_takes(const MatArgs& a);
-GemmPlan gemm_lds_plan(int64_t M, int64_t K, int64_t N, int experts, bool may_split);
-size_t gemm_lds_bytes(const GemmPlan& p, int64_t M, int64_t N);  // the splits' partial sums
 int gemm_lds(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, const GemmPlan& p, float* parts, hipStream_t s);
 
 }  // namespace fh

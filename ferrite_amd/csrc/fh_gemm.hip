@@ -622,13 +622,14 @@ int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void*
       if (a.M <= 512) {
         GemmPlan p = gemm_lds_plan(a.M, a.K, a.N, experts, false);
         if (g.splits > 1) p.splits = g.splits;
-        return gemm_lds(a, g, fmt, experts, p, nullptr, s);
+        if (gemm_lds_fits(a, p)) return gemm_lds(a, g, fmt, experts, p, nullptr, s);
       }
     } else {
       GemmPlan p = gemm_lds_plan(a.M, a.K, a.N, 0, workspace != nullptr);
       if (gemm_lds_bytes(p, a.M, a.N) > ws_bytes) p = gemm_lds_plan(a.M, a.K, a.N, 0, false);
       const int64_t tiles3 = (a.M + 2 * GM_BM - 1) / (2 * GM_BM) * (a.P == 1 ? (a.N / 16 + 11) / 12 : ((int64_t)a.items + 5) / 6);
-      if (WNv != 3 || tiles3 > cus || p.us <= 8 + 1.9 * (double)(a.K / GM_BK)) return gemm_lds(a, g, fmt, 1, p, (float*)workspace, s);
+      if (WNv != 3 || tiles3 > cus || p.us <= 8 + 1.9 * (double)(a.K / GM_BK))
+        if (gemm_lds_fits(a, p)) return gemm_lds(a, g, fmt, 1, p, (float*)workspace, s);
     }
   }
   if (g.splits > 1) return fail(FH_EUNSUP, "gathered GEMM: K in parts for up to 512 bf16 rows whose K is a multiple of 64");

@@ -19,7 +19,7 @@
 
 namespace fh {
 
-constexpr int GL_BK = 64, GL_BN = 128, GL_RUNS = GL_BN / 16;
+constexpr int GL_RUNS = GL_BN / 16;
 
 typedef short gl_short4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) gl_short4* gl_lds_short4;
@@ -427,42 +427,10 @@ bool gemm_lds_takes(const MatArgs& a) {
   return a.kind != FH_EP_PROGRAM && a.x_bf16 && !a.x_tiles && !a.y_tiles && !a.copy_tiles && !a.norm_w && a.K % GL_BK == 0 && !((uintptr_t)a.x & 15) && a.ldx % 8 == 0;
 }
 
-// Rows a tile and K's parts: the least of a model of the call's time in us, its constants measured at the 8B shapes (bfp8
-// and bfp4 alike): 8 a launch; a step of a 256-row tile 1.0 with a workgroup a CU, 1.15 a round of them with the chip
-// full; of a 128-row tile 0.8 alone on a CU, 1.38 two a CU; K in parts, 6 more for the second launch and the parts written
-// and read back at 6.5 TB/s. (Measured, 200 rows, 1 part -> the plan's: o 4096 x 4096 75 -> 26 us in 8, down
-// 14336 x 4096 203 -> 45 in 8, qkv 4096 x 6144 67 -> 30 in 5; 1024 rows: o 72 -> 53 and down 214 -> 133 in 2; at 2048
-// rows every shape is fastest in one part.) A gathered matmul (experts > 0), whose rows an expert the host does not know,
-// takes 128-row tiles in one part.
-GemmPlan gemm_lds_plan(int64_t M, int64_t K, int64_t N, int experts, bool may_split) {
-  if (experts > 0) return {128, 1, 0};
-  GemmPlan best = {};
-  double cost = 0;
-  for (int bm = 256; bm >= 128; bm /= 2) {
-    const int64_t tiles = (M + bm - 1) / bm * ((N + GL_BN - 1) / GL_BN), all = K / GL_BK;
-    for (int s = 1; s <= (may_split ? 16 : 1) && (s == 1 || all / s >= 4); ++s) {
-      const int64_t t = tiles * s;
-      // (parts of at most 256 MB: past it the tiles are over a thousand already, and parts save the last round's rest alone)
-      if (s > 1 && t * bm * GL_BN * 4 > (int64_t)256 << 20) break;
-      double step;
-      if (bm == 256) step = t <= 256 ? 1.0 : 1.15 * ((t + 255) / 256);
-      else step = 1.38 * (t / 512) + (t % 512 == 0 ? 0 : t % 512 <= 256 ? 0.8 : 1.38);
-      const double us = 8 + (all + s - 1) / s * step + (s > 1 ? 6 + 8.0 * s * M * N / 6.5e6 : 0);
-      if (cost == 0 || us < cost) { cost = us; best = {bm, s, us}; }
-    }
-  }
-  return best;
-}
-
-size_t gemm_lds_bytes(const GemmPlan& p, int64_t M, int64_t N) {
-  return p.splits < 2 ? 0 : (size_t)p.splits * ((M + p.bm - 1) / p.bm) * ((N + GL_BN - 1) / GL_BN) * p.bm * GL_BN * 4;
-}
-
 int gemm_lds(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, const GemmPlan& p, float* parts, hipStream_t s) {
-  const int64_t tm = (a.M + p.bm - 1) / p.bm, tn = a.P == 1 ? (a.N / 16 + 7) / 8 : ((int64_t)a.items + 3) / 4;
-  if (tm * tn * p.splits >= 1LL << 23) return fail(FH_EUNSUP, "fh_gemm_bfp: too many tiles");  // (a grid's threads along x stay below 2^32)
-  const int64_t n = g.counts ? (tm * tn * p.splits + 7) / 8 * 8 : tm * tn * p.splits;
-  const dim3 grid((unsigned)n, g.counts ? experts : 1);
+  const int64_t tm = (a.M + p.bm - 1) / p.bm, all = gemm_lds_grid(a, p), tn = all / p.splits / tm;
+  if (!gemm_lds_fits(a, p)) return fail(FH_EUNSUP, "fh_gemm_bfp: too many tiles");
+  const dim3 grid((unsigned)(g.counts ? (all + 7) / 8 * 8 : all), g.counts ? experts : 1);
 #define GL(F, WR, TM) do { \
     if (p.splits < 2) hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, 0>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, 1, parts); \
     else if (TM == 1 && g.split_y) hipLaunchKernelGGL((gemm_lds_kernel<F, WR, 1, 2>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \

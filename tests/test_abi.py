@@ -81,19 +81,20 @@ def test_tile_layout_and_its_refusals():
     lib.call("fh_read_probe", p, 10, p, 1, None)
 
 
-def test_gemm_takes_every_grid_a_launch_holds():
-  # a matmul of up to 2^23 - 1 tiles of 256 rows is launched, not refused (2^30 rows of K 64 and N 16 fit the card); with no
-  # GPU visible the launch itself fails, so the host's checks are all that runs
+def test_gemm_leaves_the_grid_to_the_launch():
+  # rows or columns past what one kernel's grid holds go to the kernel whose tiles are wider (2^30 rows of K 64 by 16 columns,
+  # or 65 rows by 2^30, fit the card): no call is refused for its tiles before that. With no GPU visible the launch itself
+  # fails, so the host's checks are all that runs
   if not lib.PATH.exists(): pytest.skip("libferrite_hip.so not built")
   code = """
 import ctypes
 from ferrite_amd import lib
 b = ctypes.create_string_buffer(4096)
 p = (ctypes.addressof(b) + 63) // 64 * 64
-for M in (65, 1 << 22, (1 << 30) - 256, 1 << 30, (1 << 31) - 256, 1 << 31):
-  try: lib.call("fh_gemm_bfp", p, lib.BF16, 64, M, 64, 16, p, p, lib.BFP8, None, p, lib.F32, 16, None)
+for M, N in ((65, 16), (1 << 22, 16), (1 << 30, 16), ((1 << 31) - 256, 16), (65, (1 << 30) - 128), (65, 1 << 30), (257, 1 << 29)):
+  try: lib.call("fh_gemm_bfp", p, lib.BF16, 64, M, 64, N, p, p, lib.BFP4, None, p, lib.F32, N, None)
   except Exception as e: print(type(e).__name__)
 """
   env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", PYTHONPATH=str(HEADER.parent.parent))
   r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env, check=True)
-  assert r.stdout.split() == ["RuntimeError"] * 5 + ["NotImplementedError"], r.stdout + r.stderr
+  assert r.stdout.split() == ["RuntimeError"] * 7, r.stdout + r.stderr
