@@ -588,6 +588,7 @@ __global__ __launch_bounds__(2 * GM_THREADS, 1) void gemm_pp_kernel(MatArgs a, i
 
 // The tiled kernel over a's M rows (per expert, gathered, when g.counts is set: grid.y = experts)
 int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void* workspace, size_t ws_bytes, hipStream_t s) {
+  if (g.counts && (a.ssq_in || a.kind == FH_EP_ROPE_KV || a.kind == FH_EP_RESIDUAL)) return fail(FH_EUNSUP, "gathered GEMM: STORE or SILU_GATE, no prologue");
   // 256-row tiles (8 waves, the weight's conversion shared by twice the rows) where they still give every CU a
   // workgroup or fewer (measured at 2048 rows of the 8B shapes: o 720 -> 765 TFLOP/s, down 780 -> 895; qkv and gate_up,
   // with more tiles than CUs, slower), 128-row tiles (4 waves, two workgroups a CU) otherwise
@@ -638,7 +639,6 @@ int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void*
   const int64_t tiles_m = (a.M + GM_BM * TMv - 1) / (GM_BM * TMv);
   const int64_t tiles_n = tiles_n0;
   if (tiles_m * tiles_n >= (1LL << 31)) return fail(FH_EUNSUP, "fh_gemm_bfp: too many tiles");
-  if (g.counts && (a.ssq_in || a.kind == FH_EP_ROPE_KV || a.kind == FH_EP_RESIDUAL)) return fail(FH_EUNSUP, "gathered GEMM: STORE or SILU_GATE, no prologue");
   // (gathered: a grid for the most rows an expert can have, in whole multiples of the 8 XCDs)
   const int64_t tiles = g.counts ? (tiles_m * tiles_n + 7) / 8 * 8 : tiles_m * tiles_n;
   const dim3 grid((unsigned)tiles, g.counts ? experts : 1), b(GM_THREADS * TMv);
