@@ -1,7 +1,7 @@
 // The tiled matmul by a block-float weight for bf16 rows whose K is whole steps of 64 (a prompt's matmuls, a mixture's
 // gathered experts): x straight from memory into LDS, the weight converted on its way there.
 //
-// A workgroup of 2 WR waves takes 32 WR TM rows by 128 columns (8 runs of 16, or 4 runs and their RoPE / SiLU·gate
+// A workgroup of 8 waves takes 128 TM rows by 128 columns (8 runs of 16, or 4 runs and their RoPE / SiLU·gate
 // partners), each wave 32 TM rows by two blocks of 32 columns, the second 64 columns after the first: a pair's two runs,
 // so that a lane holds both of a pair's sums and the epilogue runs on the accumulators where they are. K steps of 64:
 // x's rows go into a ring of two or three LDS stages by global_load_lds_dwordx4 (no registers, no LDS write instructions; each
@@ -19,7 +19,8 @@
 
 namespace fh {
 
-constexpr int GL_RUNS = GL_BN / 16;
+constexpr int GL_RUNS = GL_BN / 16, GL_NW = 8;  // a tile's runs, a workgroup's waves
+static_assert(GL_RUNS == GL_NW, "a wave a run of the weight");
 
 typedef short gl_short4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) gl_short4* gl_lds_short4;
@@ -164,15 +165,14 @@ __device__ __forceinline__ void row_scales(const MatArgs& a, float* rs, int n, i
 
 // MODE 0: K whole; 1: a part of K, its sums left in `parts`; 2: a part of K whose outputs go g.split_y elements after the
 // part before's (a store's only: whoever reads them adds them up)
-template <bool FOUR, int WR, int TM, int MODE>
-__global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits,
-                                                                                  float* parts) {
+template <bool FOUR, int TM, int MODE>
+__global__ __launch_bounds__(64 * GL_NW, TM == 2 ? 2 : 4) void gemm_lds_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits,
+                                                                              float* parts) {
   constexpr bool SPLIT = MODE != 0;
-  constexpr int NW = 2 * WR, BM = 32 * WR * TM, NS = TM == 2 || SPLIT ? 2 : 3;
+  constexpr int BM = 128 * TM, NS = TM == 2 || SPLIT ? 2 : 3;
   constexpr int AB = BM * GL_BK * 2, BB = GL_BK * GL_BN * 2;
-  constexpr int IA = AB / 1024 / NW;           // a wave's loads of x a step (1 KiB, 8 rows each)
-  constexpr int UPT = (GL_RUNS + NW - 1) / NW;  // runs a wave takes, a lane a row of the step
-  constexpr int WL = 2 * (GL_RUNS / NW);        // at least so many loads of the weight a step
+  constexpr int IA = AB / 1024 / GL_NW;  // a wave's loads of x a step (1 KiB, 8 rows each)
+  constexpr int WL = 2;                  // and of the weight: a lane a row of its run, and the row's exponent
   constexpr int RB = FOUR ? 8 : 16;
   using Row = typename std::conditional<FOUR, uint2, uint4>::type;
   __shared__ __attribute__((aligned(16))) char a0[AB];
@@ -186,10 +186,9 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
   int64_t M = a.M, ybase = 0;
   const uint8_t* wmant = a.mant;
   const uint8_t* wexps = a.exps;
-  int id = blockIdx.x, tiles = tiles_m * tiles_n, at = 0;
+  int id = blockIdx.x, tiles = tiles_m * tiles_n;
   if (g.counts) {
     const int e = blockIdx.y;
-    at = e * tiles * splits;  // (its place among the partial sums)
     M = min((int64_t)g.counts[e], a.M);
     ybase = (int64_t)e * a.M;
     wmant += e * g.expert_mant;
@@ -228,45 +227,29 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
     for (int i = 0; i < IA; ++i)
       __builtin_amdgcn_global_load_lds((gl_global)(px[i] + (int64_t)min(step, steps - 1) * GL_BK), (gl_lds)(s + (wave * IA + i) * 1024), 16, 0, 0);
   };
-  // the weight: run wave + NW i of the tile, row `lane` of the step (a run past the weight reads the first; its columns
-  // are not stored)
-  const uint8_t* pm[UPT];
-  const uint8_t* pe[UPT];
-#pragma unroll
-  for (int i = 0; i < UPT; ++i) {
-    const int lr = wave + NW * i;
-    const int64_t nb = lr < GL_RUNS ? tile_run<GL_RUNS>(a, tn, lr) : 0;
-    const int64_t k = (nb < 0 ? 0 : nb) * a.K + (int64_t)first * GL_BK + lane;
-    pm[i] = wmant + k * RB;
-    pe[i] = wexps + k;
-  }
-  Row wm[2][UPT];
-  uint32_t we[2][UPT];
+  // the weight: run `wave` of the tile, row `lane` of the step (a run past the weight reads the first; its columns are not
+  // stored)
+  const int64_t nb = tile_run<GL_RUNS>(a, tn, wave), w0 = (nb < 0 ? 0 : nb) * a.K + (int64_t)first * GL_BK + lane;
+  const uint8_t* pm = wmant + w0 * RB;
+  const uint8_t* pe = wexps + w0;
+  Row wm[2];
+  uint32_t we[2];
   auto load_w = [&](int step, int set) {
     const int64_t k = (int64_t)min(step, steps - 1) * GL_BK;
-#pragma unroll
-    for (int i = 0; i < UPT; ++i) {
-      if (GL_RUNS % NW && wave + NW * i >= GL_RUNS) continue;
-      wm[set][i] = *(const Row*)(pm[i] + k * RB);
-      we[set][i] = pe[i][k];
-    }
+    wm[set] = *(const Row*)(pm + k * RB);
+    we[set] = pe[k];
   };
   auto swz = [](int k) { return 4 * (k & 3) + ((k >> 2) & 3); };  // row k's XOR on a piece's place
   auto store_w = [&](char* s, int set) {
+    float f[16];
+    magnitudes(wm[set], f);
+    const float sc = ldexpf(1.f, (int)we[set] - 133);
+    uint32_t w[8];
 #pragma unroll
-    for (int i = 0; i < UPT; ++i) {
-      const int lr = wave + NW * i;
-      if (GL_RUNS % NW && lr >= GL_RUNS) continue;
-      float f[16];
-      magnitudes(wm[set][i], f);
-      const float sc = ldexpf(1.f, (int)we[set][i] - 133);
-      uint32_t w[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) w[q] = pack_bf16_exact(f[2 * q] * sc, f[2 * q + 1] * sc);
-      char* row = s + lane * GL_BN * 2;
-      *(uint4*)(row + ((2 * lr ^ swz(lane)) << 4)) = make_uint4(w[0], w[1], w[2], w[3]);
-      *(uint4*)(row + (((2 * lr + 1) ^ swz(lane)) << 4)) = make_uint4(w[4], w[5], w[6], w[7]);
-    }
+    for (int q = 0; q < 8; ++q) w[q] = pack_bf16_exact(f[2 * q] * sc, f[2 * q + 1] * sc);
+    char* row = s + lane * GL_BN * 2;
+    *(uint4*)(row + ((2 * wave ^ swz(lane)) << 4)) = make_uint4(w[0], w[1], w[2], w[3]);
+    *(uint4*)(row + (((2 * wave + 1) ^ swz(lane)) << 4)) = make_uint4(w[4], w[5], w[6], w[7]);
   };
 
   floatx16 acc[TM][2];
@@ -345,7 +328,7 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
     if (!live) return;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      float* p = parts + (((int64_t)(at + part * tiles + id) * NW + wave) * TM + i) * 2048 + lane;
+      float* p = parts + (((int64_t)(part * tiles + id) * GL_NW + wave) * TM + i) * 2048 + lane;
       if (m0 + wr + 32 * i < M)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -356,7 +339,7 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
   }
   __syncthreads();  // the stages are free: each wave's outputs, 16 rows at a time, in a part of x's of its own
   constexpr int CW = 16 * GL_LDC * 4, WPA = AB / CW;
-  static_assert(MODE == 1 || (NS + 2) * WPA >= NW, "the outputs' place");
+  static_assert(MODE == 1 || (NS + 2) * WPA >= GL_NW, "the outputs' place");
   float* cs = (float*)((wave < WPA ? a0 : wave < 2 * WPA ? a1 : wave < 3 * WPA ? (NS == 3 ? a2 : b1) : b0) + wave % WPA * CW);
   float* rs_s = (float*)(b0 + BB) - 32 * TM * (wave + 1);
   if (a.ssq_in) row_scales(a, rs_s, 32 * TM, m0 + wr, lane, 64);  // (each wave its own rows' 1/rms, where the weight was)
@@ -374,35 +357,26 @@ __global__ __launch_bounds__(WR * 128, TM == 2 ? 2 : 4) void gemm_lds_kernel(Mat
 // four parts' loads in flight at a time, then the epilogue. Bound by reading the parts once (splits x 4 bytes an output),
 // from the L2 of the XCD that wrote them (o at 200 rows in bfp4, both launches: 30.6 -> 24.7 us against parts dealt to
 // the XCDs part by part).
-template <int WR, int TM>
+template <int TM>
 __global__ __launch_bounds__(256) void split_sum_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits, const float* parts) {
-  constexpr int NW = 2 * WR, BM = 32 * WR * TM;
   __shared__ float rs_s[4][16];
   __shared__ __attribute__((aligned(16))) float cs_s[4][16 * GL_LDC];
-  int64_t M = a.M, ybase = 0;
-  int tiles = tiles_m * tiles_n, at = 0;
-  if (g.counts) {
-    const int e = blockIdx.y;
-    at = e * tiles * splits;
-    M = min((int64_t)g.counts[e], a.M);
-    ybase = (int64_t)e * a.M;
-    tiles_m = (int)((M + BM - 1) / BM);
-    tiles = tiles_m * tiles_n;
-  }
+  const int64_t M = a.M;
+  const int tiles = tiles_m * tiles_n;
   // (workgroups dealt to the XCDs in contiguous ranges, as the tiles' were: a tile's parts are in this XCD's L2)
   const int nb = gridDim.x, blk = nb % 8 == 0 ? (int)(blockIdx.x % 8) * (nb / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
   const int lane = threadIdx.x & 63, u = blk * 4 + (threadIdx.x >> 6);  // unit u: (tile, wave, i, half)
-  const int half = u & 1, i = (u >> 1) % TM, wave = (u >> 1) / TM % NW, id = (u >> 1) / (TM * NW);
+  const int half = u & 1, i = (u >> 1) % TM, wave = (u >> 1) / TM % GL_NW, id = (u >> 1) / (TM * GL_NW);
   if (id >= tiles) return;
   const int per_group = 8 * tiles_n, first_m = id / per_group * 8, gm = min(tiles_m - first_m, 8);
   const int tm = first_m + (id % per_group) % gm, tn = (id % per_group) / gm;
-  const int64_t m0 = (int64_t)tm * BM + ((wave >> 1) * TM + i) * 32 + 16 * half;
+  const int64_t m0 = (int64_t)tm * 128 * TM + ((wave >> 1) * TM + i) * 32 + 16 * half;
   if (m0 >= M) return;
   float* rs = rs_s[threadIdx.x >> 6];
   float* cs = cs_s[threadIdx.x >> 6];
   if (a.ssq_in) row_scales(a, rs, 16, m0, lane, 64);  // (this wave's own rows)
-  const int64_t stride = (int64_t)tiles * NW * TM * 2048;
-  const float* p = parts + (((int64_t)(at + id) * NW + wave) * TM + i) * 2048 + 512 * half + lane;
+  const int64_t stride = (int64_t)tiles * GL_NW * TM * 2048;
+  const float* p = parts + (((int64_t)id * GL_NW + wave) * TM + i) * 2048 + 512 * half + lane;
   float acc[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -420,7 +394,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(MatArgs a, SkinnyMoe g, 
 #pragma unroll
   for (int r = 0; r < 16; ++r) cs[(8 * ((r & 7) >> 2) + 4 * (lane >> 5) + (r & 3)) * GL_LDC + 32 * (r >> 3) + (lane & 31)] = acc[r];
   wave_lds_order();
-  block_epilogue(a, g, cs, tn, (wave & 1) * 32, m0, M, ybase, lane, a.ssq_in ? rs : nullptr);
+  block_epilogue(a, g, cs, tn, (wave & 1) * 32, m0, M, 0, lane, a.ssq_in ? rs : nullptr);
 }
 
 bool gemm_lds_takes(const MatArgs& a) {
@@ -430,18 +404,18 @@ bool gemm_lds_takes(const MatArgs& a) {
 int gemm_lds(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, const GemmPlan& p, float* parts, hipStream_t s) {
   const int64_t tm = (a.M + p.bm - 1) / p.bm, all = gemm_lds_grid(a, p), tn = all / p.splits / tm;
   if (!gemm_lds_fits(a, p)) return fail(FH_EUNSUP, "fh_gemm_bfp: too many tiles");
-  const dim3 grid((unsigned)(g.counts ? (all + 7) / 8 * 8 : all), g.counts ? experts : 1);
-#define GL(F, WR, TM) do { \
-    if (p.splits < 2) hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, 0>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, 1, parts); \
-    else if (TM == 1 && g.split_y) hipLaunchKernelGGL((gemm_lds_kernel<F, WR, 1, 2>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
+  if (p.splits > 1 && !g.split_y && (!parts || g.counts)) return fail(FH_EINVAL, "fh_gemm_bfp: K in parts needs a place for their sums");
+  const dim3 grid((unsigned)(g.counts ? (all + 7) / 8 * 8 : all), g.counts ? experts : 1), block(64 * GL_NW);
+#define GL(F, TM) do { \
+    if (p.splits < 2) hipLaunchKernelGGL((gemm_lds_kernel<F, TM, 0>), grid, block, 0, s, a, g, (int)tm, (int)tn, 1, parts); \
+    else if (TM == 1 && g.split_y) hipLaunchKernelGGL((gemm_lds_kernel<F, 1, 2>), grid, block, 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
     else { \
-      hipLaunchKernelGGL((gemm_lds_kernel<F, WR, TM, 1>), grid, dim3(128 * WR), 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
-      hipLaunchKernelGGL((split_sum_kernel<WR, TM>), dim3((unsigned)(tm * tn * WR * TM), g.counts ? experts : 1), dim3(256), 0, s, a, g, (int)tm, (int)tn, p.splits, (const float*)parts); \
+      hipLaunchKernelGGL((gemm_lds_kernel<F, TM, 1>), grid, block, 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
+      hipLaunchKernelGGL((split_sum_kernel<TM>), dim3((unsigned)(tm * tn * 4 * TM)), dim3(256), 0, s, a, g, (int)tm, (int)tn, p.splits, (const float*)parts); \
     } } while (0)
-#define GL_F(WR, TM) do { if (fmt == FH_BFP4) GL(true, WR, TM); else GL(false, WR, TM); } while (0)
-  if (p.bm == 256) GL_F(4, 2);
-  else GL_F(4, 1);
-#undef GL_F
+  if (p.bm == 256) { if (fmt == FH_BFP4) GL(true, 2); else GL(false, 2); }
+  else if (fmt == FH_BFP4) GL(true, 1);
+  else GL(false, 1);
 #undef GL
   return check_launch("fh_gemm_bfp");
 }

@@ -279,14 +279,12 @@ __global__ __launch_bounds__(256, KS == 1 ? 2 : 1) void attention_prefill_kernel
   }
 
   if constexpr (KS > 1) {
-    // the waves' parts meet: each leaves its sums, its max and its exponents' sum in LDS (where the tiles were); wave w
+    // the waves' parts meet: each leaves its sums, its max and its exponents' sum in LDS (where K's tiles were); wave w
     // then adds block w of the dimensions over the parts, in order, each part times 2^(its max - the largest)
     __shared__ float ml[KS][2][64];
     constexpr int PB = HD / 32;  // blocks of 32 dimensions
-    float* parts = (float*)Ks2;
-    constexpr int IN = (int)(sizeof(Ks2) / (16 * 64 * 4));  // blocks that fit where K was; the rest where V was
-    auto part = [&](int w, int d) { const int i = w * PB + d; return (i < IN ? parts + i * 1024 : (float*)Vt2 + (i - IN) * 1024) + lane; };
-    static_assert((KS * PB - IN) * 4096 <= (int)sizeof(Vt2), "the parts' place");
+    auto part = [&](int w, int d) { return (float*)Ks2 + (w * PB + d) * 1024 + lane; };
+    static_assert(KS * PB * 4096 <= (int)sizeof(Ks2), "the parts' place");
     __syncthreads();
 #pragma unroll
     for (int d = 0; d < PB; ++d)
