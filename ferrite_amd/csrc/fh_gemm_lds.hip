@@ -31,11 +31,13 @@ typedef __attribute__((address_space(3))) uint32_t* gl_lds;
 // (LDS, this wave's own: [16][GL_LDC], a row's two blocks side by side). rs: the rows' 1/rms, or null for 1. Short loops,
 // not unrolled rows: a workgroup runs this once, at the pace its instructions arrive (unrolled over the accumulators the
 // kernel was 90 KB of code, and a call of one K step took 13 us).
+// PLAIN: a store of the sums alone, whatever else the other epilogues would need left out.
 constexpr int GL_LDC = 68;
+template <bool PLAIN = false>
 __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe& g, const float* cs, int tn, int wc, int64_t m0,
                                                int64_t M, int64_t ybase, int lane, const float* rs, int64_t y0 = 0) {
-  const int kind = a.kind;
-  if (a.P == 1) {  // a lane 4 columns of a row, 4 rows a pass
+  const int kind = PLAIN ? FH_EP_STORE : a.kind;
+  if (PLAIN || a.P == 1) {  // a lane 4 columns of a row, 4 rows a pass
     const int q = lane & 15, c = 4 * q, lc = wc + (c & 31);
     const int64_t run = tile_run<GL_RUNS>(a, tn, 4 * (q >> 3) + (lc >> 4)), col = run * 16 + (lc & 15);
     const bool res = kind == FH_EP_RESIDUAL;
@@ -67,7 +69,7 @@ __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe
         for (int k = 0; k < 4; ++k) { s[k] += __shfl_xor(s[k], 2, 64); s[k] += __shfl_xor(s[k], 1, 64); }
         if (ok && !(q & 3)) a.ssq_out[m * (a.N / 16) + run] = (s[0] + s[2]) + (s[1] + s[3]);
       }
-      if (kind == FH_EP_STORE && a.argmax_parts) {
+      if (!PLAIN && kind == FH_EP_STORE && a.argmax_parts) {
         float bv = v.x;
         int bc = (int)col;
         if (v.y > bv) { bv = v.y; bc = (int)col + 1; }
@@ -348,7 +350,7 @@ __global__ __launch_bounds__(64 * GL_NW, TM == 2 ? 2 : 4) void gemm_lds_kernel(M
     for (int ii = 0; ii < TM; ++ii)  // (the accumulators' indices stay constants)
       if (ii == u >> 1) block_to_lds(cs, acc[ii], u & 1, lane);
     wave_lds_order();
-    block_epilogue(a, g, cs, tn, wc, m0 + wr + 16 * u, M, ybase, lane, a.ssq_in ? rs_s + 16 * u : nullptr, MODE == 2 ? part * g.split_y : 0);
+    block_epilogue<MODE == 2>(a, g, cs, tn, wc, m0 + wr + 16 * u, M, ybase, lane, a.ssq_in ? rs_s + 16 * u : nullptr, MODE == 2 ? part * g.split_y : 0);
     wave_lds_order();
   }
 }
