@@ -1,6 +1,7 @@
 """The tiled matmul of bf16 rows whose x goes straight into LDS (fh_gemm_lds.hip): every epilogue at the edges of its
-tiles, in one part of K against the kernel that fp32 rows take (the same bf16 products in the same order: the same bits),
-and with K in parts within fp32 summation's error of that. Rows past M of x's buffer hold NaN: none may reach a sum."""
+tiles of 128 and 256 rows, in one part of K against the kernel that fp32 rows take (the same bf16 products in the same order:
+the same bits), and with K in parts within fp32 summation's error of that. Rows past M of x's buffer hold NaN: none may reach
+a sum."""
 import ctypes
 import pytest
 import torch
@@ -8,6 +9,22 @@ from ferrite_amd import llama as G
 
 pytestmark = pytest.mark.gpu
 HD = 64
+# (M, K, N): the plan's rows a tile and parts of K. Both tiles, whole and in parts; one row or column block more or less than
+# a tile; parts of unequal length (32 steps in 7, 64 in 13)
+PLANS = {(65, 64, 16): (128, 1), (96, 192, 144): (128, 1), (127, 1536, 576): (128, 6), (128, 4096, 128): (128, 16), (129, 320, 2064): (128, 1),
+         (200, 4096, 1024): (128, 16), (257, 576, 960): (128, 1), (300, 1024, 4096): (128, 1), (1000, 512, 6144): (256, 1),
+         (129, 2048, 4112): (256, 7), (130, 4096, 2064): (256, 13), (257, 4096, 4096): (256, 4), (200, 1536, 6144): (256, 4)}
+# the same for qkv matmuls: heads and kv heads of HD
+ROPES = {(65, 64, 1, 1): (128, 1), (130, 576, 9, 3): (128, 1), (200, 576, 4, 1): (128, 1), (96, 4096, 5, 2): (128, 16), (300, 4096, 9, 3): (128, 10),
+         (129, 2048, 33, 15): (128, 4), (257, 4096, 33, 15): (256, 4)}
+
+
+def parts_bytes(lib, M, K, N, plan):
+  """The workspace of the plan that the test is for."""
+  bm, splits = plan
+  n = lib.load().fh_gemm_workspace_bytes(M, K, N)
+  assert n == (splits * -(-M // bm) * bm * -(-N // 128) * 128 * 4 if splits > 1 else 0)
+  return n
 
 
 def both(ops, lib, x, bw, make, out_shape, dtype, ws_bytes):
@@ -26,8 +43,7 @@ def both(ops, lib, x, bw, make, out_shape, dtype, ws_bytes):
 
 
 @pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
-@pytest.mark.parametrize("M,K,N", [(65, 64, 16), (96, 192, 144), (127, 1536, 576), (128, 4096, 128), (129, 320, 2064),
-                                   (200, 4096, 1024), (257, 576, 960), (300, 1024, 4096), (1000, 512, 6144)])
+@pytest.mark.parametrize("M,K,N", list(PLANS))
 def test_every_epilogue_at_tile_edges(cuda, fmt, M, K, N):
   from ferrite_amd import lib, ops
   g = torch.Generator(device="cuda").manual_seed(M + 3 * K + 7 * N)
@@ -35,7 +51,7 @@ def test_every_epilogue_at_tile_edges(cuda, fmt, M, K, N):
   x = torch.full((M + 8, K), float("nan"), dtype=torch.bfloat16, device="cuda")
   x[:M] = rand(M, K)
   x = x[:M]
-  n = lib.load().fh_gemm_workspace_bytes(M, K, N)
+  n = parts_bytes(lib, M, K, N, PLANS[M, K, N])
 
   def check(bw, make, shape, dtype, bound, what):
     old, one, split = both(ops, lib, x, bw, make, shape, dtype, n)
@@ -47,7 +63,10 @@ def test_every_epilogue_at_tile_edges(cuda, fmt, M, K, N):
   w = rand(K, N) * 0.02
   bw = ops.pack(w, fmt)
   mag = (x.double().abs() @ ops.dequant(bw).double().abs())
-  near = 2 ** -21 * mag  # sums of exact products in another order: at most K / 16 roundings of 2^-24 of sum |x w|, K <= 4096 twice over
+  # sums of exact products in another order: K / 16 roundings a side, each of at most 2^-24 of a partial sum, which products of
+  # random signs keep within 4 sum |x w| / sqrt(K); of random signs themselves, 2^-24 of sum |x w| in all whatever K, and
+  # eight times that for the largest of millions of outputs
+  near = 2 ** -21 * mag
   def store(out):
     parts = torch.zeros(M, N // 16, dtype=torch.int64, device="cuda")
     return ops.epilogue(lib.EP_STORE, argmax_parts=parts), [parts]
@@ -95,7 +114,7 @@ def cache_parts(data, kind, rows):
 
 
 @pytest.mark.parametrize("kind", ["fp32", "bf16", "bfp8", "bfp4"])
-@pytest.mark.parametrize("M,K,heads,kv", [(65, 64, 1, 1), (130, 576, 9, 3), (200, 576, 4, 1), (96, 4096, 5, 2), (300, 4096, 9, 3)])
+@pytest.mark.parametrize("M,K,heads,kv", list(ROPES))
 def test_rope_where_the_pairs_end_inside_a_tile(cuda, kind, M, K, heads, kv):
   """A qkv matmul whose pairs of runs are no whole tiles (SmolLM's 30 in tiles of 4 among them), rows at place 0 among
   the others, on fp32 rows, on bf16 rows with K whole (the same bits) and with K in parts (fp32 sums in another order; the
@@ -115,7 +134,7 @@ def test_rope_where_the_pairs_end_inside_a_tile(cuda, kind, M, K, heads, kv):
     data, dt, length = ops.cache_fields(cache)
     return ops.epilogue(lib.EP_ROPE_KV, heads=heads, kv_heads=kv, head_dim=HD, cos_tab=cos, sin_tab=sin, rope_rows=64, places=places,
                         cache_rows=rows, cache=data, cache_dtype=dt, cache_len=length), [data]
-  old, one, split = both(ops, lib, x, bw, rope, (M, heads * HD), torch.float32, lib.load().fh_gemm_workspace_bytes(M, K, N))
+  old, one, split = both(ops, lib, x, bw, rope, (M, heads * HD), torch.float32, parts_bytes(lib, M, K, N, ROPES[M, K, heads, kv]))
   for a, b in zip(old, one): assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
   # against 64 bits: q turned by its row's place, k turned and v as they are in the cache rows
   y = (x.double() @ ops.dequant(bw).double()).reshape(M, -1, HD)

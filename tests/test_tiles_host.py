@@ -102,3 +102,27 @@ def test_packing_in_tiles_where_it_is_the_faster(tmp_path):
   got = {(int(k), int(r)): t == "1" for k, r, t in (l.split() for l in out)}
   for (K, runs), tiles in got.items():
     assert tiles == (K >= 8 and K * runs >= 131072 and (runs + 15) // 16 * 256 < 2 ** 32 and -(-K // 64) < 65536), (K, runs)
+
+
+PLAN = r'''
+#include "fh_gemm.h"
+#include <cstdio>
+int main(int c, char** v) {
+  for (int i = 1; i + 2 < c; i += 3) {
+    const fh::GemmPlan p = fh::gemm_lds_plan(atoll(v[i]), atoll(v[i + 1]), atoll(v[i + 2]), 0, true);
+    printf("%d %d\n", p.bm, p.splits);
+  }
+}
+'''
+
+
+def test_the_tiled_matmuls_tests_take_the_plans_they_name(tmp_path):
+  """The shapes of the tiled matmul's GPU tests have the tiles and the parts of K that they are there for, and both tiles
+  are there whole and in parts."""
+  from test_gpu_16_gemm_lds import HD, PLANS, ROPES
+  want = [(s, p) for s, p in PLANS.items()] + [((M, K, (h + 2 * kv) * HD), p) for (M, K, h, kv), p in ROPES.items()]
+  args = [str(x) for s, _ in want for x in s]
+  out = subprocess.run([str(program(tmp_path, PLAN)), *args], capture_output=True, text=True, check=True).stdout.splitlines()
+  assert [tuple(map(int, l.split())) for l in out] == [p for _, p in want]
+  for plans in (PLANS, ROPES): assert {(bm, s > 1) for bm, s in plans.values()} >= {(128, False), (128, True), (256, True)}
+  assert (256, 1) in PLANS.values()
