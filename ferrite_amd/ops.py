@@ -14,9 +14,15 @@ def _ptr(t):  # (a pointer argument takes a plain integer)
   return t.data_ptr() if t is not None else None
 
 
+try:  # (names of torch's own, which make no stream object a call; a torch without them takes the public one)
+  from torch._C import _cuda_getCurrentRawStream as _raw_stream, _cuda_getDevice as _device
+except ImportError:
+  _raw_stream, _device = lambda device: torch.cuda.current_stream(device).cuda_stream, lambda: None
+
+
 def _stream():
-  """The current device's current stream, raw (what torch.cuda.current_stream().cuda_stream is, without the objects)."""
-  return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+  """The current device's current stream, raw: torch.cuda.current_stream().cuda_stream."""
+  return _raw_stream(_device())
 
 
 def _dev(*ts):

@@ -98,3 +98,17 @@ for M, N in ((65, 16), (1 << 22, 16), (1 << 30, 16), ((1 << 31) - 256, 16), (65,
   env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", PYTHONPATH=str(HEADER.parent.parent))
   r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env, check=True)
   assert r.stdout.split() == ["RuntimeError"] * 7, r.stdout + r.stderr
+
+
+def test_streams_of_a_torch_without_its_raw_names(monkeypatch):
+  # ops asks torch for the raw stream by names of its own; where they are gone, the public call gives the same
+  import importlib.util, types
+  import torch
+  from ferrite_amd import ops
+  for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"): monkeypatch.delattr(torch._C, n, raising=False)
+  spec = importlib.util.spec_from_file_location("ops_of_another_torch", ops.__file__)
+  m = importlib.util.module_from_spec(spec)
+  monkeypatch.setitem(sys.modules, spec.name, m)
+  spec.loader.exec_module(m)
+  monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: types.SimpleNamespace(cuda_stream=77 if device is None else 0))
+  assert m._stream() == 77
