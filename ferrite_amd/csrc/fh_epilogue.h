@@ -98,14 +98,14 @@ __device__ inline void cache_put(const MatArgs& a, int ch, int32_t crow, int d, 
 // RoPE, where half = head_dim / 32; gate and up for SiLU·gate, where half = split / 16 and there is one group).
 __host__ __device__ inline int64_t pair_first(int64_t item, int half) { return item / half * (2 * half) + item % half; }
 
-// Where a RoPE pair's first half lies: column j of run `run` is dimension d of head h, its partner dimension d1, and
-// `turn` whether the head is one of q's or k's, whose pairs turn by row (place, d) and (place, d1) of the tables. A run
-// past the weight (-1: a tile's last pairs where it has no more) is no head's: nothing turns, so no table is read.
+// Where a RoPE pair's first half lies, heads of hd: column j of run `run` is dimension d of head h, its partner dimension
+// d1, and `turn` whether the head is one of the first `turning`, q's and k's, whose pairs turn by row (place, d) and (place,
+// d1) of the tables. A run past the weight (-1: a tile's last pairs where it has no more) is no head's, its d none: nothing
+// turns, so no table is read.
 struct RopePair { int h, d, d1; bool turn; };
-__host__ __device__ inline RopePair rope_pair(const MatArgs& a, int64_t run, int j) {
-  const int hd = a.head_dim, c0 = run < 0 ? 0 : (int)run * 16 + j;  // (c0 < N < 2^31)
-  const int h = c0 / hd, d = c0 % hd;
-  return {h, d, d + hd / 2, run >= 0 && h < a.heads + a.kv_heads};
+__host__ __device__ inline RopePair rope_pair(int hd, int turning, int64_t run, int j) {
+  const int c0 = (int)run * 16 + j, h = c0 / hd, d = c0 % hd;  // (c0 < N < 2^31)
+  return {h, d, d + hd / 2, run >= 0 && h < turning};
 }
 
 // A grouped (mixture-of-experts) skinny matmul's extras (fh_skinny.hip): grid.y = expert, its weight `expert_mant` /

@@ -28,6 +28,41 @@ __host__ __device__ inline int64_t tile_run(const MatArgs& a, int tn, int lr) {
   return lr < RUNS / 2 ? nb0 : nb0 + a.pair_half;
 }
 
+// 1/rms of 16 rows from m0 on (past the matrix: its last row's) into rs (LDS), from the sums of squares their maker left by
+// runs of 16, by one wave: a row's sums lie along the lanes (a load of a wave is one piece of a row), 16 rows at once and two
+// loads of each in flight, then the lanes' sums meet for all 16 rows together. (Two threads a row, each reading every other
+// sum in turn, take 32 rows' lines a load: 30 us a 256-row tile of K 4096, or 57 by the waves that own the rows, against 5.)
+__device__ __forceinline__ void row_scales16(const MatArgs& a, float* rs, int64_t m0, int lane) {
+  const float* q = a.ssq_in + min(m0, a.M - 1) * a.ssq_parts;
+  const int last = (int)min((int64_t)15, max((int64_t)0, a.M - 1 - m0));
+  float v[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) v[r] = 0.f;
+#pragma unroll 1
+  for (int i0 = 0; i0 < a.ssq_parts; i0 += 128) {
+    const int i = i0 + lane, j = i + 64;
+    const bool oki = i < a.ssq_parts, okj = j < a.ssq_parts;
+    float u[2][16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const uint32_t row = min(r, last) * a.ssq_parts;  // (a.ssq_parts < 2^27)
+      u[0][r] = q[row + (oki ? i : 0)];
+      u[1][r] = q[row + (okj ? j : 0)];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) { v[r] += oki ? u[0][r] : 0.f; v[r] += okj ? u[1][r] : 0.f; }
+  }
+  wave_reduce16(v);
+  if (!(lane & 3)) rs[reduce16_index(lane)] = 1.0f / sqrtf(v[0] / (float)a.K + a.eps);
+}
+
+// RoPE's per-row values for a tile's epilogue, staged in LDS: row ar's place and cache row (m: the row, clamped into the
+// matrix)
+__device__ inline void stage_rope_rows(const MatArgs& a, int32_t* rows_s, int bm, int ar, int64_t m) {
+  rows_s[ar] = a.places[m];
+  rows_s[bm + ar] = a.cache_rows[m];
+}
+
 // gemm_tiles' kernel for bf16 rows whose K is whole steps of 64 (fh_gemm_lds.hip): tiles of 128 columns in K steps of 64
 constexpr int GL_BK = 64, GL_BN = 128;
 struct GemmPlan { int bm; int splits; double us; };  // rows a tile, K's parts, and the time expected of it

@@ -33,13 +33,6 @@ constexpr int GM_LDC = GM_BN + 4;    // LDS row of the fp32 output tile
 constexpr int GM_THREADS = 256;
 constexpr int GM_GROUP = 8;          // row tiles a group (tile order)
 
-// RoPE's per-row values for the epilogue, staged in LDS while the tile's first loads are in flight: row ar's place and
-// cache row (m: the row, clamped into the matrix)
-__device__ inline void stage_rope_rows(const MatArgs& a, int32_t* rows_s, int bm, int ar, int64_t m) {
-  rows_s[ar] = a.places[m];
-  rows_s[bm + ar] = a.cache_rows[m];
-}
-
 // The tile's epilogue: every output of the fp32 tile Cs [BM][BN + 4] (staged in LDS: each output sees its row's 1/rms
 // and its pair partner, whichever wave computed it) through a's epilogue, NT threads (those of whole passes over the
 // tile's columns: NT / BN of them a pass, the rest idle; a pass's threads start at a multiple of 64, so a run's 16
@@ -113,7 +106,7 @@ __device__ inline void gemm_epilogue(const MatArgs& a, const SkinnyMoe& g, const
     const int64_t c0 = run * 16 + j;
     const bool rope = kind == FH_EP_ROPE_KV;
     const int hd = rope ? a.head_dim : 1;
-    const auto [h, d, d1, turn] = rope ? rope_pair(a, run, j) : RopePair{};  // (turn: x cos + (-x2, x1) sin, models/llama.py:92-93)
+    const auto [h, d, d1, turn] = rope_pair(hd, rope ? a.heads + a.kv_heads : 0, run, j);  // (turn: x cos + (-x2, x1) sin, models/llama.py:92-93)
     constexpr int S = NT / H, RB = 8;
     for (int rb = t / H; rb < BM; rb += RB * S) {
       float cs0[RB], cs1[RB], sn0[RB], sn1[RB], sc[RB];
@@ -299,18 +292,6 @@ __global__ __launch_bounds__(GM_THREADS * TM, 3 - TM) void gemm_kernel(MatArgs a
   load(0, x0, w0, e0);
   load(GM_BK, x1, w1, e1);
 
-  // each row's 1 / rms from the sums of squares its maker left by runs of 16 (two threads a row)
-  if (a.ssq_in) {  // (NORM, or rows that already hold x * w)
-    float s = 0.f;
-    if (xok) {
-      const float* q = a.ssq_in + xrow * a.ssq_parts;
-      for (int i = ah; i < a.ssq_parts; i += 2) s += q[i];
-    }
-    s += __shfl_xor(s, 1, 64);
-    if (ah == 0) rs_s[ar] = 1.0f / sqrtf(s / (float)K + a.eps);
-  } else if (ah == 0) {
-    rs_s[ar] = 1.f;
-  }
   if (a.kind == FH_EP_ROPE_KV && ah == 1) stage_rope_rows(a, rows_s, BM, ar, xr0);
 
   floatx16 acc[2][2];
@@ -353,6 +334,14 @@ __global__ __launch_bounds__(GM_THREADS * TM, 3 - TM) void gemm_kernel(MatArgs a
     store(k0 + 2 * GM_BK, 0, x0, w0, e0);  // (past the last step: a stage nobody reads)
   }
 
+  // each row's 1 / rms (here and not while the first loads are in flight: the loop's registers are free)
+  if (a.ssq_in) {  // (NORM, or rows that already hold x * w)
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll 1
+    for (int r = 32 * w; r < 32 * w + 32; r += 16) row_scales16(a, rs_s + r, m0 + r, lane);
+  } else if (ah == 0) {
+    rs_s[ar] = 1.f;
+  }
   // the output tile, fp32, through LDS: block (i, j)'s value r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4,
   // column l % 32
   __syncthreads();
@@ -513,22 +502,10 @@ __global__ __launch_bounds__(2 * GM_THREADS, 1) void gemm_pp_kernel(MatArgs a, i
     __builtin_amdgcn_s_setprio(0);
   };
 
-  // each row's 1 / rms from the sums of squares its maker left by runs of 16 (two threads a row)
-  auto row_scales = [&] {
-    const int ar = t >> 1, ah = t & 1;
-    const int64_t xrow = min(m0 + ar, M - 1);
-    if (a.ssq_in) {
-      float s = 0.f;
-      if (m0 + ar < M) {
-        const float* q = a.ssq_in + xrow * a.ssq_parts;
-        for (int i = ah; i < a.ssq_parts; i += 2) s += q[i];
-      }
-      s += __shfl_xor(s, 1, 64);
-      if (ah == 0) rs_s[ar] = 1.0f / sqrtf(s / (float)K + a.eps);
-    } else if (ah == 0) {
-      rs_s[ar] = 1.f;
-    }
-    if (a.kind == FH_EP_ROPE_KV && ah == 1) stage_rope_rows(a, rows_s, BM, ar, xrow);
+  // RoPE's places and cache rows of the rows
+  auto stage_rows = [&] {
+    const int ar = t >> 1;
+    if (a.kind == FH_EP_ROPE_KV && (t & 1)) stage_rope_rows(a, rows_s, BM, ar, min(m0 + ar, M - 1));
   };
   // Each group runs a loop of its own (the same barriers, in the same order), so that the compiler sees one group's
   // loads alone and waits only for the set a store takes, not for the loads issued after it. Step s's operands are
@@ -538,7 +515,7 @@ __global__ __launch_bounds__(2 * GM_THREADS, 1) void gemm_pp_kernel(MatArgs a, i
   // (An odd count of steps ends with a step of zero weights.)
   if (wgrp) {
     load_w(0, 0); load_w(GM_BK, 1); store_w(0, 0, 0); load_w(2 * GM_BK, 0);
-    row_scales();
+    stage_rows();
     __syncthreads();
     for (int s = 0; s * GM_BK < K; s += 2) {
       compute(0);
@@ -552,7 +529,7 @@ __global__ __launch_bounds__(2 * GM_THREADS, 1) void gemm_pp_kernel(MatArgs a, i
     }
   } else {
     load_x(0, 0); load_x(GM_BK, 1); store_x(0, 0); load_x(2 * GM_BK, 0);
-    row_scales();
+    stage_rows();
     __syncthreads();
     for (int s = 0; s * GM_BK < K; s += 2) {
       store_x(1, 1); load_x((s + 3) * GM_BK, 1);
@@ -566,6 +543,14 @@ __global__ __launch_bounds__(2 * GM_THREADS, 1) void gemm_pp_kernel(MatArgs a, i
     }
   }
 
+  // each row's 1 / rms
+  if (a.ssq_in) {
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll 1
+    for (int r = 32 * w; r < 32 * w + 32; r += 16) row_scales16(a, rs_s + r, m0 + r, lane);
+  } else if (!(t & 1)) {
+    rs_s[t >> 1] = 1.f;
+  }
   // the output tile, fp32, through LDS (the stages are free: the last barrier passed every wave's products), in one
   // pass or in two of 128 rows (waves 0-3's rows, then 4-7's)
   for (int h = 0; h < BM / CROWS; ++h) {

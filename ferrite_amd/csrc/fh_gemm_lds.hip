@@ -28,16 +28,21 @@ typedef const __attribute__((address_space(1))) uint32_t* gl_global;
 typedef __attribute__((address_space(3))) uint32_t* gl_lds;
 
 // A wave's 16 rows m0 .. by two blocks of 32 columns (columns wc and 64 + wc of the tile) through a's epilogue, from cs
-// (LDS, this wave's own: [16][GL_LDC], a row's two blocks side by side). rs: the rows' 1/rms, or null for 1. Short loops,
+// (LDS, this wave's own: [16][GL_LDC], a row's two blocks side by side). rs: the rows' 1/rms, or null for 1; place, crow:
+// RoPE's places and cache rows of them (all in LDS). Short loops,
 // not unrolled rows: a workgroup runs this once, at the pace its instructions arrive (unrolled over the accumulators the
 // kernel was 90 KB of code, and a call of one K step took 13 us).
-// PLAIN: a store of the sums alone, whatever else the other epilogues would need left out.
+// EPI: which of the epilogues this is the code of (GL_PLAIN: a store of the sums alone), a kernel each: one kernel of all of
+// them needs their registers together, and with 128 rows a tile, where two workgroups a CU leave 128 a lane, kept 80 to 140
+// bytes a lane of scratch (the 8B gate_up at 300 rows 125 us with 80, 156 with 136).
 constexpr int GL_LDC = 68;
-template <bool PLAIN = false>
+enum { GL_SUMS, GL_SILU, GL_ROPE, GL_PLAIN };
+template <int EPI>
 __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe& g, const float* cs, int tn, int wc, int64_t m0,
-                                               int64_t M, int64_t ybase, int lane, const float* rs, int64_t y0 = 0) {
-  const int kind = PLAIN ? FH_EP_STORE : a.kind;
-  if (PLAIN || a.P == 1) {  // a lane 4 columns of a row, 4 rows a pass
+                                               int64_t M, int64_t ybase, int lane, const float* rs, const int32_t* place,
+                                               const int32_t* crow, int64_t y0 = 0) {
+  const int kind = EPI == GL_PLAIN ? FH_EP_STORE : a.kind;
+  if constexpr (EPI == GL_SUMS || EPI == GL_PLAIN) {  // FH_EP_STORE, FH_EP_RESIDUAL: a lane 4 columns of a row, 4 rows a pass
     const int q = lane & 15, c = 4 * q, lc = wc + (c & 31);
     const int64_t run = tile_run<GL_RUNS>(a, tn, 4 * (q >> 3) + (lc >> 4)), col = run * 16 + (lc & 15);
     const bool res = kind == FH_EP_RESIDUAL;
@@ -69,7 +74,7 @@ __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe
         for (int k = 0; k < 4; ++k) { s[k] += __shfl_xor(s[k], 2, 64); s[k] += __shfl_xor(s[k], 1, 64); }
         if (ok && !(q & 3)) a.ssq_out[m * (a.N / 16) + run] = (s[0] + s[2]) + (s[1] + s[3]);
       }
-      if (!PLAIN && kind == FH_EP_STORE && a.argmax_parts) {
+      if (EPI == GL_SUMS && kind == FH_EP_STORE && a.argmax_parts) {
         float bv = v.x;
         int bc = (int)col;
         if (v.y > bv) { bv = v.y; bc = (int)col + 1; }
@@ -89,7 +94,7 @@ __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe
   // the pairs: a lane a column of the first run (its partner in the second block), 2 rows a pass; a run is 16 lanes
   const int c = lane & 31, j = lane & 15;
   const int64_t run = tile_run<GL_RUNS>(a, tn, (wc + c) >> 4), c0 = run * 16 + j;
-  if (kind == FH_EP_SILU_GATE) {
+  if constexpr (EPI == GL_SILU) {
     float sc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) sc[i] = g.scale_rows ? g.row_w[ybase + min(m0 + (lane >> 5) + 2 * i, M - 1)] : 1.f;
@@ -103,22 +108,21 @@ __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe
     return;
   }
   const int hd = a.head_dim;
-  const auto [h, d, d1, turn] = rope_pair(a, run, j);  // (turn: x cos + (-x2, x1) sin, models/llama.py:92-93)
-  for (int i0 = 0; i0 < 8; i0 += 4) {
-    float cs0[4], cs1[4], sn0[4], sn1[4];
-    int32_t crow[4];
+  const auto [h, d, d1, turn] = rope_pair(hd, a.heads + a.kv_heads, run, j);  // (turn: x cos + (-x2, x1) sin, models/llama.py:92-93)
+  float tab[2][4][4];  // 4 rows' table values, and the next 4's: all loads before the first store, which may alias them
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t m = min(m0 + (lane >> 5) + 2 * (i0 + u), M - 1);
-      crow[u] = a.cache_rows[m];
-      cs0[u] = cs1[u] = 1.f;
-      sn0[u] = sn1[u] = 0.f;
-      if (turn) {
-        const int64_t place = rope_place(a, a.places[m]);
-        cs0[u] = a.cos_tab[place * hd + d]; cs1[u] = a.cos_tab[place * hd + d1];
-        sn0[u] = a.sin_tab[place * hd + d]; sn1[u] = a.sin_tab[place * hd + d1];
-      }
+  for (int u = 0; u < 8; ++u) {
+    float* v = tab[u >> 2][u & 3];
+    v[0] = v[1] = 1.f;
+    v[2] = v[3] = 0.f;
+    if (turn) {
+      const int64_t at = rope_place(a, place[(lane >> 5) + 2 * u]) * hd;
+      v[0] = a.cos_tab[at + d]; v[1] = a.cos_tab[at + d1];
+      v[2] = a.sin_tab[at + d]; v[3] = a.sin_tab[at + d1];
     }
+  }
+#pragma unroll 1
+  for (int i0 = 0; i0 < 8; i0 += 4) {  // (a loop of two: the put into a cache is long)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int r = (lane >> 5) + 2 * (i0 + u);
@@ -127,16 +131,21 @@ __device__ __forceinline__ void block_epilogue(const MatArgs& a, const SkinnyMoe
       const float s = rs ? rs[r] : 1.f;
       float x0 = cs[r * GL_LDC + c] * s, x1 = cs[r * GL_LDC + 32 + c] * s;
       if (turn) {
-        const float t0 = x0 * cs0[u] - x1 * sn0[u], t1 = x1 * cs1[u] + x0 * sn1[u];
+        const float* v = tab[0][u];
+        const float t0 = x0 * v[0] - x1 * v[2], t1 = x1 * v[1] + x0 * v[3];
         x0 = t0; x1 = t1;
       }
       if (h < a.heads) {
         float* q = (float*)a.y + m * a.ldy + (int64_t)h * hd;
         q[d] = x0; q[d1] = x1;
       } else {
-        cache_put(a, h - a.heads, crow[u], d, d1, j, x0, x1);
+        cache_put(a, h - a.heads, crow[r], d, d1, j, x0, x1);
       }
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) tab[0][u][k] = tab[1][u][k];
   }
 }
 
@@ -151,23 +160,9 @@ __device__ __forceinline__ void block_to_lds(float* cs, const floatx16 (&v)[2], 
         for (int r = 0; r < 8; ++r) cs[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * GL_LDC + 32 * j + (lane & 31)] = v[j][8 * hh + r];
 }
 
-// 1/rms of rows m0 .. m0 + n - 1 into rs (LDS), from the sums of squares their maker left by runs of 16, two of the
-// workgroup's threads a row
-__device__ __forceinline__ void row_scales(const MatArgs& a, float* rs, int n, int64_t m0, int t, int threads) {
-  for (int r = t >> 1; r < n; r += threads >> 1) {
-    float s = 0.f;
-    if (m0 + r < a.M) {
-      const float* q = a.ssq_in + (m0 + r) * a.ssq_parts;
-      for (int i = t & 1; i < a.ssq_parts; i += 2) s += q[i];
-    }
-    s += __shfl_xor(s, 1, 64);
-    if (!(t & 1)) rs[r] = 1.0f / sqrtf(s / (float)a.K + a.eps);
-  }
-}
-
 // MODE 0: K whole; 1: a part of K, its sums left in `parts`; 2: a part of K whose outputs go g.split_y elements after the
 // part before's (a store's only: whoever reads them adds them up)
-template <bool FOUR, int TM, int MODE>
+template <bool FOUR, int TM, int MODE, int EPI>
 __global__ __launch_bounds__(64 * GL_NW, TM == 2 ? 2 : 4) void gemm_lds_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits,
                                                                               float* parts) {
   constexpr bool SPLIT = MODE != 0;
@@ -343,14 +338,23 @@ __global__ __launch_bounds__(64 * GL_NW, TM == 2 ? 2 : 4) void gemm_lds_kernel(M
   constexpr int CW = 16 * GL_LDC * 4, WPA = AB / CW;
   static_assert(MODE == 1 || (NS + 2) * WPA >= GL_NW, "the outputs' place");
   float* cs = (float*)((wave < WPA ? a0 : wave < 2 * WPA ? a1 : wave < 3 * WPA ? (NS == 3 ? a2 : b1) : b0) + wave % WPA * CW);
-  float* rs_s = (float*)(b0 + BB) - 32 * TM * (wave + 1);
-  if (a.ssq_in) row_scales(a, rs_s, 32 * TM, m0 + wr, lane, 64);  // (each wave its own rows' 1/rms, where the weight was)
+  float* rs_s = (float*)b0;  // where the weight was: the rows' 1/rms, and RoPE's places and cache rows
+  int32_t* rows_s = (int32_t*)b0 + BM;
+  if (MODE == 0 && (a.ssq_in || EPI == GL_ROPE)) {
+    if (a.ssq_in)
+#pragma unroll 1
+      for (int r = 16 * wave; r < BM; r += 16 * GL_NW) row_scales16(a, rs_s + r, m0 + r, lane);
+    if (EPI == GL_ROPE && t < BM) stage_rope_rows(a, rows_s, BM, t, min(m0 + t, M - 1));
+    __syncthreads();
+  }
+#pragma unroll 1
   for (int u = 0; u < 2 * TM && m0 + wr + 16 * u < M; ++u) {
 #pragma unroll
     for (int ii = 0; ii < TM; ++ii)  // (the accumulators' indices stay constants)
       if (ii == u >> 1) block_to_lds(cs, acc[ii], u & 1, lane);
     wave_lds_order();
-    block_epilogue<MODE == 2>(a, g, cs, tn, wc, m0 + wr + 16 * u, M, ybase, lane, a.ssq_in ? rs_s + 16 * u : nullptr, MODE == 2 ? part * g.split_y : 0);
+    block_epilogue<EPI>(a, g, cs, tn, wc, m0 + wr + 16 * u, M, ybase, lane, MODE == 0 && a.ssq_in ? rs_s + wr + 16 * u : nullptr,
+                              rows_s + wr + 16 * u, rows_s + BM + wr + 16 * u, MODE == 2 ? part * g.split_y : 0);
     wave_lds_order();
   }
 }
@@ -359,24 +363,27 @@ __global__ __launch_bounds__(64 * GL_NW, TM == 2 ? 2 : 4) void gemm_lds_kernel(M
 // four parts' loads in flight at a time, then the epilogue. Bound by reading the parts once (splits x 4 bytes an output),
 // from the L2 of the XCD that wrote them (o at 200 rows in bfp4, both launches: 30.6 -> 24.7 us against parts dealt to
 // the XCDs part by part).
-template <int TM>
+template <int TM, int EPI>
 __global__ __launch_bounds__(256) void split_sum_kernel(MatArgs a, SkinnyMoe g, int tiles_m, int tiles_n, int splits, const float* parts) {
   __shared__ float rs_s[4][16];
+  __shared__ int32_t rows_s[4][32];
   __shared__ __attribute__((aligned(16))) float cs_s[4][16 * GL_LDC];
   const int64_t M = a.M;
   const int tiles = tiles_m * tiles_n;
   // (workgroups dealt to the XCDs in contiguous ranges, as the tiles' were: a tile's parts are in this XCD's L2)
   const int nb = gridDim.x, blk = nb % 8 == 0 ? (int)(blockIdx.x % 8) * (nb / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
-  const int lane = threadIdx.x & 63, u = blk * 4 + (threadIdx.x >> 6);  // unit u: (tile, wave, i, half)
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, u = blk * 4 + w;  // unit u: (tile, wave, i, half)
   const int half = u & 1, i = (u >> 1) % TM, wave = (u >> 1) / TM % GL_NW, id = (u >> 1) / (TM * GL_NW);
   if (id >= tiles) return;
   const int per_group = 8 * tiles_n, first_m = id / per_group * 8, gm = min(tiles_m - first_m, 8);
   const int tm = first_m + (id % per_group) % gm, tn = (id % per_group) / gm;
   const int64_t m0 = (int64_t)tm * 128 * TM + ((wave >> 1) * TM + i) * 32 + 16 * half;
   if (m0 >= M) return;
-  float* rs = rs_s[threadIdx.x >> 6];
-  float* cs = cs_s[threadIdx.x >> 6];
-  if (a.ssq_in) row_scales(a, rs, 16, m0, lane, 64);  // (this wave's own rows)
+  float* rs = rs_s[w];
+  float* cs = cs_s[w];
+  int32_t* rows = rows_s[w];  // (this wave's own rows)
+  if (a.ssq_in) row_scales16(a, rs, __builtin_amdgcn_readfirstlane((int)m0), lane);  // (m0 < 2^31: below 2^23 tiles)
+  if (EPI == GL_ROPE && lane < 16) stage_rope_rows(a, rows, 16, lane, min(m0 + lane, M - 1));
   const int64_t stride = (int64_t)tiles * GL_NW * TM * 2048;
   const float* p = parts + (((int64_t)id * GL_NW + wave) * TM + i) * 2048 + 512 * half + lane;
   float acc[16];
@@ -396,7 +403,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(MatArgs a, SkinnyMoe g, 
 #pragma unroll
   for (int r = 0; r < 16; ++r) cs[(8 * ((r & 7) >> 2) + 4 * (lane >> 5) + (r & 3)) * GL_LDC + 32 * (r >> 3) + (lane & 31)] = acc[r];
   wave_lds_order();
-  block_epilogue(a, g, cs, tn, (wave & 1) * 32, m0, M, 0, lane, a.ssq_in ? rs : nullptr);
+  block_epilogue<EPI>(a, g, cs, tn, (wave & 1) * 32, m0, M, 0, lane, a.ssq_in ? rs : nullptr, rows, rows + 16);
 }
 
 bool gemm_lds_takes(const MatArgs& a) {
@@ -408,17 +415,24 @@ int gemm_lds(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, const G
   if (!gemm_lds_fits(a, p)) return fail(FH_EUNSUP, "fh_gemm_bfp: too many tiles");
   if (p.splits > 1 && !g.split_y && (!parts || g.counts)) return fail(FH_EINVAL, "fh_gemm_bfp: K in parts needs a place for their sums");
   const dim3 grid((unsigned)(g.counts ? (all + 7) / 8 * 8 : all), g.counts ? experts : 1), block(64 * GL_NW);
+#define GL_RUN(F, TM, MODE, EPI) hipLaunchKernelGGL((gemm_lds_kernel<F, TM, MODE, EPI>), grid, block, 0, s, a, g, (int)tm, (int)tn, p.splits, parts)
+#define GL_SUM(TM, EPI) hipLaunchKernelGGL((split_sum_kernel<TM, EPI>), dim3((unsigned)(tm * tn * 4 * TM)), dim3(256), 0, s, a, g, (int)tm, (int)tn, p.splits, (const float*)parts)
 #define GL(F, TM) do { \
-    if (p.splits < 2) hipLaunchKernelGGL((gemm_lds_kernel<F, TM, 0>), grid, block, 0, s, a, g, (int)tm, (int)tn, 1, parts); \
-    else if (TM == 1 && g.split_y) hipLaunchKernelGGL((gemm_lds_kernel<F, 1, 2>), grid, block, 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
-    else { \
-      hipLaunchKernelGGL((gemm_lds_kernel<F, TM, 1>), grid, block, 0, s, a, g, (int)tm, (int)tn, p.splits, parts); \
-      hipLaunchKernelGGL((split_sum_kernel<TM>), dim3((unsigned)(tm * tn * 4 * TM)), dim3(256), 0, s, a, g, (int)tm, (int)tn, p.splits, (const float*)parts); \
-    } } while (0)
+    if (p.splits > 1 && TM == 1 && g.split_y) GL_RUN(F, 1, 2, GL_PLAIN); \
+    else if (p.splits > 1) { \
+      GL_RUN(F, TM, 1, GL_PLAIN); \
+      if (a.P == 1) GL_SUM(TM, GL_SUMS); \
+      else if (a.kind == FH_EP_SILU_GATE) GL_SUM(TM, GL_SILU); \
+      else GL_SUM(TM, GL_ROPE); \
+    } else if (a.P == 1) GL_RUN(F, TM, 0, GL_SUMS); \
+    else if (a.kind == FH_EP_SILU_GATE) GL_RUN(F, TM, 0, GL_SILU); \
+    else GL_RUN(F, TM, 0, GL_ROPE); } while (0)
   if (p.bm == 256) { if (fmt == FH_BFP4) GL(true, 2); else GL(false, 2); }
   else if (fmt == FH_BFP4) GL(true, 1);
   else GL(false, 1);
 #undef GL
+#undef GL_SUM
+#undef GL_RUN
   return check_launch("fh_gemm_bfp");
 }
 

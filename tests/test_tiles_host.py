@@ -12,9 +12,9 @@ template <int RUNS> static int walk(const fh::MatArgs& a) {  // every pair lane 
     for (int p = 0; p < RUNS / 2; ++p) {
       const int64_t run = fh::tile_run<RUNS>(a, tn, p);
       for (int j = 0; j < 16; ++j) {
-        const fh::RopePair r = fh::rope_pair(a, run, j);
+        const fh::RopePair r = fh::rope_pair(a.head_dim, a.heads + a.kv_heads, run, j);
         const bool in = r.d >= 0 && r.d < a.head_dim / 2 && r.d1 == r.d + a.head_dim / 2;
-        if (!in || r.h < 0 || (run < 0 && r.turn)) { printf("run %ld j %d: h %d d %d turn %d\n", (long)run, j, r.h, r.d, r.turn); return -1; }
+        if (run < 0 ? r.turn : !in || r.h < 0) { printf("run %ld j %d: h %d d %d turn %d\n", (long)run, j, r.h, r.d, r.turn); return -1; }
         if (run >= 0 && ((int64_t)r.h * a.head_dim + r.d != run * 16 + j || r.turn != (r.h < a.heads + a.kv_heads))) return -2;
       }
       past += run < 0;
@@ -126,3 +126,4 @@ def test_the_tiled_matmuls_tests_take_the_plans_they_name(tmp_path):
   assert [tuple(map(int, l.split())) for l in out] == [p for _, p in want]
   for plans in (PLANS, ROPES): assert {(bm, s > 1) for bm, s in plans.values()} >= {(128, False), (128, True), (256, True)}
   assert (256, 1) in PLANS.values()
+
