@@ -584,25 +584,11 @@ int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void*
   }();
   const int64_t tiles_n0 = a.P == 1 ? (a.N / 16 + 7) / 8 : ((int64_t)a.items + 3) / 4;
   const int64_t tiles2 = (a.M + 2 * GM_BM - 1) / (2 * GM_BM) * tiles_n0;
-  // gemm_pp_kernel for bf16 rows without the norm, its 256-row tiles 128, 192 or 256 columns wide: the widest whose
-  // tiles fill the CUs' rounds (at most one round, or the last at least 7/8 full) and no narrower tile takes fewer
-  // rounds of as much work; none filling them, the 4-wave kernel (qkv's 384 tiles of 2048 rows x 128 columns ran at
-  // 656 TFLOP/s against 712-750 for 128-row tiles two a CU)
-  int WNv = 0;
-  if (!g.counts && a.x_bf16 && !a.x_tiles && !a.norm_w) {
-    const int64_t mt = (a.M + 2 * GM_BM - 1) / (2 * GM_BM);
-    int64_t best = 0;
-    for (int wn = 2; wn <= 4; ++wn) {
-      const int64_t tiles = mt * (a.P == 1 ? (a.N / 16 + 4 * wn - 1) / (4 * wn) : ((int64_t)a.items + 2 * wn - 1) / (2 * wn));
-      const int64_t rounds = (tiles + cus - 1) / cus;
-      const bool fills = tiles <= cus || tiles * 8 >= rounds * cus * 7;
-      if (fills && (best == 0 || rounds * wn <= best)) { WNv = wn; best = rounds * wn; }
-    }
-  }
-  // gemm_lds (fh_gemm_lds.hip) for whatever it takes, but where one round of 192-column tiles of gemm_pp_kernel beats it
-  // (1.9 us a step: qkv at 2048 rows 130 us in its 256 tiles against 136 in 384 of 128 columns, at 1500 rows 113 against
-  // 134), and a mixture's experts past 512 rows a pass, several 128-row tiles an expert, where gemm_kernel's are
-  // faster (the Mixtral layer at 1000 tokens: 1168 us against 1279; at 300 even, at 100 616 against 485)
+  GemmWide w = {};
+  if (!g.counts && a.x_bf16 && !a.x_tiles && !a.norm_w) w = gemm_wide_plan(a, cus);
+  // gemm_lds (fh_gemm_lds.hip) for whatever it takes, but where one round of gemm_pp_kernel's wider tiles beats it
+  // (gemm_wide_us). And a mixture's experts past
+  // 512 rows a pass, several 128-row tiles an expert, where gemm_kernel's are faster (the Mixtral layer at 1000 tokens: 1168 us against 1279; at 300 even, at 100 616 against 485)
   if (gemm_lds_takes(a)) {
     if (g.counts) {
       if (a.M <= 512) {
@@ -613,13 +599,11 @@ int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void*
     } else {
       GemmPlan p = gemm_lds_plan(a.M, a.K, a.N, 0, workspace != nullptr);
       if (gemm_lds_bytes(p, a.M, a.N) > ws_bytes) p = gemm_lds_plan(a.M, a.K, a.N, 0, false);
-      const int64_t tiles3 = (a.M + 2 * GM_BM - 1) / (2 * GM_BM) * (a.P == 1 ? (a.N / 16 + 11) / 12 : ((int64_t)a.items + 5) / 6);
-      if (WNv != 3 || tiles3 > cus || p.us <= 8 + 1.9 * (double)(a.K / GM_BK))
-        if (gemm_lds_fits(a, p)) return gemm_lds(a, g, fmt, 1, p, (float*)workspace, s);
+      if (p.us <= gemm_wide_us(w, a.K, cus) && gemm_lds_fits(a, p)) return gemm_lds(a, g, fmt, 1, p, (float*)workspace, s);
     }
   }
   if (g.splits > 1) return fail(FH_EUNSUP, "gathered GEMM: K in parts for up to 512 bf16 rows whose K is a multiple of 64");
-  const bool pp = WNv != 0;
+  const bool pp = w.wn != 0;
   const int TMv = (pp || (!g.counts && tiles2 <= cus)) ? 2 : 1;
   const int64_t tiles_m = (a.M + GM_BM * TMv - 1) / (GM_BM * TMv);
   const int64_t tiles_n = tiles_n0;
@@ -630,11 +614,10 @@ int gemm_tiles(const MatArgs& a, const SkinnyMoe& g, int fmt, int experts, void*
   const int tm = (int)tiles_m, tn = (int)tiles_n;
   const int which = (fmt == FH_BFP4) * 4 + a.x_bf16 * 2 + (a.norm_w != nullptr);
   if (pp) {
-    const int64_t tnw = a.P == 1 ? (a.N / 16 + 4 * WNv - 1) / (4 * WNv) : ((int64_t)a.items + 2 * WNv - 1) / (2 * WNv);
-    const dim3 gridw((unsigned)(tiles_m * tnw));
-    const int tnv = (int)tnw;
-#define GM_PP(F) do { if (WNv == 2) hipLaunchKernelGGL((gemm_pp_kernel<F, 2>), gridw, b, 0, s, a, tm, tnv, g); \
-                      else if (WNv == 3) hipLaunchKernelGGL((gemm_pp_kernel<F, 3>), gridw, b, 0, s, a, tm, tnv, g); \
+    const dim3 gridw((unsigned)w.tiles);
+    const int tnv = (int)(w.tiles / tiles_m);
+#define GM_PP(F) do { if (w.wn == 2) hipLaunchKernelGGL((gemm_pp_kernel<F, 2>), gridw, b, 0, s, a, tm, tnv, g); \
+                      else if (w.wn == 3) hipLaunchKernelGGL((gemm_pp_kernel<F, 3>), gridw, b, 0, s, a, tm, tnv, g); \
                       else hipLaunchKernelGGL((gemm_pp_kernel<F, 4>), gridw, b, 0, s, a, tm, tnv, g); } while (0)
     if (fmt == FH_BFP4) GM_PP(true);
     else GM_PP(false);

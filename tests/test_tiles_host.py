@@ -127,3 +127,41 @@ def test_the_tiled_matmuls_tests_take_the_plans_they_name(tmp_path):
   for plans in (PLANS, ROPES): assert {(bm, s > 1) for bm, s in plans.values()} >= {(128, False), (128, True), (256, True)}
   assert (256, 1) in PLANS.values()
 
+
+CHOICE = r'''
+#include "fh_gemm.h"
+#include <cstdio>
+int main(int c, char** v) {  // M K N pairs: the kernel that bf16 rows take, with K in parts allowed
+  for (int i = 1; i + 3 < c; i += 4) {
+    fh::MatArgs a = {};
+    a.M = atoll(v[i]); a.K = atoll(v[i + 1]); a.N = atoll(v[i + 2]); a.P = atoi(v[i + 3]); a.items = (int)(a.N / 16 / a.P);
+    const fh::GemmPlan p = fh::gemm_lds_plan(a.M, a.K, a.N, 0, true);
+    const fh::GemmWide w = fh::gemm_wide_plan(a, 256);
+    if (p.us <= fh::gemm_wide_us(w, a.K, 256)) printf("lds%d\n", p.bm);
+    else printf("pp%d\n", w.wn);
+  }
+}
+'''
+
+
+def test_the_faster_kernel_past_a_round(tmp_path):
+  """Past one round of tiles a prompt's matmuls take the kernel and tile that measured fastest: each line one that another
+  rule got wrong (us measured in lds128, lds256 and one round of the wide tiles). lds128: 128-row tiles, two a CU."""
+  want = {(4096, 2048, 3072, 2): "lds128",   # 81, 97, 100 (192 columns)
+          (3000, 4096, 6144, 2): "lds128",   # 220, 233
+          (800, 4096, 28672, 2): "lds128",   # 273, 287
+          (1600, 2048, 11264, 2): "lds128",  # 118, 126
+          (1200, 2048, 11264, 2): "lds256",  # 88, 85
+          (2048, 1024, 5632, 2): "lds128",   # 46, 56, 61
+          (2048, 4096, 28672, 2): "lds256",  # 597, 533
+          (4096, 4096, 6144, 2): "lds256",   # 268, 248
+          (1400, 4096, 6144, 2): "pp3",      # 138, 138, 130
+          (2048, 4096, 6144, 2): "pp3",      # 151, 143, 142
+          (2300, 14336, 4096, 1): "pp3",     # 393 with K in parts, 326
+          (3000, 14336, 4096, 1): "pp4",     # 433 with K in parts, 398
+          (4096, 14336, 4096, 1): "pp4",     # 580, 498, 469
+          (4096, 4096, 4096, 1): "lds256",   # 154, 178
+          (2048, 14336, 4096, 1): "lds256"}  # one round: 238
+  exe = program(tmp_path, CHOICE)
+  out = subprocess.run([str(exe), *(str(x) for s in want for x in s)], capture_output=True, text=True, check=True).stdout.split()
+  assert dict(zip(want, out)) == want
