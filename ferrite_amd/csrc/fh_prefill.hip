@@ -14,7 +14,7 @@
 // scores are -1e30 (the reference adds -1e9; either leaves exp() at 0). Query tiles are issued longest first (the second half of the heads shortest first). A
 // block-float cache's runs are decoded exactly into the bf16 tiles (their values are bf16 values).
 #include <math.h>
-#include "fh_common.h"
+#include "fh_prefill.h"
 
 namespace fh {
 
@@ -22,7 +22,6 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
 constexpr int PA_BQ = 128;      // query rows a workgroup (32 a wave)
-constexpr int PA_BK = 64;       // keys a tile
 constexpr float PA_MASKED = -1e30f;
 
 struct PrefArgs {
@@ -452,10 +451,7 @@ extern "C" int fh_attention_prefill(const float* q, int64_t ldq, const void* cac
     return n;
   }();
   hipStream_t s = as_stream(stream);
-  // the keys split among a workgroup's waves where its tiles of 32 rows are still one round of a workgroup a CU and there
-  // is more than one key tile (32 heads of 128: 100 rows 9.0 -> 7.5 us, 64 after 1900 51 -> 30; past one round it loses:
-  // 300 rows 13 -> 18, 512 19 -> 24; one key tile 5.2 -> 7.1)
-  const bool split = (int64_t)((T + 31) / 32) * heads <= cus && p0 + T > PA_BK;
+  const bool split = prefill_splits_keys(T, heads, head_dim, p0, cus);
   const int bq = split ? 32 : PA_BQ;
   const dim3 g((T + bq - 1) / bq, heads), b(256);
   if (split) {

@@ -22,7 +22,8 @@ def test_gemv_slices(cuda, fmt, rows, K, N):
 
 @pytest.mark.parametrize("kind", ["bf16", "fp32", "bfp8", "bfp4"])
 @pytest.mark.parametrize("heads,kv,hd", [(4, 2, 128), (9, 3, 64)])
-@pytest.mark.parametrize("T,p0", [(1, 0), (1, 64), (31, 33), (32, 64), (33, 63), (100, 0), (129, 100), (200, 824), (40, 1000)])
+@pytest.mark.parametrize("T,p0", [(1, 0), (1, 64), (31, 33), (32, 64), (33, 63), (100, 0), (129, 100), (200, 824), (40, 1000),
+                                  (1, 320), (33, 320), (60, 300)])
 def test_prefill_attention_of_few_rows(cuda, kind, heads, kv, hd, T, p0):
   """A short prompt's causal attention, its keys split among a workgroup's waves (some of whose tiles lie wholly past a
   row), against float64 on the values the matrix cores take (bf16 q, k and v): the weights' bf16 rounding is at most 2^-9

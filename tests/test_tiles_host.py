@@ -165,3 +165,24 @@ def test_the_faster_kernel_past_a_round(tmp_path):
   exe = program(tmp_path, CHOICE)
   out = subprocess.run([str(exe), *(str(x) for s in want for x in s)], capture_output=True, text=True, check=True).stdout.split()
   assert dict(zip(want, out)) == want
+
+
+KEYS = r'''
+#include "fh_prefill.h"
+#include <cstdio>
+int main(int c, char** v) {
+  for (int i = 1; i + 3 < c; i += 4) printf("%d\n", fh::prefill_splits_keys(atoi(v[i]), atoi(v[i + 1]), atoi(v[i + 2]), atoll(v[i + 3]), 256));
+}
+'''
+
+
+def test_prompt_keys_split_where_it_is_the_faster(tmp_path):
+  """A short prompt's keys are split among a workgroup's waves where that gains in bf16 and does not lose in a block float,
+  by one rule for all formats (us whole and split, in bf16, then in bfp8)."""
+  want = {(100, 32, 128, 300): 1, (64, 32, 128, 1900): 1, (64, 32, 128, 4000): 1, (300, 32, 128, 0): 0,  # 51 30; 140 97 bfp8; past a round 13 18
+          (64, 32, 128, 0): 0, (64, 32, 128, 64): 0, (33, 1, 128, 33): 0,  # one tile 5.2 7.1; two 8.4 8.8, 10.5 13.2; 10.0 12.2 bfp8
+          (320, 1, 128, 0): 0, (200, 1, 128, 64): 0, (320, 1, 128, 1): 1,  # five: 17.1 15.4, 16.4 19.6; 17.0 18.3 bfp8; six
+          (2, 9, 64, 64): 0, (96, 9, 64, 64): 1, (320, 9, 64, 0): 1,       # 7.6 8.1 bfp8; 10.1 8.8 bfp8; five: 12.9 11.8 bfp8
+          (1, 300, 64, 5000): 0}
+  out = subprocess.run([str(program(tmp_path, KEYS)), *(str(x) for k in want for x in k)], capture_output=True, text=True, check=True).stdout.split()
+  assert dict(zip(want, map(int, out))) == want
