@@ -25,7 +25,9 @@
 // time.
 //
 // The epilogue takes each wave's blocks through its own part of LDS, 32 rows at a time, so that a row's outputs leave
-// in 16-byte stores (or, with the fused elementwise program, a row's columns a wave at a time).
+// in 16-byte stores. The fused elementwise program runs there in place, 4 rows a pass of the wave: an element at a time
+// its decoding is what these tiles' 8 waves a CU wait for (of 9 ops: fp32 4096 x 16 x 4096 413 us, so 237, which 64 x 64
+// tiles of 20 KiB of LDS, 8 waves a SIMD, took too; bf16 2048^3 125 us, so 57; one op 47, so 31).
 #include "fh_program.h"
 
 namespace fh {
@@ -117,8 +119,23 @@ __device__ inline void matmul_epilogue(const MmArgs& m, const fh_program& p, con
     }
     wave_lds_order();
     const int64_t row0 = r0 + 32 * i;
+    if (PROG) {
+      constexpr int R = 64 / (32 * TN), E = TM * TN > 4 ? 2 : 4;  // rows a pass of the wave, passes at a time (2: registers)
+      const int c = lane % (32 * TN), rl = lane / (32 * TN);
+      const int64_t rows = m.M - row0, col = min(col0 + c, m.N - 1);
+      for (int rr = 0; rr < 32 && rr < rows; rr += E * R) {  // (whole waves: places past M or N read the last there is)
+        const int r = rr + rl;
+        float v[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = cs[(r + e * R) * CLD + c];
+        prog_eval_rows<E>(p, v, bi, row0 + r, R, m.M - 1, col);
+#pragma unroll
+        for (int e = 0; e < E; ++e) cs[(r + e * R) * CLD + c] = v[e];
+      }
+      wave_lds_order();
+    }
     const bool inside = row0 + 32 <= m.M && col0 + 32 * TN <= m.N;
-    if (!PROG && m.cvec && inside && m.c_dtype != FH_I32) {
+    if (m.cvec && inside && m.c_dtype != FH_I32) {
       if (m.c_dtype == FH_BF16) {
         constexpr int L = 4 * TN;  // lanes a row, 8 columns each
 #pragma unroll
@@ -141,11 +158,7 @@ __device__ inline void matmul_epilogue(const MmArgs& m, const fh_program& p, con
       for (int e = lane; e < 32 * 32 * TN; e += 64) {
         const int r = e / (32 * TN), c = e % (32 * TN);
         const int64_t row = row0 + r, col = col0 + c;
-        if (row < m.M && col < m.N) {
-          float v = cs[r * CLD + c];
-          if (PROG) v = prog_eval(p, v, bi, row, col);
-          prog_store(m.c, m.c_dtype, cbase + row * m.ldc + col, v);
-        }
+        if (row < m.M && col < m.N) prog_store(m.c, m.c_dtype, cbase + row * m.ldc + col, cs[r * CLD + c]);
       }
     }
   }

@@ -69,6 +69,90 @@ __device__ inline float prog_eval(const fh_program& p, float acc, int64_t b, int
   return last;
 }
 
+// prog_apply of E elements, decoded once
+template <int E>
+__device__ inline void prog_apply_rows(int op, float (&x)[E], float (&y)[E], float (&o)[E]) {
+#define PROG_EACH(code) case code: _Pragma("unroll") for (int e = 0; e < E; ++e) o[e] = prog_apply(code, x[e], y[e]); break;
+  switch (op) {
+    PROG_EACH(FH_OP_ADD) PROG_EACH(FH_OP_SUB) PROG_EACH(FH_OP_MUL) PROG_EACH(FH_OP_MAX) PROG_EACH(FH_OP_CMPLT)
+    PROG_EACH(FH_OP_CMPNE) PROG_EACH(FH_OP_KEEP) PROG_EACH(FH_OP_DROP) PROG_EACH(FH_OP_RELU) PROG_EACH(FH_OP_EXP)
+    PROG_EACH(FH_OP_EXP2) PROG_EACH(FH_OP_LOG) PROG_EACH(FH_OP_LOG2) PROG_EACH(FH_OP_RECIP) PROG_EACH(FH_OP_SQRT)
+    PROG_EACH(FH_OP_FTOB) PROG_EACH(FH_OP_ITOF) PROG_EACH(FH_OP_FTOI) PROG_EACH(FH_OP_COPY)
+    default:  // sine and cosine, long: one copy of their code, an element after the other (the values move down one place
+              // instead of being indexed: they stay registers)
+#pragma unroll 1
+      for (int n = 0; n < E; ++n) {
+        const float v = op == FH_OP_SIN ? sinf(x[0]) : cosf(x[0]);
+#pragma unroll
+        for (int e = 0; e + 1 < E; ++e) { x[e] = x[e + 1]; o[e] = o[e + 1]; }
+        o[E - 1] = v;
+      }
+  }
+#undef PROG_EACH
+}
+
+// 16 bytes of a program in scalar registers, taken out one after the other
+struct ProgBytes {
+  uint64_t lo, hi;
+  __device__ explicit ProgBytes(const int8_t* b) : lo(((const uint64_t*)b)[0]), hi(((const uint64_t*)b)[1]) {}
+  __device__ int next() {
+    const int v = (int)(lo & 255);
+    lo = lo >> 8 | hi << 56;
+    hi >>= 8;
+    return v;
+  }
+};
+
+typedef float prog_regs __attribute__((ext_vector_type(16)));
+
+// prog_eval at E rows r0, r0 + step, .. (past last_row that one) of a column c in one pass of the whole wave: their loads
+// in flight together, each op decoded once. What an element costs is that decoding, a chain of scalar branches (the loop
+// over it uniform, or each becomes several) that a tiled kernel's few waves leave bare. acc: the matmul's results in, the
+// program's out.
+template <int E>
+__device__ inline void prog_eval_rows(const fh_program& p, float (&acc)[E], int64_t b, int64_t r0, int64_t step, int64_t last_row, int64_t c) {
+  static_assert(FH_MAX_OPS == 15, "the registers' places: 15 is the matmul's result");
+  prog_regs reg[E];  // (registers taken by an index of the whole wave)
+  float o[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) { reg[e][15] = acc[e]; o[e] = acc[e]; }
+  ProgBytes ops(p.op), as(p.a), bs(p.b);
+  const int n_ops = p.n_ops;
+#pragma unroll 1
+  for (int i = 0; i < n_ops; ++i) {
+    float xy[2][E];
+    const float imm = p.imm[i];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      float (&v)[E] = xy[s];
+      const int code = s ? bs.next() : as.next();
+      if ((code & 24) == 16) {
+        const int k = code - 16;
+        const int64_t at0 = b * p.in_stride[k][0] + c * p.in_stride[k][2], ld = p.in_stride[k][1];
+        int64_t at[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) at[e] = at0 + min(r0 + e * step, last_row) * ld;
+#define PROG_LOAD(type, expr) do { const type* in = (const type*)p.in[k]; type w[E]; \
+          _Pragma("unroll") for (int e = 0; e < E; ++e) w[e] = in[at[e]]; \
+          _Pragma("unroll") for (int e = 0; e < E; ++e) v[e] = (expr); } while (0)
+        if (p.in_dtype[k] == FH_BF16) PROG_LOAD(uint16_t, bf16_to_f(w[e]));
+        else if (p.in_dtype[k] == FH_I32) PROG_LOAD(int32_t, (float)w[e]);
+        else PROG_LOAD(float, w[e]);
+#undef PROG_LOAD
+      } else {
+        const int at = code < 16 ? code : 15;
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = code == FH_OPND_IMM ? imm : reg[e][at];
+      }
+    }
+    prog_apply_rows<E>(ops.next(), xy[0], xy[1], o);
+#pragma unroll
+    for (int e = 0; e < E; ++e) reg[e][i] = o[e];
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) acc[e] = o[e];
+}
+
 __device__ inline void prog_store(void* out, int dtype, int64_t at, float v) {
   if (dtype == FH_BF16) ((uint16_t*)out)[at] = (uint16_t)bf16_rne_f(v);
   else if (dtype == FH_I32) ((int32_t*)out)[at] = (int32_t)truncf(v);

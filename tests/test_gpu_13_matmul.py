@@ -144,3 +144,52 @@ def test_tiles_and_strides_give_the_same_bits(cuda, M, K, N):
     assert torch.equal(again, got), pad
   half = ops().matmul(a, b, out_dtype=torch.bfloat16)
   assert torch.equal(half, got.to(torch.bfloat16))  # rounded once, to nearest even, in vector and in single stores
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16, torch.int32])
+@pytest.mark.parametrize("batch,M,K,N", [
+  (3, 5, 33, 17), (1, 64, 64, 64), (2, 65, 64, 63),   # 64 x 64 tiles: inside one, one whole, a row more and a column less
+  (1, 2047, 64, 2056),                                # 128 x 128 from LDS loads, the last row and piece past whole tiles
+  (1, 4095, 64, 4104), (1, 4097, 16, 4099),           # 128 x 256 from LDS loads; 256 x 256 by registers
+])
+def test_programs_give_the_elementwise_kernels_bits(cuda, batch, M, K, N, out_dtype):
+  """A matmul's program against the plain matmul followed by the same program in the elementwise kernel, bit for bit:
+  15 ops, every op in one of the three programs, operands from results far back, immediates, the matmul's result and
+  inputs of each type (one broadcast over rows, one over columns), at the tiles' edges and for fp32 operands too; C's
+  places between its rows stay as they were."""
+  import ctypes
+  from ferrite_amd import lib
+  g = torch.Generator(device="cuda").manual_seed(batch + M + K + N)
+  rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+  ins = [rnd(batch, M, N), rnd(batch, 1, N).to(torch.bfloat16), torch.randint(-9, 9, (1, M, 1), generator=g, device="cuda", dtype=torch.int32)]
+  strides = [(M * N, N, 1), (N, 0, 1), (0, 1, 0)]
+  acc, imm, x, y, z = lib.OPND_ACC, lib.OPND_IMM, 16, 17, 18
+  programs = [
+    [("add", acc, x), ("mul", 0, y), ("sub", 1, z), ("max", 2, acc), ("cmplt", 0, 3), ("cmpne", 1, imm, 0.5), ("keep", 4, 2), ("drop", 4, x),
+     ("add", 6, 7), ("relu", 8, 8), ("sin", 0, 0), ("cos", 10, 10), ("mul", 9, 11), ("add", 12, 5), ("sub", 13, 0)],
+    [("relu", acc, acc), ("add", 0, imm, 1.0), ("log", 1, 1), ("log2", 1, 1), ("sqrt", 1, 1), ("recip", 4, 4), ("exp", 5, 5), ("exp2", 2, 2),
+     ("add", 6, 7), ("mul", 8, 3), ("ftob", 9, 9), ("max", 10, y), ("itof", z, z), ("add", 11, 12), ("copy", 13, 13)],
+    [("ftoi", acc, acc)]]
+  def made(ops_, inputs, st):
+    p = lib.Program()
+    p.n_ops, p.n_inputs = len(ops_), len(inputs)
+    for k, (t, s) in enumerate(zip(inputs, st)):
+      p.input[k], p.in_dtype[k] = t.data_ptr(), {torch.float32: lib.F32, torch.bfloat16: lib.BF16, torch.int32: lib.I32}[t.dtype]
+      for i in range(3): p.in_stride[k][i] = s[i]
+    for i, o in enumerate(ops_): p.op[i], p.a[i], p.b[i], p.imm[i] = lib.OP[o[0]], o[1], o[2], o[3] if len(o) > 3 else 0.0
+    return p
+  out_code = {torch.float32: lib.F32, torch.bfloat16: lib.BF16, torch.int32: lib.I32}[out_dtype]
+  a, b = rnd(batch, M, K), rnd(batch, K, N)
+  for da, db in ((torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)):
+    A, B = a.to(da), b.to(db)
+    plain = ops().matmul(A, B)
+    for prog in programs:
+      swap = [tuple(19 if i in (1, 2) and v == acc else v for i, v in enumerate(o)) for o in prog]
+      q = made(swap, ins + [plain], strides + [(M * N, N, 1)])
+      want = torch.empty(batch, M, N, device="cuda", dtype=out_dtype)
+      lib.call("fh_map", ctypes.byref(q), want.data_ptr(), out_code, batch, M, N, M * N, N, ops()._stream())
+      for pad in (0, 3):
+        wide = torch.full((batch, M, N + pad), 77, device="cuda", dtype=out_dtype)
+        ops().matmul(A, B, made(prog, ins, strides), out=wide[:, :, :N])
+        assert torch.equal(wide[:, :, :N], want), (da, len(prog), pad)
+        assert (wide[:, :, N:] == 77).all()
