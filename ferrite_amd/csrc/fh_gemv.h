@@ -6,7 +6,7 @@
 namespace fh {
 
 // rows a lane has in flight at once, by format and batch rows (about 4 KiB of weight a wave and run at batch 1)
-__host__ __device__ constexpr int gemv_group(bool four, int b, int p) { return (b <= 2 ? 4 : b <= 4 ? 2 : 1) * (four ? 2 : 1) + 0 * p; }
+__host__ __device__ constexpr int gemv_group(bool four, int b) { return (b <= 2 ? 4 : b <= 4 ? 2 : 1) * (four ? 2 : 1); }
 
 // threads a workgroup at most: 16 waves for one row, 8 for more (whose partial sums need the registers)
 __host__ __device__ constexpr int gemv_threads(int b) { return b == 1 ? 1024 : 512; }
@@ -27,7 +27,7 @@ inline GemvPlan gemv_plan(int64_t K, int64_t N, int fmt, int kind, int batch) {
   p.most = p.P == 1 ? 8 : 4;
   p.items = (int)(N / 16 / p.P);
   const int b = batch < p.most ? batch : p.most;
-  const int unit = 64 * gemv_group(fmt == FH_BFP4, b, p.P);
+  const int unit = 64 * gemv_group(fmt == FH_BFP4, b);
   const int64_t units = (K + unit - 1) / unit;
   const int64_t most = std::min<int64_t>(fmt == FH_BFP4 ? 16 : 8, gemv_threads(b) / 64);
   int64_t W = 1;

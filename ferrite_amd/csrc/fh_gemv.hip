@@ -26,7 +26,7 @@ __global__ __launch_bounds__(gemv_threads(B)) void gemv_kernel(const uint8_t* __
                                                               int K, int rows, int ldx, int pair_half, MatArgs a) {
   constexpr int V = B * P * 16;       // a lane's partial sums: [b][p][j]
   constexpr int G = B * P;
-  constexpr int U = gemv_group(FOUR, B, P);
+  constexpr int U = gemv_group(FOUR, B);
   constexpr int RB = FOUR ? 8 : 16;   // bytes of a run's row
   using Row = typename std::conditional<FOUR, uint2, uint4>::type;
   const int lane = threadIdx.x & 63;

@@ -281,7 +281,9 @@ class Decoder:
   def prefill(self, ids, slot=0, p0=0, chunk=None):
     """A prompt's tokens at places p0 .. p0 + len(ids) - 1 of sequence `slot`, on the matrix cores (in chunks of
     `chunk` tokens, as models/llama.py:498-504 prefills): their keys and values go into the cache; returns the last
-    token's logits ([1][vocab] fp32) and its greedy pick ([1] int32)."""
+    token's logits ([1][vocab] fp32) and its greedy pick ([1] int32). Each call repeats its bits, but chunks give the
+    whole prompt's values within the rounding of fp32 sums: the order in which a matmul adds K and attention the keys
+    follows the rows of a call."""
     ids = [int(i) for i in ids]
     T = len(ids)
     if T < 1 or p0 < 0 or p0 + T > min(self.context, self.c.places): raise ValueError("prefill: the prompt's places past the cache or RoPE's tables")

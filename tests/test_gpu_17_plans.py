@@ -9,8 +9,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 2, 8])
 @pytest.mark.parametrize("K,N", [(1, 16), (63, 32), (64, 48), (65, 64), (576, 960), (1000, 576), (1536, 1536), (2048, 16), (4160, 4096), (4096, 4112)])
 def test_gemv_slices(cuda, fmt, rows, K, N):
-  """The GEMV's K slices: a wave as few as 64 rows where there are few items, as many as its loads in flight cover past
-  that. Exact products summed in fp32: K roundings of at most 2^-24 of sum |x w| each, and far fewer in its tree."""
+  """The GEMV's K slices: whole groups of a wave's loads in flight, the last a part of one, at edges of 64 rows and of the
+  groups. Exact products summed in fp32: K roundings of at most 2^-24 of sum |x w| each, and far fewer in its tree."""
   from ferrite_amd import ops
   g = torch.Generator(device="cuda").manual_seed(K + 5 * N + rows)
   x = torch.randn(rows, K, generator=g, device="cuda")
