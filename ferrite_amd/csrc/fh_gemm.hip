@@ -43,16 +43,25 @@ __device__ inline void gemm_epilogue(const MatArgs& a, const SkinnyMoe& g, const
                                      const int32_t* crow_s) {
   constexpr int LDC = BN + 4, RUNS = BN / 16, H = BN / 2;
   const int kind = a.kind;
-  if (a.P == 1 && kind == FH_EP_PROGRAM) {  // (a loop of its own: the program's decoding, hoisted out of the loop,
-                                            // runs only here)
+  if (a.P == 1 && kind == FH_EP_PROGRAM) {  // (a loop of its own: the program's decoding runs only here, once for E rows of
+                                            // a column, whole waves together; places past M or the weight read the last)
     if (t >= NT / BN * BN) return;
+    constexpr int S = NT / BN, E = 4;
+    static_assert(BM % (S * E) == 0, "whole passes");
     const int c = t % BN;
     const int64_t run = tile_run<RUNS>(a, tn, c >> 4);
-    const int64_t col = run * 16 + (c & 15);
-    for (int r = t / BN; r < BM; r += NT / BN) {
-      const int64_t m = m0 + r;
-      if (m < M && run >= 0)
-        store_out(a.y, a.y_bf16, (ybase + m) * a.ldy + col, prog_eval(a.prog, Cs[r * LDC + c] * rs_s[r], 0, m, col));
+    const int64_t col = run >= 0 ? run * 16 + (c & 15) : 0;
+    for (int rb = 0; rb < BM && m0 + rb < M; rb += S * E) {
+      const int r = rb + t / BN;
+      float v[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = Cs[(r + e * S) * LDC + c] * rs_s[r + e * S];
+      prog_eval_rows<E>(a.prog, v, 0, m0 + r, S, M - 1, col);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int64_t m = m0 + r + e * S;
+        if (m < M && run >= 0) store_out(a.y, a.y_bf16, (ybase + m) * a.ldy + col, v[e]);
+      }
     }
   } else if (a.P == 1) {  // FH_EP_STORE, FH_EP_RESIDUAL: a thread a column, NT / BN rows a pass; a run is 16 lanes
     if (t >= NT / BN * BN) return;

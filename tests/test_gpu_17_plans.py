@@ -230,3 +230,45 @@ def test_moe_experts_keeps_a_workspace_for_more_rows(cuda):
     before = torch.cuda.memory_allocated()
     ops.moe_experts(x, ex, dense, out=out, ws=ws)
     assert (torch.cuda.max_memory_allocated() > before) == more, (rows, sized)
+
+
+@pytest.mark.parametrize("kind", ["fp32", "bf16", "norm"])
+@pytest.mark.parametrize("M,K,N", [(65, 96, 48), (129, 96, 272), (300, 64, 640), (2048, 64, 1552), (1700, 128, 6144), (2048, 64, 8208)])
+def test_gemm_programs_give_the_elementwise_kernels_bits(cuda, kind, M, K, N):
+  """A block-float matmul's program past 64 rows (128 and 256 row tiles, the two-group kernel's widths; rows and runs past the
+  matrix in the last tiles) against the plain store of the same kernels followed by the same program in the elementwise
+  kernel, bit for bit: fp32 and bf16 outputs, inputs by row, by column and by both."""
+  import ctypes
+  from ferrite_amd import lib, ops
+  g = torch.Generator(device="cuda").manual_seed(M + K + N)
+  rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+  x = rnd(M, K) if kind != "bf16" else rnd(M, K).to(torch.bfloat16)
+  bw = ops.pack(rnd(K, N) * 0.1, "bfp4" if M % 2 else "bfp8")
+  norm = {"norm_w": rnd(K), "ssq_in": x.float().square().reshape(M, K // 16, 16).sum(-1), "eps": 1e-5} if kind == "norm" else {}
+  ins, strides = [rnd(M, N), rnd(N).to(torch.bfloat16), rnd(M)], [(0, N, 1), (0, 0, 1), (0, 1, 0)]
+  chain = [("mul", lib.OPND_ACC, 17), ("add", 0, 16), ("sub", 1, 18), ("exp2", 0, 0), ("max", 2, lib.OPND_ACC), ("cmplt", 3, 4), ("keep", 5, 2), ("add", 6, 1)]
+  def made(ops_, inputs, st):
+    p = lib.Program()
+    p.n_ops, p.n_inputs = len(ops_), len(inputs)
+    for k, (t, s) in enumerate(zip(inputs, st)):
+      p.input[k], p.in_dtype[k] = t.data_ptr(), lib.BF16 if t.dtype == torch.bfloat16 else lib.F32
+      for i in range(3): p.in_stride[k][i] = s[i]
+    for i, (op, a, b) in enumerate(ops_): p.op[i], p.a[i], p.b[i] = lib.OP[op], a, b
+    return p
+  # (the plain sums by the same kernels: a program that gives them back)
+  plain = ops.epilogue(lib.EP_PROGRAM, **norm)
+  plain.program = ctypes.pointer(made([("copy", lib.OPND_ACC, lib.OPND_ACC), ("copy", 0, 0)], [], []))
+  sums = ops.gemm(x, bw, plain)
+  w = ops.dequant(bw).double()
+  xs = x.double() if kind != "norm" else x.double() * norm["norm_w"].double() / (x.double().square().mean(-1, keepdim=True) + 1e-5).sqrt()
+  assert ((sums.double() - xs @ w).abs() <= 2 ** -7 * (xs.abs() @ w.abs())).all()  # (rows rounded to bf16 for the matrix cores)
+  ep = ops.epilogue(lib.EP_PROGRAM, **norm)
+  ep.program = ctypes.pointer(made(chain, ins, strides))
+  swapped = made([(op, *(19 if v == lib.OPND_ACC else v for v in ab)) for op, *ab in chain], ins + [sums], strides + [(0, N, 1)])
+  for dt, code in ((torch.float32, lib.F32), (torch.bfloat16, lib.BF16)):
+    want = torch.empty(M, N, device="cuda", dtype=dt)
+    lib.call("fh_map", ctypes.byref(swapped), want.data_ptr(), code, 1, M, N, M * N, N, ops._stream())
+    wide = torch.full((M, N + 8), 77, device="cuda", dtype=dt)
+    ops.gemm(x, bw, ep, out=wide[:, :N])
+    assert torch.equal(wide[:, :N], want), dt
+    assert (wide[:, N:] == 77).all()
