@@ -56,6 +56,28 @@ __device__ __forceinline__ void row_scales16(const MatArgs& a, float* rs, int64_
   if (!(lane & 3)) rs[reduce16_index(lane)] = 1.0f / sqrtf(v[0] / (float)a.K + a.eps);
 }
 
+// row_scales16 of 32 rows: of few sums (a load a row) all 32 in flight at once, where a second pass would be half of the call
+__device__ __forceinline__ void row_scales32(const MatArgs& a, float* rs, int64_t m0, int lane) {
+  if (a.ssq_parts > 64) {
+#pragma unroll 1
+    for (int r = 0; r < 32; r += 16) row_scales16(a, rs + r, m0 + r, lane);
+    return;
+  }
+  const float* q = a.ssq_in + min(m0, a.M - 1) * a.ssq_parts;
+  const int last = (int)min((int64_t)31, max((int64_t)0, a.M - 1 - m0));
+  const bool ok = lane < a.ssq_parts;
+  float v[2][16];
+#pragma unroll
+  for (int r = 0; r < 32; ++r) v[r >> 4][r & 15] = q[min(r, last) * a.ssq_parts + (ok ? lane : 0)];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[h][r] = ok ? v[h][r] : 0.f;
+    wave_reduce16(v[h]);
+    if (!(lane & 3)) rs[16 * h + reduce16_index(lane)] = 1.0f / sqrtf(v[h][0] / (float)a.K + a.eps);
+  }
+}
+
 // RoPE's per-row values for a tile's epilogue, staged in LDS: row ar's place and cache row (m: the row, clamped into the
 // matrix)
 __device__ inline void stage_rope_rows(const MatArgs& a, int32_t* rows_s, int bm, int ar, int64_t m) {

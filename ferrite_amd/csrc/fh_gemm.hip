@@ -301,6 +301,14 @@ __global__ __launch_bounds__(GM_THREADS * TM, 3 - TM) void gemm_kernel(MatArgs a
   load(0, x0, w0, e0);
   load(GM_BK, x1, w1, e1);
 
+  // each row's 1 / rms, while the first loads are in flight (a branch out of line: in line it moves the K loop's registers, fp32
+  // rows 2-3% slower; after the loop, 2 us a call)
+  if (__builtin_expect(a.ssq_in != nullptr, 0)) {  // (NORM, or rows that already hold x * w)
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    row_scales32(a, rs_s + 32 * w, m0 + 32 * w, lane);
+  } else if (ah == 0) {
+    rs_s[ar] = 1.f;
+  }
   if (a.kind == FH_EP_ROPE_KV && ah == 1) stage_rope_rows(a, rows_s, BM, ar, xr0);
 
   floatx16 acc[2][2];
@@ -343,14 +351,6 @@ __global__ __launch_bounds__(GM_THREADS * TM, 3 - TM) void gemm_kernel(MatArgs a
     store(k0 + 2 * GM_BK, 0, x0, w0, e0);  // (past the last step: a stage nobody reads)
   }
 
-  // each row's 1 / rms (here and not while the first loads are in flight: the loop's registers are free)
-  if (a.ssq_in) {  // (NORM, or rows that already hold x * w)
-    const int w = __builtin_amdgcn_readfirstlane(wave);
-#pragma unroll 1
-    for (int r = 32 * w; r < 32 * w + 32; r += 16) row_scales16(a, rs_s + r, m0 + r, lane);
-  } else if (ah == 0) {
-    rs_s[ar] = 1.f;
-  }
   // the output tile, fp32, through LDS: block (i, j)'s value r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4,
   // column l % 32
   __syncthreads();
@@ -555,8 +555,7 @@ __global__ __launch_bounds__(2 * GM_THREADS, 1) void gemm_pp_kernel(MatArgs a, i
   // each row's 1 / rms
   if (a.ssq_in) {
     const int w = __builtin_amdgcn_readfirstlane(wave);
-#pragma unroll 1
-    for (int r = 32 * w; r < 32 * w + 32; r += 16) row_scales16(a, rs_s + r, m0 + r, lane);
+    row_scales32(a, rs_s + 32 * w, m0 + 32 * w, lane);
   } else if (!(t & 1)) {
     rs_s[t >> 1] = 1.f;
   }
