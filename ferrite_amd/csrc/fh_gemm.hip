@@ -44,7 +44,8 @@ __device__ inline void gemm_epilogue(const MatArgs& a, const SkinnyMoe& g, const
   constexpr int LDC = BN + 4, RUNS = BN / 16, H = BN / 2;
   const int kind = a.kind;
   if (a.P == 1 && kind == FH_EP_PROGRAM) {  // (a loop of its own: the program's decoding runs only here, once for E rows of
-                                            // a column, whole waves together; places past M or the weight read the last)
+                                            // a column, whole waves together; places past M or the weight read the last.
+                                            // A row a pass, fp32 2048^3 with one op 115 us, nine 284; so 90, 144)
     if (t >= NT / BN * BN) return;
     constexpr int S = NT / BN, E = 4;
     static_assert(BM % (S * E) == 0, "whole passes");
